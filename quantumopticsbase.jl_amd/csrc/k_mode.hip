@@ -24,7 +24,7 @@
 //                 loaded linearly into LDS planes, the mode product runs from
 //                 LDS into output planes, and the output chunk is written
 //                 back linearly.
-//   k_zgemm       everything wider: a 64 x 64 x 16 LDS-tiled complex GEMM
+//   k_zgemm       everything wider: an LDS-tiled complex GEMM
 //                 with arbitrary element strides and a batch index, used for
 //                 factors wider than 64 and for DenseOperator on a density
 //                 matrix (and qob_gemm).
@@ -35,6 +35,7 @@
 #include <map>
 #include <mutex>
 #include <numeric>
+#include <type_traits>
 #include <unordered_set>
 
 namespace qob {
@@ -294,26 +295,47 @@ __global__ void __launch_bounds__(CHUNK_NT) k_mode_chunk(const cplx<R> *__restri
 // C[m, n] = alpha * sum_k A[m, k] B[k, n] + beta * C[m, n] for every batch
 // index z, with element (m, k) of A at A + z sa + m sam + k sak, (k, n) of B
 // at B + z sb + k sbk + n sbn, (m, n) of C at C + z sc + m scm + n scn.
-// Tiles of BM x BN outputs, K in chunks of BK through double-buffered LDS
-// planes (real and imaginary parts apart).  Four waves in a 2 x 2 grid; the
-// MFMA rows run along n and its columns (lane % 16) along m, so a C column
-// with scm = 1 is stored as 16-element runs.
-constexpr int GBM = 64, GBN = 64, GBK = 16, GPAD = 4, GNT = 256;
+// Tiles of BM x BN outputs, K in chunks of 16 through two LDS buffers.  Four
+// waves in a 2 x 2 grid; the MFMA rows run along n and its columns (lane % 16)
+// along m, so a C column with scm = 1 is stored as 16-element runs.
+//
+// Bound by the MFMA rate.  A wave issues in order, so whatever it issues
+// between its MFMAs and does not overlap costs matrix time:
+//   - LDS rows hold interleaved complex elements and are BM + 1 long: a chunk
+//     whose threads run along k is staged without bank conflicts (separate
+//     real and imaginary planes with 64 + 16 columns: 8-way conflicts, a
+//     third of the kernel), and one 16-byte read gives a fragment's both parts;
+//   - a whole chunk costs one pointer addition per load and nothing else
+//     (with the bounds checks of the last chunk on every chunk: 64 instead of
+//     68 TFLOP/s);
+//   - a chunk is staged before the MFMAs of the previous chunk's last k-step;
+//   - registers are capped (WPE waves per SIMD), which also keeps the
+//     accumulators out of the accumulation registers (the compiler copied
+//     them there and back on every chunk).
+// Measured (ComplexF64 / ComplexF32, square, against one 64 x 64 tile shape
+// with none of these): 4096: 7.64 / 4.22 ms (71.9 / 130 TFLOP/s) from 9.76 /
+// 4.69; 3001: 3.21 / 1.76 from 4.05 / 1.97; 1000: 130 / 76 us from 186 / 110;
+// 200: 11 / 7.8 us from 40 / 25.  Not kept: loads two chunks ahead (no
+// change), k split over wave groups of one workgroup (no gain from 64^3 to
+// 4096^3), 8 k per chunk, a 64 x 64 tile (1-3% faster above 3000^3 in
+// ComplexF32, slower below 2000^3).
+constexpr int GNT = 256, GBK = 16, GPAD = 1;
 
-template <typename R>
-__global__ void __launch_bounds__(GNT) k_zgemm(int64_t M, int64_t N, int64_t K, const cplx<R> *__restrict__ A,
+template <typename R, int BM, int BN, int WPE>
+__global__ void __launch_bounds__(GNT, WPE) k_zgemm(int64_t M, int64_t N, int64_t K, const cplx<R> *__restrict__ A,
                                                int64_t sam, int64_t sak, int64_t sa, const cplx<R> *__restrict__ B,
                                                int64_t sbk, int64_t sbn, int64_t sb, cplx<R> *__restrict__ C,
                                                int64_t scm, int64_t scn, int64_t sc, int64_t tiles_m, int64_t tiles_n,
                                                double2 alpha_, double2 beta_, int beta_zero) {
     using T = cplx<R>;
     using V = typename mf<R>::v4;
-    constexpr int LA = GBM + GPAD, LB = GBN + GPAD;
-    constexpr int AE = GBM * GBK / GNT, BE = GBN * GBK / GNT;
-    constexpr int TMW = GBM / 32, TNW = GBN / 32;  // 16 x 16 tiles per wave along m and n
+    constexpr int LA = BM + GPAD, LB = BN + GPAD;
+    constexpr int BK = GBK, KS = BK / 4;  // k and MFMA k-steps per chunk
+    constexpr int AE = BM * BK / GNT, BE = BN * BK / GNT;
+    constexpr int TMW = BM / 32, TNW = BN / 32;  // 16 x 16 tiles per wave along m and n
+    constexpr int BUF = BK * (LA + LB);          // elements per buffer: A [k][m], then B [k][n]
     extern __shared__ unsigned char lds_raw[];
-    R *As = (R *)lds_raw;             // [buf][plane][k][m]
-    R *Bs = As + 2 * 2 * GBK * LA;    // [buf][plane][k][n]
+    T *lds = (T *)lds_raw;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lr = lane & 15, lk = lane >> 4;
     const int wm = wave & 1, wn = wave >> 1;
@@ -321,43 +343,57 @@ __global__ void __launch_bounds__(GNT) k_zgemm(int64_t M, int64_t N, int64_t K, 
     const int64_t tn = bid % tiles_n;
     bid /= tiles_n;
     const int64_t tm = bid % tiles_m, z = bid / tiles_m;
-    A += z * sa;
-    B += z * sb;
     C += z * sc;
-    const int64_t m0 = tm * GBM, n0 = tn * GBN;
-    const bool amf = sam <= sak;  // consecutive threads along m (else along k)
-    const bool bnf = sbn <= sbk;  // consecutive threads along n (else along k)
+    const int64_t m0 = tm * BM, n0 = tn * BN;
+    // Element i of this thread's share of a chunk: (am + i amst, ak + i akst)
+    // of A, consecutive threads along the dimension of the smaller stride.
+    // Rows past M and columns past N read the last one instead (they only
+    // reach outputs that are not stored).
+    const bool amf = sam <= sak, bnf = sbn <= sbk;
+    const int am = amf ? tid % BM : tid / BK, ak = amf ? tid / BM : tid % BK;
+    const int bn = bnf ? tid % BN : tid / BK, bk = bnf ? tid / BN : tid % BK;
+    const int amst = amf ? 0 : GNT / BK, akst = amf ? GNT / BM : 0;
+    const int bnst = bnf ? 0 : GNT / BK, bkst = bnf ? GNT / BN : 0;
+    const T *pa[AE], *pb[BE];
+#pragma unroll
+    for (int i = 0; i < AE; ++i) {
+        const int64_t m = m0 + am + i * amst;
+        pa[i] = A + z * sa + (m < M ? m : M - 1) * sam + (ak + i * akst) * sak;
+    }
+#pragma unroll
+    for (int i = 0; i < BE; ++i) {
+        const int64_t n = n0 + bn + i * bnst;
+        pb[i] = B + z * sb + (n < N ? n : N - 1) * sbn + (bk + i * bkst) * sbk;
+    }
+    const int64_t stepa = BK * sak, stepb = BK * sbk;
+    // The chunk at k0 into registers.  When the whole chunk lies
+    // below K nothing but loads and pointer additions is issued; else every
+    // load past K takes the operand's first element and is zeroed when it is
+    // staged (a load under a branch would be waited for at the branch's end,
+    // before the MFMAs it should overlap).
     T ra[AE], rb[BE];
-    auto load = [&](int64_t k0) {
+    auto load = [&](auto whole, int64_t k0) {
 #pragma unroll
         for (int i = 0; i < AE; ++i) {
-            const int e = tid + GNT * i;
-            const int m = amf ? e % GBM : e / GBK, k = amf ? e / GBM : e % GBK;
-            ra[i] = (m0 + m < M && k0 + k < K) ? A[(m0 + m) * sam + (k0 + k) * sak] : czero<T>();
+            ra[i] = ldg(whole || k0 + ak + i * akst < K ? pa[i] : A);
+            pa[i] += stepa;
         }
 #pragma unroll
         for (int i = 0; i < BE; ++i) {
-            const int e = tid + GNT * i;
-            const int n = bnf ? e % GBN : e / GBK, k = bnf ? e / GBN : e % GBK;
-            rb[i] = (n0 + n < N && k0 + k < K) ? B[(k0 + k) * sbk + (n0 + n) * sbn] : czero<T>();
+            rb[i] = ldg(whole || k0 + bk + i * bkst < K ? pb[i] : B);
+            pb[i] += stepb;
         }
     };
-    auto store = [&](int buf) {
-        R *a = As + buf * 2 * GBK * LA, *b = Bs + buf * 2 * GBK * LB;
+    const int wa = ak * LA + am, wast = akst * LA + amst;
+    const int wb = BK * LA + bk * LB + bn, wbst = bkst * LB + bnst;
+    auto store = [&](auto buf, auto whole, int64_t k0) {
+        T *l = lds + buf * BUF;
 #pragma unroll
-        for (int i = 0; i < AE; ++i) {
-            const int e = tid + GNT * i;
-            const int m = amf ? e % GBM : e / GBK, k = amf ? e / GBM : e % GBK;
-            a[k * LA + m] = ra[i].x;
-            a[GBK * LA + k * LA + m] = ra[i].y;
-        }
+        for (int i = 0; i < AE; ++i)
+            l[wa + i * wast] = whole || k0 + ak + i * akst < K ? ra[i] : czero<T>();
 #pragma unroll
-        for (int i = 0; i < BE; ++i) {
-            const int e = tid + GNT * i;
-            const int n = bnf ? e % GBN : e / GBK, k = bnf ? e / GBN : e % GBK;
-            b[k * LB + n] = rb[i].x;
-            b[GBK * LB + k * LB + n] = rb[i].y;
-        }
+        for (int i = 0; i < BE; ++i)
+            l[wb + i * wbst] = whole || k0 + bk + i * bkst < K ? rb[i] : czero<T>();
     };
     V cr[TNW][TMW], ci[TNW][TMW];
 #pragma unroll
@@ -367,35 +403,67 @@ __global__ void __launch_bounds__(GNT) k_zgemm(int64_t M, int64_t N, int64_t K, 
             cr[p][q] = V{0, 0, 0, 0};
             ci[p][q] = V{0, 0, 0, 0};
         }
-    const int64_t nk = (K + GBK - 1) / GBK;
-    load(0);
-    store(0);
-    __syncthreads();
-    for (int64_t kc = 0; kc < nk; ++kc) {
-        const int buf = (int)(kc & 1);
-        if (kc + 1 < nk) load((kc + 1) * GBK);  // in flight during this chunk's MFMAs
-        const R *a = As + buf * 2 * GBK * LA, *b = Bs + buf * 2 * GBK * LB;
+    const int fa = lk * LA + wm * (BM / 2) + lr, fb = BK * LA + lk * LB + wn * (BN / 2) + lr;
+    // fragments of k-step ks of a buffer, read one k-step ahead of the MFMAs
+    // that use them
+    T af[2][TNW], bf[2][TMW];
+    auto frag = [&](auto buf, int ks, int s) {
+        const T *l = lds + buf * BUF + 4 * ks * LA, *m = lds + buf * BUF + 4 * ks * LB;
 #pragma unroll
-        for (int ks = 0; ks < GBK / 4; ++ks) {
-            const int k = 4 * ks + lk;
-            T af[TNW], bf[TMW];
+        for (int p = 0; p < TNW; ++p) af[s][p] = m[fb + 16 * p];
 #pragma unroll
-            for (int p = 0; p < TNW; ++p) {
-                const int n = wn * (GBN / 2) + 16 * p + lr;
-                af[p] = mk(b[k * LB + n], b[GBK * LB + k * LB + n]);
+        for (int q = 0; q < TMW; ++q) bf[s][q] = l[fa + 16 * q];
+    };
+    const int64_t nk = (K + BK - 1) / BK, nfull = K / BK;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    // Chunk c, in buffer buf = c mod 2.  fast: chunk c + 1 exists and is whole.
+    auto chunk = [&](auto buf, auto fast, int64_t c) {
+        using Next = std::integral_constant<int, 1 - buf>;
+        if (fast || c + 1 < nk) load(fast, (c + 1) * BK);  // in flight during this chunk's MFMAs
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int s = ks & 1;
+            if (ks + 1 < KS) {
+                frag(buf, ks + 1, s ^ 1);
+            } else if (fast || c + 1 < nk) {
+                // The next chunk is staged and its first fragments are read
+                // before the last k-step's MFMAs, which hide both: the other
+                // buffer was last read before the previous barrier, and every
+                // read of this one is complete at this barrier.
+                store(Next(), fast, (c + 1) * BK);
+                __syncthreads();
+                frag(Next(), 0, s ^ 1);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            // the four real products of cmma4, each over all tiles before the
+            // next, so that an accumulator's two updates are far apart
 #pragma unroll
-            for (int q = 0; q < TMW; ++q) {
-                const int m = wm * (GBM / 2) + 16 * q + lr;
-                bf[q] = mk(a[k * LA + m], a[GBK * LA + k * LA + m]);
-            }
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int p = 0; p < TNW; ++p)
+                for (int p = 0; p < TNW; ++p)
 #pragma unroll
-                for (int q = 0; q < TMW; ++q) cmma4<R>(af[p], bf[q], cr[p][q], ci[p][q]);
+                    for (int q = 0; q < TMW; ++q) {
+                        cr[p][q] = h == 0 ? mf<R>::mma(af[s][p].x, bf[s][q].x, cr[p][q])
+                                          : mf<R>::mma(-af[s][p].y, bf[s][q].y, cr[p][q]);
+                        ci[p][q] = h == 0 ? mf<R>::mma(af[s][p].x, bf[s][q].y, ci[p][q])
+                                          : mf<R>::mma(af[s][p].y, bf[s][q].x, ci[p][q]);
+                    }
         }
-        if (kc + 1 < nk) store(buf ^ 1);  // buf ^ 1 was last read before the previous barrier
-        __syncthreads();
+    };
+    load(std::false_type(), 0);
+    store(I0(), std::false_type(), 0);
+    __syncthreads();
+    frag(I0(), 0, 0);
+    int64_t c = 0;
+    for (; c + 2 < nfull; c += 2) {
+        chunk(I0(), std::true_type(), c);
+        chunk(I1(), std::true_type(), c + 1);
+    }
+    if (c + 1 < nfull) chunk(I0(), std::true_type(), c++);
+    for (; c < nk; ++c) {
+        if (c & 1) chunk(I1(), std::false_type(), c);
+        else chunk(I0(), std::false_type(), c);
     }
     const T alpha = mk((R)alpha_.x, (R)alpha_.y), beta = mk((R)beta_.x, (R)beta_.y);
 #pragma unroll
@@ -404,8 +472,8 @@ __global__ void __launch_bounds__(GNT) k_zgemm(int64_t M, int64_t N, int64_t K, 
         for (int q = 0; q < TMW; ++q)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t n = n0 + wn * (GBN / 2) + 16 * p + mf<R>::row(lane, r);
-                const int64_t m = m0 + wm * (GBM / 2) + 16 * q + lr;
+                const int64_t n = n0 + wn * (BN / 2) + 16 * p + mf<R>::row(lane, r);
+                const int64_t m = m0 + wm * (BM / 2) + 16 * q + lr;
                 if (m < M && n < N) {
                     T *c = C + m * scm + n * scn;
                     T v = cmul(alpha, mk((R)cr[p][q][r], (R)ci[p][q][r]));
@@ -552,25 +620,33 @@ hipError_t launch_zgemm(qob_dtype dt, int64_t M, int64_t N, int64_t K, const voi
         // no product: C = beta C, element by element (beta = 0 writes zeros)
         return hipErrorInvalidValue;
     }
-    const int64_t tmn = (M + GBM - 1) / GBM, tnn = (N + GBN - 1) / GBN;
-    const int64_t nblk = tmn * tnn * batch;
-    if (nblk > 0x7fffffff) return hipErrorInvalidValue;
-    const size_t esz = dt == QOB_C64 ? 8 : 4;
-    const size_t lds = (size_t)2 * 2 * GBK * ((GBM + GPAD) + (GBN + GPAD)) * esz;
+#define QOB_ZG(RR, BMV, BNV, WV)                                                                               \
+    do {                                                                                                        \
+        const int64_t tmn = (M + BMV - 1) / BMV, tnn = (N + BNV - 1) / BNV, nblk = tmn * tnn * batch;           \
+        if (nblk > 0x7fffffff) return hipErrorInvalidValue;                                                     \
+        const size_t lds = (size_t)2 * GBK * ((BMV + GPAD) + (BNV + GPAD)) * sizeof(cplx<RR>);                  \
+        auto k = k_zgemm<RR, BMV, BNV, WV>;                                                                    \
+        hipError_t e = raise_lds(k, lds);                                                                       \
+        if (e != hipSuccess) return e;                                                                          \
+        hipLaunchKernelGGL(k, dim3((unsigned)nblk), dim3(GNT), lds, s, M, N, K, (const cplx<RR> *)A, sam, sak, sa, \
+                           (const cplx<RR> *)B, sbk, sbn, sb, (cplx<RR> *)C, scm, scn, sc, tmn, tnn, alpha, beta, bz); \
+        return hipGetLastError();                                                                               \
+    } while (0)
+    // Tile: a launch takes about (rounds of tiles over the CUs) x (tile area),
+    // the 32 x 32 tile at 0.92 of the 64 x 32 tile's rate (68 against 72
+    // TFLOP/s at 4096^3 in ComplexF64).  With few tiles per CU the smaller
+    // one also keeps more waves in flight (700^3: 52 against 58 us).
+    const int64_t ncu = device_cu_count();
+    const int64_t nl = ((M + 63) / 64) * ((N + 31) / 32) * batch, ns = ((M + 31) / 32) * ((N + 31) / 32) * batch;
+    const int64_t rl = (nl + ncu - 1) / ncu, rs = (ns + ncu - 1) / ncu;
+    const bool large = rl > 2 && 200 * rl < 109 * rs;
     if (dt == QOB_C64) {
-        auto k = k_zgemm<double>;
-        hipError_t e = raise_lds(k, lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k, dim3((unsigned)nblk), dim3(GNT), lds, s, M, N, K, (const double2 *)A, sam, sak, sa,
-                           (const double2 *)B, sbk, sbn, sb, (double2 *)C, scm, scn, sc, tmn, tnn, alpha, beta, bz);
-    } else {
-        auto k = k_zgemm<float>;
-        hipError_t e = raise_lds(k, lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k, dim3((unsigned)nblk), dim3(GNT), lds, s, M, N, K, (const float2 *)A, sam, sak, sa,
-                           (const float2 *)B, sbk, sbn, sb, (float2 *)C, scm, scn, sc, tmn, tnn, alpha, beta, bz);
+        if (large) QOB_ZG(double, 64, 32, 3);
+        QOB_ZG(double, 32, 32, 4);
     }
-    return hipGetLastError();
+    if (large) QOB_ZG(float, 64, 32, 3);
+    QOB_ZG(float, 32, 32, 4);
+#undef QOB_ZG
 }
 
 hipError_t launch_zgemv(qob_dtype dt, const void *F, int64_t m, int64_t n, const void *x, void *y, void *part,

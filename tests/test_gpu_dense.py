@@ -218,6 +218,31 @@ def test_qob_gemm(transa, dtype):
     assert np.array_equal(dN.to_numpy(), np.zeros((m, n)))
 
 
+# (m, n, k) around the GEMM's tiles (32 and 64 by 32) and its chunks of 16 k;
+# the last three have enough tiles for the 64 x 32 tile
+GEMM_EDGES = [(1, 1, 1), (31, 33, 15), (33, 31, 16), (32, 65, 17), (65, 32, 33), (63, 64, 48),
+              (1345, 1217, 31), (1344, 1216, 32), (2111, 800, 18)]
+
+
+@pytest.mark.parametrize("mnk", GEMM_EDGES)
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("dtype", DTS)
+def test_qob_gemm_tile_edges(mnk, transa, dtype):
+    g = np.random.default_rng(11)
+    m, n, k = mnk
+    A = (cg(g, k, m) if transa else cg(g, m, k)).astype(dtype).astype(complex)
+    B = cg(g, k, n).astype(dtype).astype(complex)
+    C0 = cg(g, m, n).astype(dtype).astype(complex)
+    dA, dB = Q.DeviceArray.from_numpy(A, dtype), Q.DeviceArray.from_numpy(B, dtype)
+    opA = A.T if transa else A
+    for beta in (0.0, 0.5j):
+        dC = Q.DeviceArray.from_numpy(C0 if beta else np.full((m, n), np.nan + 0j), dtype)
+        _lib.call("qob_gemm", Q.context().h, dA.qdt, transa, m, n, k, _lib.c64(0.5 - 1j), dA.ptr, dB.ptr,
+                  _lib.c64(beta), dC.ptr, None)
+        want = (0.5 - 1j) * (opA @ B) + (beta * C0 if beta else 0)
+        assert rel(dC.to_numpy(), want) < TOLS[dtype]
+
+
 @pytest.mark.parametrize("kind", ["dense", "sparse"])
 def test_mixed_element_types_like_reference(kind):
     """test/test_operators_lazytensor.jl:239-253: a LazyTensor on the reference
