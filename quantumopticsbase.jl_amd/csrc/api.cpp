@@ -1833,6 +1833,95 @@ static qob_status chain_step(const Apply &ap, OpNode &owner, const std::string &
     return QOB_OK;
 }
 
+// A pass of one factor, over `total` elements: the mode kernels (k_mode_fib
+// without an LDS round trip, k_mode_chunk for n1 < 16) pad the factor to
+// multiples of 16 both ways, the group kernel to multiples of 8 and 2.  Up to
+// width 16 the mode kernels run at copy speed; wider ones, measured on a
+// 2160^2 / 5940^2 / 1600^2 ComplexF64 rho with n1 >= 16 (mode / group kernel):
+// width 20: 46 / 27 us, 33: 376 / 345 us, 40: 27 / 38 us; with n1 = 1 width 33:
+// 928 / 369 us, 40: 61 / 33 us.  On a few thousand elements (a Ket) the group
+// kernel has too few tiles for its factor's load.
+static bool mode_better(int64_t total, int64_t n1, int d) {
+    const int f = (d + 15) / 16 * 16, g8 = (d + 7) / 8 * 8, g2 = (d + 1) / 2 * 2;
+    return d <= 16 || total < (1 << 16) || (n1 >= 16 && 10 * f * f < 17 * g8 * g2);
+}
+
+// Square dense factors of any width up to ANY_MAXD (in site order) through
+// passes that each apply the factors of a group of consecutive sites
+// (k_ltany.hip).  A group takes the next factor while two workgroups of its
+// tiles share a CU's LDS, or while the whole product stays one pass (left
+// application of (33, 12, 15) in ComplexF64, one workgroup per CU: 609 us in
+// one pass, 730 us in two; chain of modes 1546 us); with few tiles, while
+// they stay small.  done is left false when some factor does not fit a pass.
+static qob_status apply_lt_any(const Apply &ap, const std::vector<ChainOp> &ops, const std::vector<int64_t> &sh,
+                               const void *in, void *out, cd alpha, cd beta, bool &done) {
+    done = false;
+    const int N = (int)sh.size();
+    const int64_t D = prod(sh, 0, N);
+    std::vector<AnyPass> passes;
+    for (size_t i = 0; i < ops.size();) {
+        // the group starts at its first factor's site, or at site 1 when the
+        // dimensions before it are too few rows for a tile
+        int s0 = ops[i].site;
+        if (ap.lead == 1 && prod(sh, 0, s0) < 16) s0 = 0;
+        const int64_t n1 = ap.lead * prod(sh, 0, s0);
+        if (n1 != 1 && n1 < 16) return QOB_OK;
+        AnyPass best;
+        size_t j = i;
+        for (size_t k = i; k < ops.size() && k - i < ANY_MAXMODES; ++k) {
+            AnyPass S;
+            const int64_t P = prod(sh, s0, ops[k].site + 1);
+            if (P > (1 << 14)) break;
+            S.n1 = n1;
+            S.P = (int)P;
+            S.n3 = prod(sh, ops[k].site + 1, N) * ap.trail;
+            for (size_t t = i; t <= k; ++t) {
+                const ChainOp &c = ops[t];
+                AnyMode &M = S.m[S.nmodes++];
+                M.d = (int)c.d_in;
+                M.m1 = (int)prod(sh, s0, c.site);
+                QOB_TRY(dense_dev(*c.f->de, c.f->var ^ (ap.trans ? V_T : V_N), ap.dt, M.A));
+            }
+            int dsum = 0;
+            for (int t = 0; t < S.nmodes; ++t) dsum += S.m[t].d;
+            AnyPass F = S;
+            const size_t lds = any_plan(ap.dt, F);
+            if (!lds) break;
+            const bool whole = i == 0 && k + 1 == ops.size();
+            const int64_t nt = n1 == 1 ? (S.n3 + F.units - 1) / F.units : F.nrb * S.n3;
+            if (k == i || (nt >= 64 ? lds <= 80 * 1024 || whole : P <= 2560 && dsum <= 64)) {
+                best = S;
+                j = k + 1;
+            }
+        }
+        if (j == i) return QOB_OK;
+        passes.push_back(best);
+        i = j;
+    }
+    void *t[2] = {nullptr, nullptr};
+    const size_t bytes = (size_t)(D * ap.lead * ap.trail) * esize(ap.dt);
+    if (passes.size() > 1) QOB_TRY(ws_get(ap.ctx, ap.s, WS_TMP1, bytes, t[0]));
+    if (passes.size() > 2) QOB_TRY(ws_get(ap.ctx, ap.s, WS_TMP2, bytes, t[1]));
+    const void *src = in;
+    for (size_t i = 0; i < passes.size(); ++i) {
+        const bool last = i + 1 == passes.size();
+        void *dst = last ? out : t[i & 1];
+        const AnyPass &S = passes[i];
+        const AnyMode &M = S.m[0];
+        if (S.nmodes == 1 && M.d == S.P && mode_better(ap.lead * ap.trail * D, S.n1, M.d)) {
+            QOB_TRY(run_mode(ap, M.A, M.d, M.d, src, dst, S.n1, S.n3, last ? alpha : cd(1, 0), last ? beta : cd(0, 0)));
+            src = dst;
+            continue;
+        }
+        hipError_t e = launch_lt_any(ap.dt, passes[i], src, dst, d2(last ? alpha : cd(1, 0)),
+                                     d2(last ? beta : cd(0, 0)), ap.s);
+        if (e != hipSuccess) return fail(QOB_EHIP, "LazyTensor site-group launch: %s", hipGetErrorString(e));
+        src = dst;
+    }
+    done = true;
+    return QOB_OK;
+}
+
 // LazyTensor through the tensor-product chain: _tp_sum_matmul!
 // (src/operators_lazytensor.jl:443-488) with the operator list of
 // _tpops_tuple (:523-535, square identities dropped) followed by the
@@ -1961,6 +2050,12 @@ static qob_status apply_lt_chain(const Apply &ap, OpNode &op, const void *in, vo
         // n_ops == 0: result = alpha * b + beta * result (:453-458)
         if (Din != Dout) return fail(QOB_EDIM, "LazyTensor without factors on unequal dimensions");
         return apply_embed(ap, Dout, Din, in, out, a, beta);
+    }
+    if (g_fused_lt && sh_in == sh_out && Din < (1 << 30)) {
+        bool ok = true, done = false;
+        for (const ChainOp &c : ops) ok = ok && c.f->kind == K_DENSE && c.d_in == c.d_out && c.d_in <= ANY_MAXD;
+        if (ok) QOB_TRY(apply_lt_any(ap, ops, sh_in, in, out, a, beta, done));
+        if (done) return QOB_OK;
     }
     // shapes after each step
     std::vector<int64_t> cur = sh_in;

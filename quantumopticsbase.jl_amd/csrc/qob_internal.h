@@ -332,6 +332,33 @@ hipError_t launch_lt_reg(qob_dtype dt, const FusedModes &M, const void *in, void
 hipError_t launch_lt_reg_tile(qob_dtype dt, const FusedModes &M, const void *in, void *out, int64_t ntiles,
                               int64_t nrb, int64_t ld, double2 alpha, double2 beta, hipStream_t s);
 
+// Dense factors of any width up to 40 on a group of consecutive sites, applied
+// in one pass over the view (n1, P, n3) (k_ltany.hip).  The caller sets n1
+// (1, or at least 16), n3, P, nmodes and each mode's d, factor A and m1, the
+// product of the group's dimensions before it; any_plan fills in the rest.
+enum { ANY_MAXMODES = 16, ANY_MAXD = 40 };
+struct AnyMode {
+    int d = 0, m1 = 1, m1p = 1;  // width, stride in the tile, stride in LDS
+    int pf = 0;                  // fibres per unit of the tile
+    const void *A = nullptr;     // d x d, column-major
+};
+struct AnyPass {
+    int64_t n1 = 1, n3 = 1;
+    int P = 1, nmodes = 0;
+    int W = 1, lw = 0;          // rows of a tile and their log2 (1, 0 for n1 == 1)
+    int units = 1;              // blocks of P elements (n1 == 1) or rows (W) of a tile
+    int nrb = 1;                // row tiles of n1
+    int nfac = 0, ntile = 0;    // LDS elements of the padded factors and of a tile
+    int lin = 0;                // 1: the result leaves through LDS, in memory order
+    int padd = 0;               // 1: one LDS element of padding after every m[0].d elements
+    uint32_t fm0 = 0, fl0 = 0;  // FastDiv of m[0].d
+    uint32_t fmr = 0, flr = 0;  // FastDiv of nrb
+    AnyMode m[ANY_MAXMODES];
+};
+size_t any_plan(qob_dtype dt, AnyPass &S);
+hipError_t launch_lt_any(qob_dtype dt, AnyPass S, const void *in, void *out, double2 alpha, double2 beta,
+                         hipStream_t s);
+
 // Fused reductions over a square gather plan (FP64 partials, one per block):
 //   mode 0: sum_J conj(u[J]) (H v)[J]          (expect / bilinear on a Ket)
 //   mode 1: sum_J (H V[:, J])[J], V n x n       (tr(H V), expect on rho)

@@ -351,3 +351,61 @@ def test_register_chain_kernel(case, dtype):
         finally:
             _tune("fused_reg", old)
     assert rel(outs[0], outs[1]) < TOLS[dtype]
+
+
+# square dense factors on groups of sites (k_ltany.hip): odd and even widths,
+# widths around 8, 16 and 24 and the widest, sites without a factor before,
+# between and after, a first factor behind a short prefix, several passes
+ANY_CASES = [
+    ((5, 7, 6), (1, 2, 3)), ((4, 3, 33), (1, 3)), ((40, 2, 7), (1, 3)), ((2, 3, 11, 9), (3, 4)),
+    ((20, 13, 5, 6), (1, 2, 3, 4)), ((3, 17, 2), (2,)), ((24, 23), (1, 2)), ((8, 9), (1, 2)), ((25, 1, 18), (1, 2, 3)),
+    ((3, 2, 3, 2, 3, 2), (1, 2, 3, 4, 5, 6)), ((18, 4, 39), (1, 3)), ((10, 30, 33), (1, 2, 3)),
+]
+
+
+@pytest.mark.parametrize("case", range(len(ANY_CASES)))
+@pytest.mark.parametrize("dtype", DTS)
+def test_lazytensor_site_groups(case, dtype):
+    """Every state form against the oracle, 1 / few / many columns and rows
+    (ragged row tiles), and the mode-by-mode chain (fused_lt = 0)."""
+    dims, idx = ANY_CASES[case]
+    g = np.random.default_rng(500 + case)
+    oop = rand_lt(g, dims, dims, idx, ("dense",) * len(idx))
+    qop = to_q(oop)
+    for ncols, ab in ((1, (1.0, 0.0)), (18, (complex(0.3, 0.8), complex(-0.5, 0.25))), (77, (1.0, -0.5))):
+        run_all_paths(oop, qop, g, *ab, dtype, TOLS[dtype], ncols=ncols)
+        run_all_paths(O.dagger(oop), Q.dagger(qop), g, *ab, dtype, TOLS[dtype], ncols=ncols)
+    D, nc = int(np.prod(dims)), 300  # enough tiles for the large-state rules
+    B = Q.Operator(qop.basis_r, gb(nc), cg(g, D, nc), dtype)
+    T = Q.Operator(gb(nc), qop.basis_l, cg(g, nc, D), dtype)
+    outs = []
+    for fused in (1, 0):
+        old = _tune("fused_lt", fused)
+        try:
+            R = Q.Operator(qop.basis_l, gb(nc), np.full((D, nc), np.nan + 0j), dtype)
+            S = Q.Operator(gb(nc), qop.basis_r, np.full((nc, D), np.nan + 0j), dtype)
+            outs.append((Q.mul_(R, qop, B, 0.5j, 0.0).to_numpy(), Q.mul_(S, T, qop, 0.5j, 0.0).to_numpy()))
+        finally:
+            _tune("fused_lt", old)
+    assert rel(outs[0][0], outs[1][0]) < TOLS[dtype]
+    assert rel(outs[0][1], outs[1][1]) < TOLS[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTS)
+def test_lazytensor_site_groups_nan_stays_in_its_fibres(dtype):
+    """A NaN or infinity in the state reaches the elements that depend on it
+    and no others (padding lanes and clamped reads multiply nothing)."""
+    dims, idx = (5, 7, 3), (1, 3)
+    g = np.random.default_rng(3)
+    oop = rand_lt(g, dims, dims, idx, ("dense",) * 2)
+    qop = to_q(oop)
+    x = cg(g, 105, 40)
+    for bad in (np.nan, np.inf):
+        y = x.copy()
+        y[2 + 5 * 3 + 35 * 1, 7] = bad
+        R = Q.Operator(qop.basis_l, gb(40), np.zeros((105, 40), complex), dtype)
+        got = Q.mul_(R, qop, Q.Operator(qop.basis_r, gb(40), y, dtype), 1.0, 0.0).to_numpy()
+        hit = ~np.isfinite(got)
+        want = np.zeros((105, 40), bool)
+        want[[a + 5 * 3 + 35 * c for a in range(5) for c in range(3)], 7] = True
+        assert np.array_equal(hit, want)
