@@ -1405,7 +1405,9 @@ static qob_status lazy_plan(OpNode &owner, const std::string &key, const std::ve
 // group's weight w_F(J) = sum_t c_t prod_s v_{t,s}[bit_s(J)] is stored as a
 // constant or as tables over windows of <= 8 bits (program layout in
 // k_qubit.hip).  Returns false when a term does not fit this form.
-int g_qubit_split = 0;  // 1: high-bit flips in a second, strided pass; 0: partner tiles read in one pass
+// 1: the flips of every bit above the tile in a second, strided pass; 0: by
+// qubit_split_of (partner tiles read in one pass, long single states in two)
+int g_qubit_split = 0;
 
 struct QubitProgHost {
     std::vector<int32_t> prog;     // flips inside a tile (all flips when prog_hi is empty)
@@ -1413,10 +1415,17 @@ struct QubitProgHost {
     std::vector<cd> vals;
 };
 
-// tb: tile bits of the launch; states longer than a tile (and at most 2 tb
-// bits) get their high-bit flips in a separate program.
+// Second pass of a state: flips of bits >= s in strided tiles of 2^tb states,
+// c of their bits the lowest ones (s == 0: no second pass).
+struct QubitSplitSpec {
+    int s = 0, tb = 0;
+    int c(int nbits) const { return tb - (nbits - s); }
+};
+
+// tb: tile bits of the first pass.  With a second pass, the groups whose flips
+// stay inside its tiles go to a separate program.
 static bool compile_qubit(int nbits, const std::vector<TermSpec> &terms, QubitProgHost &Q, int tb,
-                          int split_flag = -1) {
+                          const QubitSplitSpec &sp) {
     struct QT {
         cd coef;
         uint32_t F;
@@ -1463,7 +1472,9 @@ static bool compile_qubit(int nbits, const std::vector<TermSpec> &terms, QubitPr
         std::map<int, std::vector<cd>> win;
     };
     std::vector<GroupOut> outs[2];  // [0]: first pass, [1]: high-bit pass
-    const bool split = (split_flag < 0 ? g_qubit_split : split_flag) && nbits > tb && nbits <= 2 * tb;
+    auto second = [&](uint32_t F) {
+        return sp.s > 0 && (F >> sp.s) != 0 && ((F & ((1u << sp.s) - 1u)) >> sp.c(nbits)) == 0;
+    };
     for (auto &gq : groups) {
         GroupOut go;
         go.F = gq.first;
@@ -1496,7 +1507,7 @@ static bool compile_qubit(int nbits, const std::vector<TermSpec> &terms, QubitPr
                 tab[idx] += w;
             }
         }
-        outs[(split && (go.F >> tb) != 0) ? 1 : 0].push_back(std::move(go));
+        outs[second(go.F) ? 1 : 0].push_back(std::move(go));
     }
     auto put_cd = [](std::vector<int32_t> &P, cd z) {
         int32_t w[4];
@@ -1540,7 +1551,8 @@ struct QubitPlan {
     bool ok = false;
     int nbits = 0;
     int tbits = 12;
-    int32_t hi_off = -1;  // offset of the high-bit program in prog, or -1
+    int32_t hi_off = -1;  // offset of the second pass's program in prog, or -1
+    QubitSplitSpec hi;
     DevBuf prog, vals;
     qob_dtype dt = QOB_C64;
     std::shared_ptr<RefreshMap> rmap;
@@ -1626,11 +1638,44 @@ int g_qubit_enable = 1;
 extern int g_qubit_tbits;
 int qubit_tbits(qob_dtype dt);
 
+// log2 of the tile of a single state (or of each column of a matrix).
+static int qubit_single_tbits(int nbits, qob_dtype dt) {
+    // Small tiles put a single state on more CUs: 18 sites 9.5 (2^12) -> 6.8 us
+    // (2^10) in ComplexF64, 9.7 (2^11) -> 7.7 us in ComplexF32; above 2^20
+    // states ComplexF32 does better with half the partner tiles (21 sites: 22
+    // against 24 us), ComplexF64 with more workgroups per CU (21 sites: 35
+    // against 40 us).
+    if (g_qubit_tbits) return g_qubit_tbits;
+    return dt == QOB_C64 || nbits <= 20 ? 10 : 11;
+}
+
+// The second pass of one state of nbits bits whose first pass has 2^tb-state
+// tiles.
+static QubitSplitSpec qubit_split_of(int nbits, int tb, qob_dtype dt, bool single) {
+    QubitSplitSpec sp;
+    if (g_qubit_split) {
+        if (nbits > tb && nbits <= 2 * tb) sp.s = sp.tb = tb;
+        return sp;
+    }
+    // 64 KB tiles of 9 high bits and a run of 128 bytes.  Two passes read or
+    // write the state's size five times; one pass does so once per flip
+    // dimension that leaves the L2 as well (nbits - 17 of them), but needs one
+    // launch and, below 64 MB of state, reads them from the Infinity Cache.
+    // Chains, three states in turn, one / two passes: ComplexF64 21 sites 35 /
+    // 37 us, 22: 81 / 72, 23: 178 / 132; ComplexF32 23: 78 / 81, 24: 163 / 147.
+    if (single && nbits >= (dt == QOB_C64 ? 22 : 24)) {
+        sp.tb = dt == QOB_C64 ? 12 : 13;
+        sp.s = nbits - 9;
+    }
+    return sp;
+}
+
 static qob_status qubit_plan(OpNode &op, bool trans, qob_dtype dt, hipStream_t s, std::shared_ptr<QubitPlan> &out,
                              bool nosplit = false) {
     std::lock_guard<std::mutex> g(op.mu);
-    const int tbd = qubit_tbits(dt);
-    const int split = nosplit ? 0 : g_qubit_split;
+    const int tbd = g_qubit_tbits;
+    // a plan without a second pass serves both where there would be none
+    const int split = nosplit && (g_qubit_split || op.m >= (1 << 22)) ? -1 : g_qubit_split;
     const std::string k = "qb:" + std::to_string(op.version) + (trans ? ":T:" : ":N:") + std::to_string((int)dt) +
                           ":" + std::to_string(tbd) + ":" + std::to_string(split);
     auto it = op.qplans.find(k);
@@ -1641,14 +1686,14 @@ static qob_status qubit_plan(OpNode &op, bool trans, qob_dtype dt, hipStream_t s
         std::vector<cd> base;
         int nbits = 0;
         QubitProgHost H;
-        // a state smaller than the tile gets a tile of its own size, at least
-        // 2^11 (one workgroup with half or more of its lanes busy)
         const bool terms = qubit_terms(op, trans, specs, store, nbits, &base);
-        const int tb = nbits < tbd ? std::max(std::min(tbd, 11), nbits) : tbd;
-        if (terms && compile_qubit(nbits, specs, H, tb, split)) {
+        const int tb = qubit_single_tbits(nbits, dt);
+        const QubitSplitSpec sp = nosplit ? QubitSplitSpec() : qubit_split_of(nbits, tb, dt, true);
+        if (terms && compile_qubit(nbits, specs, H, tb, sp)) {
             std::vector<int32_t> all = H.prog;
             if (!H.prog_hi.empty()) {
                 P->hi_off = (int32_t)all.size();
+                P->hi = sp;
                 all.insert(all.end(), H.prog_hi.begin(), H.prog_hi.end());
             }
             QOB_TRY(P->prog.upload(all.data(), all.size() * 4));
@@ -1669,7 +1714,7 @@ static qob_status qubit_plan(OpNode &op, bool trans, qob_dtype dt, hipStream_t s
                     std::vector<TermSpec> unit = specs;
                     for (size_t q = 0; q < unit.size(); ++q) unit[q].coef = (q == t) ? base[q] : cd(0, 0);
                     QubitProgHost U;
-                    same = compile_qubit(nbits, unit, U, tb, split) && U.prog.size() == H.prog.size() &&
+                    same = compile_qubit(nbits, unit, U, tb, sp) && U.prog.size() == H.prog.size() &&
                            U.prog_hi.size() == H.prog_hi.size() && U.vals.size() == H.vals.size();
                     if (!same) break;
                     std::vector<int32_t> ua = U.prog;
@@ -2095,15 +2140,14 @@ static qob_status apply_qubit(const Apply &ap, OpNode &op, const void *in, void 
     S.nbits = P->nbits;
     S.prog_off = 0;
     S.prog_hi_off = P->hi_off;
+    S.hi_shift = P->hi.s;
     S.in = in;
     S.out = out;
-    hipError_t e = hipSuccess;
-    if (P->hi_off >= 0)  // high-bit flips first: out = alpha * high + beta * out
-        e = launch_qubit_hi_cols(ap.dt, S, ap.trail, P->tbits, (const int32_t *)P->prog.p, P->vals.p, d2(alpha),
-                                 d2(beta), ap.s);
-    if (e == hipSuccess)
-        e = launch_qubit_cols(ap.dt, S, ap.trail, P->tbits, (const int32_t *)P->prog.p, P->vals.p, d2(alpha),
-                              d2(beta), make_double2(0, 0), ap.s);
+    hipError_t e = launch_qubit_cols(ap.dt, S, ap.trail, P->tbits, (const int32_t *)P->prog.p, P->vals.p, d2(alpha),
+                                     d2(beta), make_double2(0, 0), ap.s);
+    if (e == hipSuccess && P->hi_off >= 0)  // high-bit flips: out += alpha * high
+        e = launch_qubit_hi_cols(ap.dt, S, ap.trail, P->hi.tb, (const int32_t *)P->prog.p, P->vals.p, d2(alpha),
+                                 ap.s);
     if (e != hipSuccess) return fail(QOB_EHIP, "qubit launch: %s", hipGetErrorString(e));
     done = true;
     return QOB_OK;
@@ -3526,7 +3570,7 @@ qob_status qob_batch_create(qob_ctx ctx, int n, const qob_op *ops, qob_dtype dt,
         std::vector<std::vector<RowLists>> store;
         int nb = 0;
         QubitProgHost H;
-        if (!qubit_terms(*ops[j]->node, false, specs, store, nb) || !compile_qubit(nb, specs, H, B->tbits))
+        if (!qubit_terms(*ops[j]->node, false, specs, store, nb) || !compile_qubit(nb, specs, H, B->tbits, qubit_split_of(nb, B->tbits, dt, false)))
             return fail(QOB_EUNSUPPORTED, "operator %d is not a qubit sum of monomial factors", j);
         // rebase the value offsets of this state's programs into the shared pool
         const int32_t vb = (int32_t)vals.size();
@@ -3608,6 +3652,7 @@ qob_status qob_batch_bind(qob_ctx ctx, qob_batch b, int slot, void *const *in, v
         S[j].nbits = b->nbits[j];
         S[j].prog_off = b->prog_off[j];
         S[j].prog_hi_off = b->prog_hi_off[j];
+        S[j].hi_shift = b->tbits;
         S[j].in = in[j];
         S[j].out = out[j];
     }
@@ -3624,15 +3669,13 @@ qob_status qob_batch_apply(qob_ctx ctx, qob_batch b, int slot, qob_c64 alpha, qo
                            qob_stream s) {
     if (!ctx || !b) return fail(QOB_EARG, "null argument");
     if (slot < 0 || slot >= QOB_BATCH_SLOTS || !b->bound[slot]) return fail(QOB_EARG, "slot %d not bound", slot);
-    hipError_t e = hipSuccess;
-    if (b->nitems_hi > 0)  // high-bit flips first: out = alpha * high + beta * out
+    hipError_t e = launch_qubit(b->dt, (const QubitStateDev *)b->slot[slot].p, (const QubitItemDev *)b->items.p,
+                                b->nitems, b->tbits, (const int32_t *)b->prog.p, b->vals.p, d2(alpha), d2(beta),
+                                d2(gamma), strm(ctx, s), &b->xs);
+    if (e == hipSuccess && b->nitems_hi > 0)  // high-bit flips: out += alpha * high
         e = launch_qubit_hi(b->dt, (const QubitStateDev *)b->slot[slot].p, (const QubitItemDev *)b->items_hi.p,
-                            b->nitems_hi, b->tbits, (const int32_t *)b->prog.p, b->vals.p, d2(alpha), d2(beta),
-                            strm(ctx, s), &b->xs_hi);
-    if (e == hipSuccess)
-        e = launch_qubit(b->dt, (const QubitStateDev *)b->slot[slot].p, (const QubitItemDev *)b->items.p, b->nitems,
-                         b->tbits, (const int32_t *)b->prog.p, b->vals.p, d2(alpha), d2(beta), d2(gamma),
-                         strm(ctx, s), &b->xs);
+                            b->nitems_hi, b->tbits, (const int32_t *)b->prog.p, b->vals.p, d2(alpha), strm(ctx, s),
+                            &b->xs_hi);
     if (e != hipSuccess) return fail(QOB_EHIP, "batch apply: %s", hipGetErrorString(e));
     return QOB_OK;
 }

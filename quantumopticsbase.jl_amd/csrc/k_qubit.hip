@@ -177,18 +177,13 @@ struct LoMap {
 };
 
 // Tile coordinates of the second pass (strided tile, see k_qubit_hi).
-template <int TBITS> struct HiMap {
+struct HiMap {
     uint32_t mid, lowmask;  // lowmask = 2^c - 1
-    int c;
-    __device__ __forceinline__ uint32_t J(uint32_t q) const {
-        return ((q >> c) << TBITS) | mid | (q & lowmask);
-    }
-    __device__ __forceinline__ bool in_tile(uint32_t F) const {
-        return ((F & ((1u << TBITS) - 1u)) >> c) == 0;
-    }
-    __device__ __forceinline__ uint32_t fq(uint32_t F) const {
-        return ((F >> TBITS) << c) | (F & ((1u << TBITS) - 1u));
-    }
+    int c, s;
+    __device__ __forceinline__ uint32_t J(uint32_t q) const { return ((q >> c) << s) | mid | (q & lowmask); }
+    // the second pass's program holds flips inside its tiles only
+    __device__ __forceinline__ bool in_tile(uint32_t) const { return true; }
+    __device__ __forceinline__ uint32_t fq(uint32_t F) const { return ((F >> s) << c) | (F & lowmask); }
 };
 
 // acc[k] += w_F(J) * in[J ^ F] over the groups of one program, for the
@@ -278,12 +273,7 @@ __device__ __forceinline__ void qb_run(const int32_t *__restrict__ pg, const T *
             const int32_t *rn = r + 8 * (g + 1 < nconst ? g + 1 : g);
             const uint32_t Fn = (uint32_t)rn[0];
             const T wn = rec_weight<T>(rn + 4);
-            if (m.in_tile(F)) {
-                qb_uniform<T, NTH, EPT>(wt, (const char *)tile, (tid ^ m.fq(F)) * (uint32_t)sizeof(T), acc);
-            } else {
-#pragma unroll
-                for (int k = 0; k < EPT; ++k) acc[k] = cfma(wt, ldg(in + (m.J(tid + k * NTH) ^ F)), acc[k]);
-            }
+            qb_uniform<T, NTH, EPT>(wt, (const char *)tile, (tid ^ m.fq(F)) * (uint32_t)sizeof(T), acc);
             F = Fn;
             wt = wn;
         }
@@ -395,10 +385,6 @@ __global__ void __launch_bounds__(NTH) k_qubit(const QubitStateDev *__restrict__
         const uint32_t base = (uint32_t)w.tile << tb;
         const T *__restrict__ in = (const T *)S.in;
         T *__restrict__ out = (T *)S.out;
-        // a second pass already wrote alpha * high + beta * out: add to it
-        const bool add_out = S.prog_hi_off >= 0;
-        const bool bz = beta_zero && !add_out;
-        const T beff = add_out ? mk((typename real_of<T>::type)1, (typename real_of<T>::type)0) : beta;
         // the lane keeps its own elements in registers as well: flips of
         // the register bits (e = tid + k NTH, k = 0..EPT-1), the diagonal
         // and the gamma term read them there
@@ -419,6 +405,16 @@ __global__ void __launch_bounds__(NTH) k_qubit(const QubitStateDev *__restrict__
         for (int k = 0; k < EPT; ++k) acc[k] = czero<T>();
         const LoMap m{base, (uint32_t)tsize - 1u, tb};
         qb_run<T, NTH, EPT, true>(prog + S.prog_off, vals, tile, in, m, xv, acc, far_tiles);
+        if (flags & 512) {  // a second pass reads the result: kept in the caches
+#pragma unroll
+            for (int k = 0; k < EPT; ++k) {
+                T *o = out + base + tid + k * NTH;
+                T r = cmul(alpha, acc[k]);
+                if (!beta_zero) r = cfma(beta, ldg(o), r);
+                stg(o, r);
+            }
+            continue;
+        }
 #pragma unroll
         for (int k = 0; k < EPT; ++k) {
             const int e = tid + k * NTH;
@@ -426,7 +422,7 @@ __global__ void __launch_bounds__(NTH) k_qubit(const QubitStateDev *__restrict__
                 const uint32_t J = base + (uint32_t)e;
                 T r = cmul(alpha, acc[k]);
                 if (!gamma_zero) r = cfma(gamma, sizeof(T) == 8 ? xv[k] : tile[e], r);
-                if (!bz) r = cfma(beff, ldg(out + J), r);
+                if (!beta_zero) r = cfma(beta, ldg(out + J), r);
                 stg_stream(out + J, r);
             }
         }
@@ -657,9 +653,6 @@ __global__ void __launch_bounds__(NTH) k_qubit_pair(const QubitStateDev *__restr
         const uint32_t base = (uint32_t)w.tile << tb;
         const T *__restrict__ in = (const T *)S.in;
         T *__restrict__ out = (T *)S.out;
-        const bool add_out = S.prog_hi_off >= 0;
-        const bool bz = beta_zero && !add_out;
-        const T beff = add_out ? mk(1.0f, 0.0f) : beta;
         T xv[EPT];
 #pragma unroll
         for (int j = 0; j < EPT / 2; ++j) {
@@ -685,18 +678,34 @@ __global__ void __launch_bounds__(NTH) k_qubit_pair(const QubitStateDev *__restr
 #pragma unroll
         for (int k = 0; k < EPT; ++k) acc[k] = czero<T>();
         qb_run_pair<NTH, EPT>(prog + S.prog_off, vals, tile, in, base, (uint32_t)tsize - 1u, tb, xv, acc);
+        if (flags & 512) {  // a second pass reads the result: kept in the caches
+#pragma unroll
+            for (int j = 0; j < EPT / 2; ++j) {
+                T *p = out + base + 2 * (tid + j * NTH);
+                T v0 = cmul(alpha, acc[2 * j]), v1 = cmul(alpha, acc[2 * j + 1]), o0, o1;
+                if (!beta_zero) {
+                    qp_load<true>((const char *)p, o0, o1);
+                    v0 = cfma(beta, o0, v0);
+                    v1 = cfma(beta, o1, v1);
+                }
+                qb_f4 o;
+                o.x = v0.x; o.y = v0.y; o.z = v1.x; o.w = v1.y;
+                *(QOB_GLOBAL qb_f4 *)p = o;
+            }
+            continue;
+        }
 #pragma unroll
         for (int j = 0; j < EPT / 2; ++j) {
             const int e = 2 * (tid + j * NTH);
             if (e < tsize) {
                 T rr[2];
                 T old[2];
-                if (!bz) qp_load<true>((const char *)(out + base + e), old[0], old[1]);
+                if (!beta_zero) qp_load<true>((const char *)(out + base + e), old[0], old[1]);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     T v = cmul(alpha, acc[2 * j + h]);
                     if (!gamma_zero) v = cfma(gamma, xv[2 * j + h], v);
-                    if (!bz) v = cfma(beff, old[h], v);
+                    if (!beta_zero) v = cfma(beta, old[h], v);
                     rr[h] = v;
                 }
                 qb_f4 o;
@@ -707,23 +716,23 @@ __global__ void __launch_bounds__(NTH) k_qubit_pair(const QubitStateDev *__restr
     }
 }
 
-// Second pass: flips of bits above the tile.  With h = nbits - TBITS high
-// bits and c = TBITS - h low bits, tile m holds the 2^TBITS basis states
-//   J(q) = (q >> c) << TBITS | m << c | (q & (2^c - 1)),
+// Second pass: flips of bits >= s = hi_shift (and of the lowest c bits).  With
+// h = nbits - s high bits and c = TBITS - h low bits, tile m holds the
+// 2^TBITS basis states
+//   J(q) = (q >> c) << s | m << c | (q & (2^c - 1)),
 // i.e. every combination of the high bits times a contiguous run of 2^c
-// states, so a flip of high bits (and of bits below c) stays inside the
-// tile.  Writes out = alpha * sum_high + beta * out.
+// states, so these flips stay inside the tile.  Adds
+// out += alpha * sum_high to the first pass's result.
 template <typename T, int NTH, int TBITS>
 __global__ void __launch_bounds__(NTH) k_qubit_hi(const QubitStateDev *__restrict__ states,
                                                   const QubitItemDev *__restrict__ items, int nitems,
                                                   const int32_t *__restrict__ prog, const T *__restrict__ vals,
-                                                  double2 alpha_, double2 beta_, int flags, QubitStateDev single,
+                                                  double2 alpha_, int flags, QubitStateDev single,
                                                   int ntiles1, QubitSplit xs) {
     constexpr int EPT = (1 << TBITS) / NTH;
     extern __shared__ unsigned char lds_raw[];
     T *tile = (T *)lds_raw;
-    const T alpha = to_t<T>(alpha_), beta = to_t<T>(beta_);
-    const bool beta_zero = flags & 1;
+    const T alpha = to_t<T>(alpha_);
     const int tid = threadIdx.x;
     const ItemWalk wk = qb_walk(flags, xs, nitems);
     for (int it = wk.it; it < wk.end; it += wk.step) {
@@ -740,9 +749,8 @@ __global__ void __launch_bounds__(NTH) k_qubit_hi(const QubitStateDev *__restric
             S.in = (const T *)single.in + ((int64_t)cidx << single.nbits);
             S.out = (T *)single.out + ((int64_t)cidx << single.nbits);
         }
-        const int h = S.nbits - TBITS;
-        const int c = TBITS - h;
-        const HiMap<TBITS> m{(uint32_t)w.tile << c, (1u << c) - 1u, c};
+        const int c = TBITS - (S.nbits - S.hi_shift);
+        const HiMap m{(uint32_t)w.tile << c, (1u << c) - 1u, c, S.hi_shift};
         const T *__restrict__ in = (const T *)S.in;
         T *__restrict__ out = (T *)S.out;
         __syncthreads();
@@ -760,9 +768,7 @@ __global__ void __launch_bounds__(NTH) k_qubit_hi(const QubitStateDev *__restric
 #pragma unroll
         for (int k = 0; k < EPT; ++k) {
             const uint32_t J = m.J((uint32_t)(tid + k * NTH));
-            T r = cmul(alpha, acc[k]);
-            if (!beta_zero) r = cfma(beta, ldg(out + J), r);
-            stg(out + J, r);
+            stg_stream(out + J, cfma(alpha, acc[k], ldg(out + J)));
         }
     }
 }
@@ -901,7 +907,7 @@ static unsigned qubit_grid(int nth, int nitems) {
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>(g, nitems));
 }
 
-// log2 of the tile; 0: 12 for ComplexF64 (one partner-tile read per element
+// log2 of a batch's tile; 0: 12 for ComplexF64 (one partner-tile read per element
 // fewer than 2^11: 3.1 reads per element instead of 4.1 on the 256-chain
 // batch, 10% faster), 11 for ComplexF32 (bound by issue, not traffic: larger
 // tiles measured slower)
@@ -939,15 +945,19 @@ static hipError_t launch_qubit_any(qob_dtype dt, const QubitStateDev *states, co
     if (tbits > 13) tbits = 13;
     const size_t tile_bytes = (size_t)(1 << tbits) * (dt == QOB_C64 ? 16 : 8);
     if (tile_bytes > 160 * 1024) return hipErrorInvalidValue;
-    const int nth = qubit_nth(dt, tbits);
-    const unsigned g = qubit_grid(nth, nitems);
+    // where every item has a CU of its own, twice the threads (18 sites: 6.8 ->
+    // 6.1 us in ComplexF64, 7.7 -> 6.6 us in ComplexF32)
+    const int nth = std::min(1024, qubit_nth(dt, tbits) * (!g_qubit_nth && !states && nitems <= device_cu_count() ? 2 : 1));
+    // the first of two passes reads few partner tiles: no run of tiles to keep
+    // in the L2, so every item gets a workgroup
+    const unsigned g = !states && single.prog_hi_off >= 0 ? (unsigned)nitems : qubit_grid(nth, nitems);
     // a second buffer only pays where a workgroup walks several items
     const bool dbuf = g_qubit_dbuf && 2 * tile_bytes <= 160 * 1024 && (int64_t)g < nitems;
     const size_t lds = dbuf ? 2 * tile_bytes : tile_bytes;
     QubitSplit ws;
     const int flags = (beta.x == 0.0 && beta.y == 0.0 ? 1 : 0) | (gamma.x == 0.0 && gamma.y == 0.0 ? 2 : 0) |
                       qubit_walk_flags(nitems, g, xs, ws) | (g_qubit_ntfar ? 16 | ((g_qubit_ntfar - 1) << 5) : 0) |
-                      (dbuf ? 256 : 0);
+                      (dbuf ? 256 : 0) | (!states && single.prog_hi_off >= 0 ? 512 : 0);
 #define QOB_QB(TT, NT, TB)                                                                                    \
     do {                                                                                                      \
         auto kfn = k_qubit<TT, NT, TB>;                                                                       \
@@ -1019,15 +1029,15 @@ static hipError_t launch_qubit_any(qob_dtype dt, const QubitStateDev *states, co
 
 static hipError_t launch_qubit_hi_any(qob_dtype dt, const QubitStateDev *states, const QubitItemDev *items,
                                       int nitems, int tbits, const int32_t *prog, const void *vals, double2 alpha,
-                                      double2 beta, hipStream_t s, QubitStateDev single, int ntiles1,
+                                      hipStream_t s, QubitStateDev single, int ntiles1,
                                       const QubitSplit *xs) {
     if (nitems == 0) return hipSuccess;
     if (tbits < 10 || tbits > 13) return hipErrorInvalidValue;
     const size_t lds = (size_t)(1 << tbits) * (dt == QOB_C64 ? 16 : 8);
     const int nth = qubit_nth(dt, tbits);
-    const unsigned g = qubit_grid(nth, nitems);
+    const unsigned g = states ? qubit_grid(nth, nitems) : (unsigned)nitems;
     QubitSplit ws;
-    const int flags = (beta.x == 0.0 && beta.y == 0.0 ? 1 : 0) | qubit_walk_flags(nitems, g, xs, ws);
+    const int flags = qubit_walk_flags(nitems, g, xs, ws);
 #define QOB_QH(TT, NT, TB)                                                                                    \
     do {                                                                                                      \
         auto kfn = k_qubit_hi<TT, NT, TB>;                                                                    \
@@ -1039,7 +1049,7 @@ static hipError_t launch_qubit_hi_any(qob_dtype dt, const QubitStateDev *states,
             lds_set = 160 * 1024;                                                                             \
         }                                                                                                     \
         hipLaunchKernelGGL(kfn, dim3(g), dim3(NT), lds, s, states, items, nitems, prog, (const TT *)vals,     \
-                           alpha, beta, flags, single, ntiles1, ws);                                          \
+                           alpha, flags, single, ntiles1, ws);                                          \
         return hipGetLastError();                                                                             \
     } while (0)
 #define QOB_QH_NT(TT, TB)                                  \
@@ -1063,18 +1073,19 @@ static hipError_t launch_qubit_hi_any(qob_dtype dt, const QubitStateDev *states,
 }
 
 hipError_t launch_qubit_hi(qob_dtype dt, const QubitStateDev *states, const QubitItemDev *items, int nitems, int tbits,
-                           const int32_t *prog, const void *vals, double2 alpha, double2 beta, hipStream_t s,
+                           const int32_t *prog, const void *vals, double2 alpha, hipStream_t s,
                            const QubitSplit *xs) {
-    return launch_qubit_hi_any(dt, states, items, nitems, tbits, prog, vals, alpha, beta, s, QubitStateDev(), 1, xs);
+    return launch_qubit_hi_any(dt, states, items, nitems, tbits, prog, vals, alpha, s, QubitStateDev(), 1, xs);
 }
 
 hipError_t launch_qubit_hi_cols(qob_dtype dt, QubitStateDev single, int64_t ncols, int tbits, const int32_t *prog,
-                                const void *vals, double2 alpha, double2 beta, hipStream_t s) {
-    if (single.nbits <= tbits || single.prog_hi_off < 0) return hipSuccess;
+                                const void *vals, double2 alpha, hipStream_t s) {
+    if (single.prog_hi_off < 0) return hipSuccess;
+    if (single.nbits <= tbits || single.nbits - single.hi_shift > tbits) return hipErrorInvalidValue;
     const int64_t ntiles = (int64_t)1 << (single.nbits - tbits);
     const int64_t nitems = ntiles * ncols;
     if (nitems >= (1ll << 31)) return hipErrorInvalidValue;
-    return launch_qubit_hi_any(dt, nullptr, nullptr, (int)nitems, tbits, prog, vals, alpha, beta, s, single,
+    return launch_qubit_hi_any(dt, nullptr, nullptr, (int)nitems, tbits, prog, vals, alpha, s, single,
                                (int)ntiles, nullptr);
 }
 

@@ -287,8 +287,8 @@ bool fused_supported(qob_dtype dt, const FusedModes &M);
 struct QubitStateDev {
     int32_t nbits = 0;          // state length 2^nbits
     int32_t prog_off = 0;       // program of the flips inside a tile (all flips if prog_hi_off < 0)
-    int32_t prog_hi_off = -1;   // program of the flips of bits above the tile (second pass), or -1
-    int32_t pad_ = 0;
+    int32_t prog_hi_off = -1;   // program of the second pass (flips of bits >= hi_shift), or -1
+    int32_t hi_shift = 0;
     const void *in = nullptr;
     void *out = nullptr;
 };
@@ -312,13 +312,14 @@ hipError_t launch_qubit_cols(qob_dtype dt, QubitStateDev single, int64_t ncols, 
                              const void *vals, double2 alpha, double2 beta, double2 gamma, hipStream_t s);
 hipError_t launch_qubit_axpy(qob_dtype dt, const QubitStateDev *states, const QubitItemDev *items, int nitems,
                              int tbits, double2 a, hipStream_t s);
-// Second pass over strided tiles (high-bit flips) for states with prog_hi_off >= 0:
-// out = alpha * high + beta * out; the first pass then adds to out.
+// Second pass over strided tiles of 2^tbits states (flips of bits >= hi_shift,
+// see k_qubit_hi) for states with prog_hi_off >= 0: out += alpha * high, after
+// the first pass.
 hipError_t launch_qubit_hi(qob_dtype dt, const QubitStateDev *states, const QubitItemDev *items, int nitems, int tbits,
-                           const int32_t *prog, const void *vals, double2 alpha, double2 beta, hipStream_t s,
+                           const int32_t *prog, const void *vals, double2 alpha, hipStream_t s,
                            const QubitSplit *xs = nullptr);
 hipError_t launch_qubit_hi_cols(qob_dtype dt, QubitStateDev single, int64_t ncols, int tbits, const int32_t *prog,
-                                const void *vals, double2 alpha, double2 beta, hipStream_t s);
+                                const void *vals, double2 alpha, hipStream_t s);
 // out (D x ncols) = alpha * (A_n ... A_1) in + beta * out
 hipError_t launch_lt_fused(qob_dtype dt, const FusedModes &M, const void *in, void *out, int64_t ncols,
                            double2 alpha, double2 beta, hipStream_t s, int64_t tile_ld = 0,

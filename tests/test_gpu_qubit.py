@@ -440,3 +440,52 @@ def test_complexf32_pair_lanes_batch_bitwise():
     for other in got[1:]:
         for a, b in zip(got[0], other):
             assert np.array_equal(a, b)
+
+
+def _long_terms(g, L):
+    """Neighbour and long-range flips, weights that change with high and low
+    bits, and rows without an entry, over the whole chain."""
+    terms = [(0.3, (i + 1, i + 2), [PAULI["x"], PAULI["x"]]) for i in range(0, L - 1, 2)]
+    terms += [(0.2 + 0.1j, (i + 1,), [PAULI["z"]]) for i in range(0, L, 3)]
+    terms += [(0.7, (L,), [PAULI["y"]]), (0.4j, (L - 1,), [PAULI["p"]]), (-0.6, (L - 4, L - 2), [PAULI["x"], PAULI["z"]]),
+              (0.5, (1, L), [PAULI["x"], PAULI["x"]]), (0.25, (2, L - 3), [PAULI["x"], PAULI["x"]]),
+              (0.35, (6, L - 1), [PAULI["x"], PAULI["x"]]), (0.15, (11, 12), [PAULI["x"], PAULI["y"]])]
+    return terms
+
+
+@pytest.mark.parametrize("L,dtype,tol", [(21, np.complex128, 1e-13), (22, np.complex128, 1e-13), (23, np.complex128, 1e-13),
+                                         (24, np.complex64, 1e-6), (25, np.complex64, 1e-6)])
+def test_long_single_state_two_passes(L, dtype, tol):
+    """A single state long enough for the strided second pass against the
+    same sum as a batch of one (always one pass), with beta = 0 over NaN and
+    general alpha and beta."""
+    g = np.random.default_rng(L)
+    H, _, B = build_pair(L, _long_terms(g, L))
+    n = 2 ** L
+    psi = Q.Ket(B, cg(g, n), dtype)
+    bt = Q.Batch([H], dtype)
+    for al, be in ((1.0, 0.0), (0.3 - 0.8j, 0.5 + 0.1j)):
+        y0 = np.full(n, np.nan + 0j) if be == 0 else cg(g, n)
+        got = Q.mul_(Q.Ket(B, y0, dtype), H, psi, al, be).to_numpy()
+        out = Q.DeviceArray.from_numpy(y0, dtype)
+        bt.bind(0, [psi.data], [out])
+        bt.apply(0, al, be, 0.0)
+        want = out.to_numpy()
+        assert np.all(np.isfinite(got))
+        assert O.rel_frobenius(got, want) < tol
+
+
+@pytest.mark.parametrize("L", [1, 5, 9, 10, 11, 18, 19])
+@pytest.mark.parametrize("dtype,tol", [(np.complex128, 1e-13), (np.complex64, 1e-6)])
+def test_single_state_tiles_match_one_batch(L, dtype, tol):
+    """Tile and thread rules of a single state over lengths around them."""
+    g = np.random.default_rng(60 + L)
+    H, _, B = build_pair(L, random_pauli_sum(g, L, 12))
+    n = 2 ** L
+    psi = Q.Ket(B, cg(g, n), dtype)
+    out = Q.DeviceArray(n, dtype)
+    bt = Q.Batch([H], dtype)
+    bt.bind(0, [psi.data], [out])
+    bt.apply(0, 0.3 - 0.8j, 0.0, 0.0)
+    got = Q.mul_(Q.Ket(B, np.full(n, np.nan + 0j), dtype), H, psi, 0.3 - 0.8j, 0.0).to_numpy()
+    assert O.rel_frobenius(got, out.to_numpy()) < tol
