@@ -150,19 +150,28 @@ __global__ void __launch_bounds__(BS) k_reduce1(int64_t n, const T *__restrict__
     if (threadIdx.x == 0) partials[blockIdx.x] = r;
 }
 
-// final stage: one block sums nparts partials; mode 1 writes sqrt into a double
+// final stage: one block sums the partials of one or two sets; mode 1 writes
+// sqrt into a double.  flag: out lies in pinned host memory, and the host
+// waits for seq there, which the release makes visible after the results.
 template <int MODE>
-__global__ void __launch_bounds__(BS) k_reduce2(int nparts, const double2 *__restrict__ partials, void *out) {
-    __shared__ double2 sh[BS / 64];
-    double2 acc = make_double2(0, 0);
-    for (int i = threadIdx.x; i < nparts; i += BS) {
-        acc.x += partials[i].x;
-        acc.y += partials[i].y;
+__global__ void __launch_bounds__(BS) k_reduce2(RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq) {
+    __shared__ double2 sh[2][BS / 64];
+    double2 acc = make_double2(0, 0), acc2 = make_double2(0, 0);
+    for (int i = threadIdx.x; i < a.n; i += BS) {
+        acc.x += a.p[i].x;
+        acc.y += a.p[i].y;
     }
-    double2 r = block_sum(acc, sh);
+    for (int i = threadIdx.x; i < b.n; i += BS) {
+        acc2.x += b.p[i].x;
+        acc2.y += b.p[i].y;
+    }
+    const double2 r = block_sum(acc, sh[0]);
+    const double2 r2 = b.n ? block_sum(acc2, sh[1]) : make_double2(0, 0);
     if (threadIdx.x == 0) {
         if (MODE == 1) *(double *)out = sqrt(r.x);
         else *(double2 *)out = r;
+        if (b.n) ((double2 *)out)[1] = r2;
+        if (flag) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -314,30 +323,34 @@ hipError_t launch_convert(qob_dtype from, const void *src, qob_dtype to, void *d
 }
 
 template <int MODE>
-static hipError_t reduce_any(qob_dtype dt, int64_t n, const void *x, const void *y, int64_t step,
-                             double2 *partials, void *out, hipStream_t s) {
+static hipError_t reduce1(qob_dtype dt, int64_t n, const void *x, const void *y, int64_t step, double2 *partials,
+                          hipStream_t s) {
     const int g = reduce_blocks(n);
     if (dt == QOB_C64)
         hipLaunchKernelGGL((k_reduce1<double2, MODE>), g, BS, 0, s, n, (const double2 *)x, (const double2 *)y, step, partials);
     else
         hipLaunchKernelGGL((k_reduce1<float2, MODE>), g, BS, 0, s, n, (const float2 *)x, (const float2 *)y, step, partials);
-    hipLaunchKernelGGL(k_reduce2<MODE>, 1, BS, 0, s, g, (const double2 *)partials, out);
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_partials(int nparts, const double2 *partials, double2 *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_reduce2<0>, 1, BS, 0, s, nparts, partials, (void *)out);
+hipError_t launch_partials(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
+                           hipStream_t s) {
+    if (mode == RED_DOT) return reduce1<0>(dt, n, x, y, 1, partials, s);
+    if (mode == RED_NORM) return reduce1<1>(dt, n, x, x, 1, partials, s);
+    return reduce1<2>(dt, n, x, x, n + 1, partials, s);
+}
+
+hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq, hipStream_t s) {
+    if (mode == RED_NORM) hipLaunchKernelGGL(k_reduce2<1>, 1, BS, 0, s, a, b, out, flag, seq);
+    else hipLaunchKernelGGL(k_reduce2<0>, 1, BS, 0, s, a, b, out, flag, seq);
     return hipGetLastError();
 }
 
-hipError_t launch_dot(qob_dtype dt, int64_t n, const void *x, const void *y, double2 *partials, double2 *out, hipStream_t s) {
-    return reduce_any<0>(dt, n, x, y, 1, partials, out, s);
-}
-hipError_t launch_nrm2(qob_dtype dt, int64_t n, const void *x, double2 *partials, double *out, hipStream_t s) {
-    return reduce_any<1>(dt, n, x, x, 1, partials, out, s);
-}
-hipError_t launch_trace(qob_dtype dt, int64_t n, const void *A, double2 *partials, double2 *out, hipStream_t s) {
-    return reduce_any<2>(dt, n, A, A, n + 1, partials, out, s);
+hipError_t launch_reduce(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
+                         void *out, hipStream_t s) {
+    const hipError_t e = launch_partials(dt, mode, n, x, y, partials, s);
+    if (e != hipSuccess) return e;
+    return launch_final(mode, RedSet{partials, reduce_blocks(n)}, RedSet{}, out, nullptr, 0, s);
 }
 
 hipError_t launch_scale_by_inv_norm(qob_dtype dt, int64_t n, const double *nrm, void *x, hipStream_t s) {

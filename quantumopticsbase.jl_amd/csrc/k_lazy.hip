@@ -168,7 +168,7 @@ __device__ __forceinline__ double2 block_sum256(double2 v) {
 template <typename T, int MODE>
 __global__ void __launch_bounds__(256) k_gather_dot(GatherPlanDev P, const T *__restrict__ u, const T *__restrict__ v,
                                                     int64_t n, double2 *__restrict__ partials) {
-    double2 r = make_double2(0, 0);
+    double2 r = make_double2(0, 0), p = make_double2(0, 0);
     for (int64_t J = blockIdx.x * (int64_t)256 + threadIdx.x; J < n; J += (int64_t)gridDim.x * 256) {
         Digits dg{0, 0};
         T acc;
@@ -177,6 +177,9 @@ __global__ void __launch_bounds__(256) k_gather_dot(GatherPlanDev P, const T *__
             const T a = u[J];
             r.x += (double)a.x * acc.x + (double)a.y * acc.y;
             r.y += (double)a.x * acc.y - (double)a.y * acc.x;
+            const T b = v[J];  // sum conj(u) v, which a variance needs as well
+            p.x += (double)a.x * b.x + (double)a.y * b.y;
+            p.y += (double)a.x * b.y - (double)a.y * b.x;
         } else {
             const T *col = v + J * n;
             acc = eval_terms<T, true>((uint32_t)J, P, dg, [&](int64_t K) { return col[K]; });
@@ -186,6 +189,11 @@ __global__ void __launch_bounds__(256) k_gather_dot(GatherPlanDev P, const T *__
     }
     const double2 t = block_sum256(r);
     if (threadIdx.x == 0) partials[blockIdx.x] = t;
+    if (MODE == 0) {
+        __syncthreads();
+        const double2 q = block_sum256(p);
+        if (threadIdx.x == 0) partials[gridDim.x + blockIdx.x] = q;
+    }
 }
 
 }  // namespace

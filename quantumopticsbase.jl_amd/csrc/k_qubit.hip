@@ -776,7 +776,9 @@ __global__ void __launch_bounds__(NTH) k_qubit_hi(const QubitStateDev *__restric
 // sum_J conj(u[J]) (H v)[J] for one state (expect / variance): the same tile
 // walk as k_qubit with the store replaced by an FP64 reduction; one partial
 // per workgroup (fixed item order, so the result is deterministic).  High
-// flips read partner tiles from v in global memory.
+// flips read partner tiles from v in global memory.  u and v's own tile are
+// in registers anyway, so sum conj(u) v, which a variance needs of the same
+// vectors, goes to partials[gridDim.x ...] for four more FMAs per element.
 template <typename T, int NTH, int TBITS>
 __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__restrict__ u, int ntiles,
                                                    const int32_t *__restrict__ prog, const T *__restrict__ vals,
@@ -784,12 +786,12 @@ __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__r
     constexpr int EPT = (1 << TBITS) / NTH;
     extern __shared__ unsigned char lds_raw[];
     T *tile = (T *)lds_raw;
-    __shared__ double2 red[NTH / 64];
+    __shared__ double2 red[2][NTH / 64];
     const int tid = threadIdx.x;
     const int tb = S.nbits < TBITS ? S.nbits : TBITS;
     const int tsize = 1 << tb;
     const T *__restrict__ v = (const T *)S.in;
-    double rx = 0, ry = 0;
+    double rx = 0, ry = 0, px = 0, py = 0;
     for (int it = blockIdx.x; it < ntiles; it += gridDim.x) {
         const uint32_t base = (uint32_t)it << tb;
         T xv[EPT];
@@ -814,6 +816,8 @@ __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__r
                 const T a = u[base + e];
                 rx += (double)a.x * acc[k].x + (double)a.y * acc[k].y;
                 ry += (double)a.x * acc[k].y - (double)a.y * acc[k].x;
+                px += (double)a.x * xv[k].x + (double)a.y * xv[k].y;
+                py += (double)a.x * xv[k].y - (double)a.y * xv[k].x;
             }
         }
     }
@@ -821,16 +825,21 @@ __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__r
     for (int off = 32; off > 0; off >>= 1) {
         rx += __shfl_down(rx, off, 64);
         ry += __shfl_down(ry, off, 64);
+        px += __shfl_down(px, off, 64);
+        py += __shfl_down(py, off, 64);
     }
-    if ((tid & 63) == 0) red[tid >> 6] = make_double2(rx, ry);
+    if ((tid & 63) == 0) {
+        red[0][tid >> 6] = make_double2(rx, ry);
+        red[1][tid >> 6] = make_double2(px, py);
+    }
     __syncthreads();
-    if (tid == 0) {
+    if (tid < 2) {
         double2 t = make_double2(0, 0);
         for (int w = 0; w < NTH / 64; ++w) {
-            t.x += red[w].x;
-            t.y += red[w].y;
+            t.x += red[tid][w].x;
+            t.y += red[tid][w].y;
         }
-        partials[blockIdx.x] = t;
+        partials[tid * gridDim.x + blockIdx.x] = t;
     }
 }
 

@@ -3,7 +3,7 @@
 //
 // qob_normalize_ket (api.cpp) keeps its two-stage FP64 norm partials and the
 // norm itself in the per-stream workspace, which grows on first use.  This
-// variant runs the same kernels (k_blas1.hip: launch_nrm2, then
+// variant runs the same kernels (k_blas1.hip: launch_reduce, then
 // launch_scale_by_inv_norm) on a fixed file-scope device array instead:
 //   scratch[0 .. NOALLOC_PARTS)   stage-1 partial sums (double2 each)
 //   scratch[NOALLOC_PARTS]        the norm (a double in the first half)
@@ -75,7 +75,7 @@ extern "C" qob_status qob_normalize_ket_noalloc(qob_ctx ctx, qob_dtype dt, int64
     if (!base) return set_error(QOB_EHIP, "no-allocation scratch not set up on device %d", ctx_device(ctx));
     hipStream_t st = ctx_stream(ctx, s);
     double *nrm = (double *)(base + NOALLOC_PARTS);
-    hipError_t e = launch_nrm2(dt, n, x, base, nrm, st);
+    hipError_t e = launch_reduce(dt, RED_NORM, n, x, x, base, nrm, st);
     if (e == hipSuccess) e = launch_scale_by_inv_norm(dt, n, nrm, x, st);
     if (e != hipSuccess) return set_error(QOB_EHIP, "no-allocation normalize: %s", hipGetErrorString(e));
     return QOB_OK;

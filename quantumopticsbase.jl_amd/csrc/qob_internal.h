@@ -175,8 +175,6 @@ struct GatherPlanDev {
 hipError_t launch_refresh(qob_dtype dt, int nslots, int nvals, const int32_t *ptr, const int32_t *term,
                           const double2 *bval, const int32_t *dst, const double2 *coef, void *vals, int32_t *prog,
                           hipStream_t s);
-// Final stage of a two-stage FP64 reduction: *out = sum of nparts partials.
-hipError_t launch_reduce_partials(int nparts, const double2 *partials, double2 *out, hipStream_t s);
 // Compute units of the current device, queried once per device.
 int device_cu_count();
 hipError_t launch_scale(qob_dtype dt, int64_t n, double2 a, void *x, hipStream_t s);
@@ -186,11 +184,22 @@ hipError_t launch_axpby_copy(qob_dtype dt, int64_t n, double2 a, const void *x, 
 hipError_t launch_embed(qob_dtype dt, const void *in, int64_t ri, int64_t ci, void *out, int64_t ro, int64_t co,
                         double2 a, double2 b, hipStream_t s);
 hipError_t launch_convert(qob_dtype from, const void *src, qob_dtype to, void *dst, int64_t n, hipStream_t s);
-// reductions into a device double2/double; partials must hold reduce_partials() doubles*2
+// Two-stage FP64 reductions: reduce_blocks(n) partials of a dot product, a
+// squared norm or the trace of an n x n matrix, then their sum (the root of
+// it for RED_NORM) into out, a double2 (a double for RED_NORM).  launch_final
+// sums one or two sets of partials; with flag, out and flag are pinned host
+// memory and flag becomes seq once the results are there.
+enum RedMode { RED_DOT = 0, RED_NORM = 1, RED_TRACE = 2 };
+struct RedSet {
+    const double2 *p = nullptr;
+    int n = 0;
+};
 int reduce_blocks(int64_t n);
-hipError_t launch_dot(qob_dtype dt, int64_t n, const void *x, const void *y, double2 *partials, double2 *out, hipStream_t s);
-hipError_t launch_nrm2(qob_dtype dt, int64_t n, const void *x, double2 *partials, double *out, hipStream_t s);
-hipError_t launch_trace(qob_dtype dt, int64_t n, const void *A, double2 *partials, double2 *out, hipStream_t s);
+hipError_t launch_partials(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
+                           hipStream_t s);
+hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq, hipStream_t s);
+hipError_t launch_reduce(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
+                         void *out, hipStream_t s);
 // x *= 1/|norm| or 1/trace taken from a device scalar
 hipError_t launch_scale_by_inv_norm(qob_dtype dt, int64_t n, const double *norm, void *x, hipStream_t s);
 hipError_t launch_scale_by_inv_trace(qob_dtype dt, int64_t n, int64_t ld, const double2 *tr, void *A, hipStream_t s);

@@ -182,3 +182,66 @@ def _oracle_terms(Hq):
                                  tuple(O.OSparse.from_scipy(sp.csc_matrix(f.csc)) for f in lt.operators),
                                  lt.factor))
     return out
+
+
+@pytest.mark.parametrize("qubit", [1, 0])
+@pytest.mark.parametrize("L", [1, 4, 9, 10, 11, 17])
+def test_variance_one_pass_matches_plain(L, qubit):
+    """Both sums of a variance from one pass over the state, against the dot
+    products of the plain path: FP64 sums of 2^L products, rounding below
+    2^L eps of the sums' magnitude (<= 2e-11 at 17 sites)."""
+    g = np.random.default_rng(300 + L)
+    H, _, B = build_pair(L, random_pauli_sum(g, L, 6))
+    psi = g.standard_normal(2 ** L) + 1j * g.standard_normal(2 ** L)
+    k = Q.Ket(B, psi / np.linalg.norm(psi), np.complex128)
+    ctx = Q.context()
+    _lib.call("qob_tune_set", b"qubit_enable", qubit)
+    try:
+        e, v = Q.expect(H, k), Q.variance(H, k)
+        ctx.set_mode(Q.QOB_MODE_PLAIN)
+        ep, vp = Q.expect(H, k), Q.variance(H, k)
+    finally:
+        ctx.set_mode(Q.QOB_MODE_FUSED)
+        _lib.call("qob_tune_set", b"qubit_enable", 1)
+    scale = max(1.0, abs(ep) ** 2, abs(vp))
+    assert abs(e - ep) <= 2e-11 * scale and abs(v - vp) <= 2e-11 * scale
+
+
+def test_scalars_on_many_streams_and_behind_a_long_queue():
+    """Scalar results of threads with a stream each, more calls than result
+    slots, and a result that is waited for behind milliseconds of queued work."""
+    import concurrent.futures as cf
+    import ctypes as C
+
+    ctx = Q.context()
+    g = np.random.default_rng(7)
+    n = 4099
+    xs = [g.standard_normal(n) + 1j * g.standard_normal(n) for _ in range(8)]
+    dev = [Q.DeviceArray.from_numpy(x) for x in xs]
+
+    def one(i):
+        s = C.c_void_p()
+        _lib.call("qob_stream_create", ctx.h, C.byref(s))
+        try:
+            got = []
+            for _ in range(100):
+                nrm, d = C.c_double(), _lib.qob_c64()
+                _lib.call("qob_norm", ctx.h, Q.QOB_C64, n, dev[i].ptr, C.byref(nrm), s)
+                _lib.call("qob_dot", ctx.h, Q.QOB_C64, n, dev[i].ptr, dev[(i + 1) % 8].ptr, C.byref(d), s)
+                got.append((nrm.value, complex(d.re, d.im)))
+            return got
+        finally:
+            _lib.call("qob_stream_destroy", ctx.h, s)
+
+    with cf.ThreadPoolExecutor(8) as ex:
+        for i, got in enumerate(ex.map(one, range(8))):
+            want_n, want_d = np.linalg.norm(xs[i]), np.vdot(xs[i], xs[(i + 1) % 8])
+            for a, b in got:
+                assert abs(a - want_n) <= 1e-12 * want_n and abs(b - want_d) <= 1e-12 * want_n ** 2
+
+    big = [Q.DeviceArray(1 << 24, np.complex128) for _ in range(2)]
+    for _ in range(30):  # about 0.1 ms each
+        _lib.call("qob_copy", ctx.h, Q.QOB_C64, 1 << 24, big[0].ptr, big[1].ptr, None)
+    nrm = C.c_double()
+    _lib.call("qob_norm", ctx.h, Q.QOB_C64, n, dev[0].ptr, C.byref(nrm), None)
+    assert abs(nrm.value - np.linalg.norm(xs[0])) <= 1e-12 * nrm.value
