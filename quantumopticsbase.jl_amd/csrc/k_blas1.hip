@@ -34,7 +34,8 @@ __global__ void __launch_bounds__(BS) k_scale(int64_t n, double2 a_, T *x) {
     }
 }
 
-// slot s = sum_{p in [ptr[s], ptr[s+1])} bval[p] * coef[term[p]], in FP64;
+// slot s = sum_{p in [ptr[s], ptr[s+1])} bval[p] * coef[term[p]], in FP64
+// (term -1: bval[p] itself, a value that no coefficient enters);
 // slots below nvals are plan values of element type T, the others complex
 // doubles written into the program at word offsets dst[s - nvals]
 template <typename T>
@@ -46,7 +47,8 @@ __global__ void __launch_bounds__(BS) k_refresh(int nslots, int nvals, const int
     if (s >= nslots) return;
     double re = 0, im = 0;
     for (int p = ptr[s]; p < ptr[s + 1]; ++p) {
-        const double2 b = bval[p], c = coef[term[p]];
+        const int t = term[p];
+        const double2 b = bval[p], c = t < 0 ? make_double2(1, 0) : coef[t];
         re += b.x * c.x - b.y * c.y;
         im += b.x * c.y + b.y * c.x;
     }

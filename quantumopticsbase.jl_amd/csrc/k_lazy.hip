@@ -130,6 +130,74 @@ __global__ void __launch_bounds__(256) k_gather_rows(GatherPlanDev P, const T *_
     }
 }
 
+// The same sum from the plan's fibre tables: every table load of an element is
+// issued at once, then every gathered element.  A wave's 64 elements lie in at
+// most two fibres (fib >= 64): the factors of the sites above are scalar loads
+// of both, which leaves the vector loads to the sites below and the elements.
+template <typename T, int NP>
+__global__ void __launch_bounds__(256) k_gather_fibre(GatherPlanDev P, const T *__restrict__ in, T *__restrict__ out,
+                                                      int64_t nbatch, double2 alpha_, double2 beta_, int beta_zero) {
+    const T alpha = to_t<T>(alpha_), beta = to_t<T>(beta_);
+    const T *__restrict__ fv = (const T *)P.vals + P.fv;
+    const int32_t *__restrict__ fk = P.koff + P.fk;
+    const uint32_t n = P.n, len = P.fib + P.nf;
+    // XCD x takes a contiguous eighth of the list of chunks, which has the
+    // chunks of the top digits t = 0 .. td - 1 at the same place r side by side
+    const uint32_t k = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const uint32_t chunk = fdiv(k, P.td_m, P.td_l), t = k - chunk * P.td;
+    if (chunk * 256u >= P.ts) return;
+    const uint32_t r = chunk * 256u + threadIdx.x;
+    const uint32_t J = t * P.ts + min(r, P.ts - 1);
+    const uint32_t f = fdiv(J, P.fib_m, P.fib_l), m = J - f * P.fib;
+    const uint32_t f0 = __builtin_amdgcn_readfirstlane(f), f1 = min(f0 + 1, P.nf - 1);
+    const bool nx = f != f0;
+    const T dl = fv[m], du0 = fv[P.fib + f0], du1 = fv[P.fib + f1];
+    T v[NP + 1];
+    int32_t off[NP + 1];
+    uint32_t live = 0;
+    T lv[NP + 1], u0[NP + 1], u1[NP + 1];
+    int32_t lo[NP + 1], o0[NP + 1], o1[NP + 1];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        lv[p] = fv[len * (p + 1) + m];
+        lo[p] = fk[len * p + m];
+        u0[p] = fv[len * (p + 1) + P.fib + f0];
+        u1[p] = fv[len * (p + 1) + P.fib + f1];
+        o0[p] = fk[len * p + P.fib + f0];
+        o1[p] = fk[len * p + P.fib + f1];
+    }
+    T dv = cadd(dl, nx ? du1 : du0);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const bool l = P.has_lo >> p & 1, u = P.has_up >> p & 1;
+        const T uv = nx ? u1[p] : u0[p];
+        const int32_t uo = nx ? o1[p] : o0[p];
+        v[p] = l && u ? cmul(lv[p], uv) : (l ? lv[p] : uv);
+        bool a = lo[p] != GP_DEAD && uo != GP_DEAD;
+        if (P.skip0 >> p & 1) a = a && (lv[p].x != 0 || lv[p].y != 0) && (uv.x != 0 || uv.y != 0);
+        off[p] = a ? lo[p] + uo : 0;
+        if (P.diag >> p & 1) {
+            if (a) dv = cadd(dv, v[p]);
+            a = false;
+        }
+        live |= (uint32_t)a << p;
+    }
+    for (int64_t b = blockIdx.y; b < nbatch; b += gridDim.y) {
+        const T *ib = in + b * n;
+        T *o = out + b * n + J;
+        T x[NP + 1];
+        x[NP] = ib[J];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) x[p] = ib[(int64_t)J + off[p]];
+        T acc = czero<T>();
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            if (live >> p & 1) acc = cfma(v[p], x[p], acc);
+        if (dv.x != 0 || dv.y != 0) acc = cfma(dv, x[NP], acc);
+        if (r < P.ts) *o = axpby(alpha, acc, beta, o, beta_zero != 0);
+    }
+}
+
 template <typename T, bool SQUARE>
 __global__ void __launch_bounds__(256) k_gather_cols(GatherPlanDev P, const T *__restrict__ in, int64_t n_in,
                                                      T *__restrict__ out, int64_t n_out, int64_t nrows,
@@ -216,6 +284,25 @@ hipError_t launch_gather_rows(qob_dtype dt, const GatherPlanDev &P, const void *
                               int64_t n_out, int64_t nbatch, double2 alpha, double2 beta, hipStream_t s) {
     if (n_out == 0 || nbatch == 0) return hipSuccess;
     const int bz = (beta.x == 0.0 && beta.y == 0.0);
+    if (P.np >= 0) {
+        const uint32_t chunks = (P.ts + 255) / 256 * P.td;
+        const dim3 gf((chunks + 7) / 8 * 8, (uint32_t)(nbatch < 65535 ? nbatch : 65535));
+#define QOB_GF(NP)                                                                                                   \
+    case NP:                                                                                                         \
+        if (dt == QOB_C64)                                                                                           \
+            hipLaunchKernelGGL((k_gather_fibre<double2, NP>), gf, dim3(256), 0, s, P, (const double2 *)in,           \
+                               (double2 *)out, nbatch, alpha, beta, bz);                                             \
+        else                                                                                                         \
+            hipLaunchKernelGGL((k_gather_fibre<float2, NP>), gf, dim3(256), 0, s, P, (const float2 *)in,             \
+                               (float2 *)out, nbatch, alpha, beta, bz);                                              \
+        break;
+        switch (P.np) {
+            QOB_GF(0) QOB_GF(1) QOB_GF(2) QOB_GF(3) QOB_GF(4) QOB_GF(5) QOB_GF(6)
+            default: return hipErrorInvalidValue;
+        }
+#undef QOB_GF
+        return hipGetLastError();
+    }
     const dim3 g((uint32_t)((n_out + 255) / 256), (uint32_t)(nbatch < 65535 ? nbatch : 65535));
 #define QOB_GR(TT, SQ) \
     hipLaunchKernelGGL((k_gather_rows<TT, SQ>), g, dim3(256), 0, s, P, (const TT *)in, n_in, (TT *)out, n_out, nbatch, alpha, beta, bz)

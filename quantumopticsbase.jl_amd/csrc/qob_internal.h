@@ -165,7 +165,20 @@ struct GatherPlanDev {
     int nsites = 0;
     const int32_t *site_info = nullptr;  // per site: stride_l, m, l, d_l, m_d, l_d, stride_r, d_r
     bool square = true;
+    // Fibre tables (np >= 0), the same sum over J = m + fib * f:
+    //   out[J] = (dl[m] + du[f]) in[J] + sum_p lv_p[m] uv_p[f] in[J + lo_p[m] + uo_p[f]]
+    // Values: dl[fib], du[nf], then per part lv[fib], uv[nf], from vals + fv;
+    // offsets: per part lo[fib], uo[nf], from koff + fk (GP_DEAD: an empty row).
+    int np = -1;
+    uint32_t n = 0, fib = 1, fib_m = 0, fib_l = 0, nf = 0;
+    int32_t fv = 0, fk = 0;
+    uint32_t ts = 1, td = 1, td_m = 0, td_l = 0;  // n = ts * td: stride and count of the top digits
+    uint32_t has_lo = 0, has_up = 0;  // parts with factors below / above the fibre
+    uint32_t diag = 0;                // parts whose elements are all in[J]
+    uint32_t skip0 = 0;               // parts that read nothing where a factor is zero
 };
+constexpr int32_t GP_DEAD = INT32_MIN;
+constexpr int GP_PARTS = 6;
 
 // ------------------------------------------------------------ launchers
 // All launchers return hipSuccess or the launch error; they never allocate.

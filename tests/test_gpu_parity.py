@@ -1022,3 +1022,78 @@ def test_lazyproduct(alpha, beta, dtype, tol):
     n_o = O.OLazyProduct([lp, O.ODense(D), lp], -0.5)
     n_q = Q.LazyProduct([qlp, Q.DenseOperator(B, B, D), qlp], -0.5)
     run_all_paths(n_o, n_q, g, alpha, beta, dtype=dtype, tol=tol)
+
+
+def _sparse_factor(g, d, kind):
+    """hop: one entry per row but the last; two: up to two; diag: with an empty row; num: full diagonal."""
+    v = g.standard_normal(d) + 1j * g.standard_normal(d)
+    if kind == "hop":
+        return sp.diags(v[:-1], 1, format="csc")
+    if kind == "two":
+        return sp.csc_matrix(sp.diags(v[:-1], 1) + sp.diags(v[:-1].conj(), -1))
+    if kind == "diag":
+        M = sp.lil_matrix((d, d), dtype=np.complex128)
+        M.setdiag(v)
+        M[d // 2, d // 2] = 0
+        return sp.csc_matrix(M)
+    return sp.diags(v, 0, format="csc")
+
+
+# dims, terms of {site: factor}: sums that split between the sites below and
+# above a fibre of at least 64 elements (products, one-sided groups, diagonal
+# products, up to six parts), and two that do not (a group of several entries
+# per row across every cut, seven parts)
+FIBRE_SUMS = [
+    ((601, 220), [{0: "num"}, {1: "diag"}, {0: "hop", 1: "hop"}]),
+    ((64, 2049), [{0: "two"}, {1: "two"}, {0: "hop", 1: "num"}, {0: "diag", 1: "num"}]),
+    ((2, 70, 1000), [{0: "two"}, {0: "hop", 1: "hop", 2: "hop"}, {2: "num"}]),
+    ((260, 2, 3, 101), [{1: "hop", 2: "hop"}, {0: "num", 3: "hop"}, {0: "hop", 1: "num", 2: "diag", 3: "num"}]),
+    ((3, 50000), [{0: "num"}, {1: "hop"}]),
+    ((700, 200), [{1: "num"}]),
+    ((67, 123), [{0: "two"}, {1: "hop"}, {0: "diag"}]),
+    ((64, 128), [{0: "two", 1: "num"}]),
+    ((60, 50, 50), [{1: "two", 2: "two"}, {0: "hop", 1: "hop", 2: "hop"}]),
+    ((400, 350), [{0: "two"}, {1: "two"}, {0: "hop", 1: "hop"}, {0: "hop", 1: "num"}, {0: "num", 1: "hop"}]),
+]
+
+
+@pytest.mark.parametrize("case", range(len(FIBRE_SUMS)))
+@pytest.mark.parametrize("dtype,eps", [(np.complex128, 2.3e-16), (np.complex64, 1.2e-7)])
+def test_lazysum_fibre_tables(case, dtype, eps):
+    """Sums through the fibre tables, on a Ket, a Bra and the columns of an
+    operator, with beta: each element adds at most ten products of three or
+    four rounded values, so the rounding stays below 64 eps of sum |v||x|."""
+    dims, terms = FIBRE_SUMS[case]
+    g = np.random.default_rng(900 + case)
+    bases = [Q.GenericBasis(d) for d in dims]
+    B = Q.tensor(*bases)
+    n = int(np.prod(dims))
+    coef = list(g.standard_normal(len(terms)) + 1j * g.standard_normal(len(terms)))
+    M = sp.csc_matrix((n, n), dtype=np.complex128)
+    lts = []
+    for c, t in zip(coef, terms):
+        fac = {s: _sparse_factor(g, dims[s], k) for s, k in t.items()}
+        lts.append(Q.LazyTensor(B, B, tuple(s + 1 for s in sorted(t)),
+                                tuple(Q.SparseOperator(bases[s], bases[s], fac[s]) for s in sorted(t))))
+        K = sp.identity(1, format="csc")
+        for s, d in enumerate(dims):
+            K = sp.kron(fac.get(s, sp.identity(d)), K, format="csc")
+        M = M + c * K
+    H = Q.LazySum(B, B, coef, tuple(lts))
+    A = abs(M)
+    x = (g.standard_normal((n, 3)) + 1j * g.standard_normal((n, 3))).astype(dtype)
+    y = (g.standard_normal((n, 3)) + 1j * g.standard_normal((n, 3))).astype(dtype)
+    a, b = 0.7 - 0.2j, -0.4 + 0.3j
+
+    def check(got, want, bound):
+        assert np.all(abs(got - want) <= 64 * eps * (bound + 1e-30))
+
+    for State, op, ab in ((Q.Ket, M, A), (Q.Bra, M.T, A.T)):
+        r = State(B, y[:, 0].copy(), dtype)
+        s = State(B, x[:, 0].copy(), dtype)
+        (Q.mul_(r, H, s, a, b) if State is Q.Ket else Q.mul_(r, s, H, a, b))
+        check(r.data.to_numpy(), a * (op @ x[:, 0]) + b * y[:, 0], abs(a) * (ab @ abs(x[:, 0])) + abs(b * y[:, 0]))
+    small = Q.GenericBasis(3)
+    r = Q.Operator(B, small, Q.DeviceArray.from_numpy(np.full(3 * n, np.nan, dtype)))
+    Q.mul_(r, H, Q.Operator(B, small, Q.DeviceArray.from_numpy(x.ravel(order="F"))))
+    check(r.data.to_numpy().reshape((n, 3), order="F"), M @ x, A @ abs(x))

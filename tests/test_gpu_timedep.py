@@ -246,3 +246,38 @@ def test_density_matrix_steps_with_device_coefficients(side, dtype, tol):
     finally:
         _lib.call("qob_tune_set", b"ls_materialize", 1)
         _lib.call("qob_tune_set", b"qubit_enable", 1)
+
+
+@pytest.mark.parametrize("dims", [(64, 72), (70, 120), (300, 40, 3)])
+@pytest.mark.parametrize("dtype,tol", [(np.complex128, 1e-13), (np.complex64, 1e-5)])
+def test_products_over_large_spaces_follow_time(dims, dtype, tol):
+    """Terms kept as products of per-site tables (more than 4096 local rows),
+    walked and as fibre tables: a coefficient enters one factor of its term,
+    and the other factors stay as they are when it changes."""
+    g = np.random.default_rng(17)
+    bases = [Q.GenericBasis(d) for d in dims]
+    B = Q.tensor(*bases)
+    D = len(B)
+
+    def hop(d, k):
+        return sp.csc_matrix(sp.diags(g.standard_normal(d - 1) + 1j * g.standard_normal(d - 1), k))
+
+    facs = [{s: hop(d, (-1) ** s) for s, d in enumerate(dims)}, {s: hop(d, -((-1) ** s)) for s, d in enumerate(dims)},
+            {0: sp.csc_matrix(sp.diags(g.standard_normal(dims[0]).astype(complex)))},
+            {1: hop(dims[1], 1)}]
+    ops, mats = [], []
+    for f in facs:
+        ops.append(Q.LazyTensor(B, B, tuple(s + 1 for s in f), tuple(Q.SparseOperator(bases[s], bases[s], x)
+                                                                     for s, x in f.items())))
+        K = sp.identity(1, format="csc")
+        for s, d in enumerate(dims):
+            K = sp.kron(f.get(s, sp.identity(d)), K, format="csc")
+        mats.append(K)
+    H = Q.TimeDependentSum(COEFS, tuple(ops), init_time=0.3)
+    psi = (g.standard_normal(D) + 1j * g.standard_normal(D)).astype(dtype)
+    for t in [0.3, 1.3, -2.0]:
+        H.set_time_(t)
+        out = Q.Ket(B, np.zeros(D), dtype)
+        Q.mul_(out, H, Q.Ket(B, psi, dtype))
+        M = sum((complex(c(t)) if callable(c) else c) * K for c, K in zip(COEFS, mats))
+        assert O.rel_frobenius(out.to_numpy(), M @ psi.astype(complex)) < tol, t
