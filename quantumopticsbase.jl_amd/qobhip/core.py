@@ -78,7 +78,13 @@ def context() -> Context:
     return _CTX
 
 
+_DT_CODE = {np.dtype(np.complex128): QOB_C64, np.dtype(np.complex64): QOB_C32}
+
+
 def _dt(np_dtype) -> int:
+    code = _DT_CODE.get(np_dtype)
+    if code is not None:
+        return code
     np_dtype = np.dtype(np_dtype)
     if np_dtype == np.complex128:
         return QOB_C64
@@ -614,9 +620,6 @@ def dagger(x):
 
 
 # ---------------------------------------------------------------------- mul!
-_DT_CODE = {np.dtype(np.complex128): QOB_C64, np.dtype(np.complex64): QOB_C32}
-
-
 def _check_same_dtype(*xs):
     d0 = xs[0].dtype
     for x in xs[1:]:
@@ -635,36 +638,29 @@ def mul_(result, a, b, alpha=1.0, beta=0.0):
       (Operator, op, Operator)  left application on a density matrix
       (Operator, Operator, op)  right application
     """
+    if isinstance(result, Ket) and isinstance(b, Ket) and isinstance(a, AbstractOperator):
+        if _CAPTURE_KEEP:
+            _note_capture(result, a, b)
+        if a.basis_r is not b.basis or a.basis_l is not result.basis:
+            _bases(a.basis_r, b.basis, a.basis_l, result.basis)
+        _mul_vec(result.data, a, b.data, alpha, beta)
+        return result
     if type(a).__name__ == "SuperOperator":  # S * rho on vec(rho) (src/superoperators.jl:82-85)
         from .superop import apply
         if not isinstance(result, Operator) or not isinstance(b, Operator):
             raise MethodError("a SuperOperator acts on an Operator")
         apply(a, b, result, alpha, beta)
         return result
+    if isinstance(result, Ket):
+        raise MethodError(f"no method mul!(::Ket, ::{type(a).__name__}, ::{type(b).__name__})")
     ctx = context()
     al, be = c64(alpha), c64(beta)
     _note_capture(result, a, b)
-    if isinstance(result, Ket):
-        if not (isinstance(b, Ket) and isinstance(a, AbstractOperator)):
-            raise MethodError(f"no method mul!(::Ket, ::{type(a).__name__}, ::{type(b).__name__})")
-        _bases(a.basis_r, b.basis, a.basis_l, result.basis)
-        if result.data.ptr.value == b.data.ptr.value:
-            raise ArgumentError("output must not be aliased with input")
-        if isinstance(a, Operator):
-            _gemm_dense(0, len(a.basis_l), 1, len(a.basis_r), alpha, a, b.data, beta, result.data)
-            return result
-        dtb, dtr = _dt(b.dtype), _dt(result.dtype)
-        if dtb == dtr:
-            call("qob_mul_ket", ctx.h, dtr, a._handle(), b.data.ptr, b.data.n, result.data.ptr, result.data.n, al,
-                 be, None)
-        else:
-            call("qob_mul_ket_x", ctx.h, dtb, a._handle(), b.data.ptr, b.data.n, dtr, result.data.ptr,
-                 result.data.n, al, be, None)
-        return result
     if isinstance(result, Bra):
         if not (isinstance(a, Bra) and isinstance(b, AbstractOperator)):
             raise MethodError(f"no method mul!(::Bra, ::{type(a).__name__}, ::{type(b).__name__})")
-        _bases(a.basis, b.basis_l, result.basis, b.basis_r)
+        if a.basis is not b.basis_l or result.basis is not b.basis_r:
+            _bases(a.basis, b.basis_l, result.basis, b.basis_r)
         if isinstance(b, Operator):
             _gemm_dense(1, len(b.basis_r), 1, len(b.basis_l), alpha, b, a.data, beta, result.data)
             return result
@@ -680,12 +676,15 @@ def mul_(result, a, b, alpha=1.0, beta=0.0):
         if isinstance(b, Operator) and isinstance(a, AbstractOperator) and not (
                 isinstance(a, Operator) and a is result):
             if isinstance(a, Operator):
-                _bases(a.basis_r, b.basis_l, a.basis_l, result.basis_l)
+                if a.basis_r is not b.basis_l or a.basis_l is not result.basis_l:
+                    _bases(a.basis_r, b.basis_l, a.basis_l, result.basis_l)
                 _gemm_dense(0, len(a.basis_l), len(b.basis_r), len(a.basis_r), alpha, a, b.data, beta,
                             result.data)
                 return result
-            _bases(a.basis_r, b.basis_l, a.basis_l, result.basis_l)
-            _bases(b.basis_r, result.basis_r)
+            if a.basis_r is not b.basis_l or a.basis_l is not result.basis_l:
+                _bases(a.basis_r, b.basis_l, a.basis_l, result.basis_l)
+            if b.basis_r is not result.basis_r:
+                _bases(b.basis_r, result.basis_r)
             dtb, dtr = _dt(b.dtype), _dt(result.dtype)
             if dtb == dtr:
                 call("qob_mul_op_left", ctx.h, dtr, a._handle(), b.data.ptr, len(b.basis_l), len(b.basis_r),
@@ -695,8 +694,10 @@ def mul_(result, a, b, alpha=1.0, beta=0.0):
                      dtr, result.data.ptr, len(result.basis_l), al, be, None)
             return result
         if isinstance(a, Operator) and isinstance(b, AbstractOperator):
-            _bases(a.basis_r, b.basis_l, a.basis_l, result.basis_l)
-            _bases(b.basis_r, result.basis_r)
+            if a.basis_r is not b.basis_l or a.basis_l is not result.basis_l:
+                _bases(a.basis_r, b.basis_l, a.basis_l, result.basis_l)
+            if b.basis_r is not result.basis_r:
+                _bases(b.basis_r, result.basis_r)
             dta, dtr = _dt(a.dtype), _dt(result.dtype)
             if dta == dtr:
                 call("qob_mul_op_right", ctx.h, dtr, a.data.ptr, len(a.basis_l), len(a.basis_r), b._handle(),
@@ -706,6 +707,21 @@ def mul_(result, a, b, alpha=1.0, beta=0.0):
                      dtr, result.data.ptr, len(result.basis_r), al, be, None)
             return result
     raise MethodError(f"no method mul!(::{type(result).__name__}, ::{type(a).__name__}, ::{type(b).__name__})")
+
+
+def _mul_vec(out: DeviceArray, a: AbstractOperator, x: DeviceArray, alpha, beta) -> None:
+    """out = alpha a x + beta out for the data of two vectors."""
+    if out.ptr.value == x.ptr.value:
+        raise ArgumentError("output must not be aliased with input")
+    if isinstance(a, Operator):
+        _gemm_dense(0, len(a.basis_l), 1, len(a.basis_r), alpha, a, x, beta, out)
+        return
+    dtx, dtr = _dt(x.dtype), _dt(out.dtype)
+    if dtx == dtr:
+        call("qob_mul_ket", context().h, dtr, a._handle(), x.ptr, x.n, out.ptr, out.n, c64(alpha), c64(beta), None)
+    else:
+        call("qob_mul_ket_x", context().h, dtx, a._handle(), x.ptr, x.n, dtr, out.ptr, out.n, c64(alpha), c64(beta),
+             None)
 
 
 def _bases(*pairs):
@@ -859,10 +875,10 @@ def variance(op: AbstractOperator, state) -> complex:
 
 def axpy_(y: _State, a, x: _State) -> _State:
     """y .+= a .* x on device data."""
-    _check_same_dtype(x, y)
+    code = _check_same_dtype(x, y)
     if x.data.n != y.data.n:
         raise DimensionMismatch("axpy of arrays of different length")
-    call("qob_axpy", context().h, _dt(y.dtype), y.data.n, c64(a), x.data.ptr, y.data.ptr, None)
+    call("qob_axpy", context().h, code, y.data.n, c64(a), x.data.ptr, y.data.ptr, None)
     return y
 
 

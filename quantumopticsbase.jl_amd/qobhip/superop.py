@@ -18,8 +18,8 @@ import numpy as np
 import scipy.sparse as sp
 
 from ._lib import ArgumentError, DimensionMismatch, IncompatibleBases, MethodError
-from .core import (DenseOperator, DeviceArray, GenericBasis, Operator, SparseOperator, _Adjoint,
-                   dagger as _dagger, mul_ as _mul_)
+from .core import (DenseOperator, DeviceArray, GenericBasis, Operator, SparseOperator, _Adjoint, _mul_vec,
+                   _note_capture, dagger as _dagger)
 
 
 def _data_of(op):
@@ -110,14 +110,15 @@ def apply(S: SuperOperator, rho: Operator, out: Operator | None = None, alpha=1.
     """S * rho (src/superoperators.jl:82-85) on the device: out = alpha S vec(rho) + beta out."""
     if rho.basis_l != S.basis_r[0] or rho.basis_r != S.basis_r[1]:
         raise IncompatibleBases("SuperOperator and Operator bases differ")
-    from .core import Ket
     op = S._device_op()
     if out is None:
         out = Operator(S.basis_l[0], S.basis_l[1], DeviceArray(S.data.shape[0], rho.dtype,
                                                                (len(S.basis_l[0]), len(S.basis_l[1]))))
-    vin = Ket(op.basis_r, rho.data)
-    vout = Ket(op.basis_l, out.data)
-    _mul_(vout, op, vin, alpha, beta)
+    for d, b in ((rho.data, op.basis_r), (out.data, op.basis_l)):
+        if d.n != len(b):
+            raise DimensionMismatch(f"Tried to assign data of length {d.n} to Hilbert space of size {len(b)}")
+    _note_capture(out, op, rho)
+    _mul_vec(out.data, op, rho.data, alpha, beta)
     return out
 
 
