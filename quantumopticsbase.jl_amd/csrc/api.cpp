@@ -2163,6 +2163,13 @@ static qob_status apply_lt_any(const Apply &ap, const std::vector<ChainOp> &ops,
             if (!lds) break;
             const bool whole = i == 0 && k + 1 == ops.size();
             const int64_t nt = n1 == 1 ? (S.n3 + F.units - 1) / F.units : F.nrb * S.n3;
+            // two wide factors from the right in less than a round of tiles:
+            // the chain (ComplexF32 (24, 32) 15.7 / 18.5 us, (20, 40) 18.9 / 23.0,
+            // but (16, 27) 10.6 / 10.0; ComplexF64 (27, 27) 19.8 / 20.7, but
+            // (20, 36) 24.9 / 19.5)
+            if (n1 > 1 && S.nmodes == 2 && ops.size() == 2 && nt < device_cu_count() &&
+                (ap.dt == QOB_C32 ? dsum > 44 : S.m[0].d > 20 && S.m[1].d > 20))
+                return QOB_OK;
             if (k == i || (nt >= 64 ? lds <= 80 * 1024 || whole : P <= 2560 && dsum <= 64)) {
                 best = S;
                 j = k + 1;
