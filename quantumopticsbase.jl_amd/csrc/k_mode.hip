@@ -29,7 +29,8 @@
 //                 factors wider than 64 and for DenseOperator on a density
 //                 matrix (and qob_gemm).
 //   k_zgemv       a single vector (DenseOperator on a Ket or Bra): columns
-//                 of F split over workgroups, deterministic two-stage sum.
+//                 of F split over workgroups, deterministic two-stage sum;
+//                 up to 1536 rows in one launch (k_zgemv_one).
 #include "qob_mfma.h"
 
 #include <map>
@@ -484,6 +485,14 @@ __global__ void __launch_bounds__(GNT, WPE) k_zgemm(int64_t M, int64_t N, int64_
 }
 
 // --------------------------------------------------------------- k_zgemv
+// A matrix far larger than the caches is read once at the copy rate; below
+// about 3000 columns the time is load latency, so the kernels here keep
+// several loads of each lane in flight, issued at a valid address where there
+// is nothing left to add.  A Ket and a Bra by an n x n matrix, before -> now:
+// ComplexF32 803 14.7 -> 11.3 us, 2013 26.1 -> 17.4, 6143 125 -> 114;
+// ComplexF64 2013 31.2 -> 26.1, 3009 63.9 -> 53.0.
+constexpr int GV_U = 8;
+
 // part[s][i] = sum over the columns j of split s of F[i, j] x[j]; with one
 // split the result goes straight to y (y = alpha part + beta y).  A
 // workgroup covers 64 rows (one row per lane, so every column of F is read as
@@ -497,22 +506,27 @@ __global__ void __launch_bounds__(GV_NT) k_zgemv(const cplx<R> *__restrict__ F, 
                                                  double2 alpha_, double2 beta_, int beta_zero) {
     using T = cplx<R>;
     __shared__ T red[GV_NT];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t i = (int64_t)blockIdx.x * 64 + lane;
     const int64_t j0 = (int64_t)blockIdx.y * split_len;
     const int64_t j1 = j0 + split_len < n ? j0 + split_len : n;
     T acc = czero<T>();
-    if (i < m) {
-        const T *Fi = F + i;
-        int64_t j = j0 + wave;
-        for (; j + 12 < j1; j += 16) {
-            const T f0 = Fi[j * m], f1 = Fi[(j + 4) * m], f2 = Fi[(j + 8) * m], f3 = Fi[(j + 12) * m];
-            acc = cfma(f0, x[j], acc);
-            acc = cfma(f1, x[j + 4], acc);
-            acc = cfma(f2, x[j + 8], acc);
-            acc = cfma(f3, x[j + 12], acc);
-        }
-        for (; j < j1; j += 4) acc = cfma(Fi[j * m], x[j], acc);
+    const T *Fi = F + (i < m ? i : m - 1);
+    int64_t j = j0 + wave;
+    for (; j + 4 * (GV_U - 1) < j1; j += 4 * GV_U) {
+        T f[GV_U];
+#pragma unroll
+        for (int u = 0; u < GV_U; ++u) f[u] = Fi[(j + 4 * u) * m];
+#pragma unroll
+        for (int u = 0; u < GV_U; ++u) acc = cfma(f[u], x[j + 4 * u], acc);
+    }
+    if (j < j1) {
+        T f[GV_U];
+#pragma unroll
+        for (int u = 0; u < GV_U; ++u) f[u] = Fi[(j + 4 * u < j1 ? j + 4 * u : j) * m];
+#pragma unroll
+        for (int u = 0; u < GV_U; ++u)
+            if (j + 4 * u < j1) acc = cfma(f[u], x[j + 4 * u], acc);
     }
     red[threadIdx.x] = acc;
     __syncthreads();
@@ -530,24 +544,81 @@ __global__ void __launch_bounds__(GV_NT) k_zgemv(const cplx<R> *__restrict__ F, 
     }
 }
 
-// y[i] = alpha * sum_s part[s][i] + beta * y[i], splits summed in order
+// y[i] = alpha * sum_s part[s][i] + beta * y[i]: 32 rows per workgroup, eight
+// runs of splits per row, each in order, their sums added in order.
 template <typename R>
 __global__ void __launch_bounds__(256) k_zgemv_sum(const cplx<double> *__restrict__ part, int nsplit, int64_t m,
                                                    cplx<R> *__restrict__ y, double2 alpha_, double2 beta_,
                                                    int beta_zero) {
     using T = cplx<R>;
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    double2 s = part[i];
-    for (int k = 1; k < nsplit; ++k) s = cadd(s, part[(int64_t)k * m + i]);
-    const T alpha = mk((R)alpha_.x, (R)alpha_.y), beta = mk((R)beta_.x, (R)beta_.y);
-    y[i] = axpby(alpha, mk((R)s.x, (R)s.y), beta, y + i, beta_zero != 0);
+    __shared__ double2 red[256];
+    const int r = threadIdx.x & 31, q = threadIdx.x >> 5;
+    const int64_t i = (int64_t)blockIdx.x * 32 + r;
+    const double2 *p = part + (i < m ? i : m - 1);
+    const int k0 = (int)((int64_t)nsplit * q / 8), k1 = (int)((int64_t)nsplit * (q + 1) / 8);
+    double2 s = make_double2(0, 0);
+    for (int k = k0; k < k1; k += 4) {
+        double2 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = p[(int64_t)min(k + u, k1 - 1) * m];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + u < k1) s = cadd(s, v[u]);
+    }
+    red[threadIdx.x] = s;
+    __syncthreads();
+    if (q == 0 && i < m) {
+        for (int k = 1; k < 8; ++k) s = cadd(s, red[32 * k + r]);
+        const T alpha = mk((R)alpha_.x, (R)alpha_.y), beta = mk((R)beta_.x, (R)beta_.y);
+        y[i] = axpby(alpha, mk((R)s.x, (R)s.y), beta, y + i, beta_zero != 0);
+    }
+}
+
+// The same in one launch: a workgroup covers 16 rows, lane l of wave w row
+// l % 16 and the columns 4 w + l / 16 + 64 t (runs of 16 rows).  The 64
+// partial sums of a row are added in FP64, in column order within a wave.
+template <typename R>
+__global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ F, int64_t m, int64_t n,
+                                                    const cplx<R> *__restrict__ x, cplx<R> *__restrict__ y,
+                                                    double2 alpha_, double2 beta_, int beta_zero) {
+    using T = cplx<R>;
+    __shared__ double2 red[16][16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15;
+    const int64_t i = (int64_t)blockIdx.x * 16 + r;
+    const T *Fi = F + (i < m ? i : m - 1);
+    T acc = czero<T>();
+    for (int64_t j = wave * 4 + (lane >> 4); j < n; j += 64 * GV_U) {
+        T f[GV_U], v[GV_U];
+#pragma unroll
+        for (int u = 0; u < GV_U; ++u) {
+            const int64_t jj = j + 64 * u < n ? j + 64 * u : j;
+            f[u] = Fi[jj * m];
+            v[u] = x[jj];
+        }
+#pragma unroll
+        for (int u = 0; u < GV_U; ++u)
+            if (j + 64 * u < n) acc = cfma(f[u], v[u], acc);
+    }
+    double2 s = make_double2(acc.x, acc.y);
+    for (int o = 16; o <= 32; o <<= 1) {
+        s.x += __shfl_xor(s.x, o, 64);
+        s.y += __shfl_xor(s.y, o, 64);
+    }
+    if (lane < 16) red[wave][r] = s;
+    __syncthreads();
+    if (threadIdx.x < 16 && i < m) {
+        for (int k = 1; k < 16; ++k) s = cadd(s, red[k][r]);
+        const T alpha = mk((R)alpha_.x, (R)alpha_.y), beta = mk((R)beta_.x, (R)beta_.y);
+        y[i] = axpby(alpha, mk((R)s.x, (R)s.y), beta, y + i, beta_zero != 0);
+    }
 }
 
 // y[i] = alpha * sum_l A[l + i k] x[l] + beta * y[i] (y = A^T x for a
 // column-major k x m A): one wave per output, lanes along the column (1 KiB
-// runs), then a butterfly sum over the wave in a fixed order.
-template <typename R>
+// runs), U loads of each in flight, then a butterfly sum over the wave in a
+// fixed order.
+template <typename R, int U>
 __global__ void __launch_bounds__(256) k_zgemv_t(const cplx<R> *__restrict__ A, int64_t k, int64_t m,
                                                  const cplx<R> *__restrict__ x, cplx<R> *__restrict__ y,
                                                  double2 alpha_, double2 beta_, int beta_zero) {
@@ -557,7 +628,29 @@ __global__ void __launch_bounds__(256) k_zgemv_t(const cplx<R> *__restrict__ A, 
     if (i >= m) return;
     const T *Ai = A + i * k;
     T acc = czero<T>();
-    for (int64_t l = lane; l < k; l += 64) acc = cfma(Ai[l], x[l], acc);
+    int64_t l = lane;
+    for (; l + 64 * (U - 1) < k; l += 64 * U) {
+        T a[U], v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            a[u] = Ai[l + 64 * u];
+            v[u] = x[l + 64 * u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = cfma(a[u], v[u], acc);
+    }
+    if (U > 1 && l < k) {
+        T a[U], v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t q = l + 64 * u < k ? l + 64 * u : l;
+            a[u] = Ai[q];
+            v[u] = x[q];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (l + 64 * u < k) acc = cfma(a[u], v[u], acc);
+    }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         acc.x += __shfl_xor(acc.x, o);
@@ -604,7 +697,14 @@ template <typename K> hipError_t raise_lds(K kfn, size_t bytes) {
 // and timing; the LDS chunks measured 2% faster on a (16, 32, 16) chain)
 int g_mode_kernel = 0;
 
+// Rows up to which one launch does it (k_zgemv_one): for the split kernel and
+// its sum the second launch costs more than their better use of the CUs gains
+// (n x n, ComplexF32: 803 6.2 against 4.6 + 2.8 us and a launch, 1414 8.5
+// against 5.8 + 2.8, but 2013 11.4 against 8.1 + 2.6).
+constexpr int64_t GV_ONE = 1536;
+
 int64_t zgemv_splits(int64_t m, int64_t n) {
+    if (m <= GV_ONE) return 1;
     const int64_t rt = (m + 63) / 64;
     int64_t s = 1;
     while (rt * s < 1024 && n / (s * 2) >= 64) s *= 2;
@@ -653,22 +753,32 @@ hipError_t launch_zgemv(qob_dtype dt, const void *F, int64_t m, int64_t n, const
                         double2 alpha, double2 beta, hipStream_t s) {
     if (m <= 0) return hipSuccess;
     const int bz = (beta.x == 0.0 && beta.y == 0.0);
+    if (m <= GV_ONE) {
+        const unsigned g = (unsigned)((m + 15) / 16);
+        if (dt == QOB_C64)
+            hipLaunchKernelGGL(k_zgemv_one<double>, dim3(g), dim3(1024), 0, s, (const double2 *)F, m, n,
+                               (const double2 *)x, (double2 *)y, alpha, beta, bz);
+        else
+            hipLaunchKernelGGL(k_zgemv_one<float>, dim3(g), dim3(1024), 0, s, (const float2 *)F, m, n,
+                               (const float2 *)x, (float2 *)y, alpha, beta, bz);
+        return hipGetLastError();
+    }
     const int64_t ns = zgemv_splits(m, n);
     const int64_t len = (n + ns - 1) / ns;
     if (ns > 1 && !part) return hipErrorInvalidValue;
-    dim3 g((unsigned)((m + 63) / 64), (unsigned)ns);
+    dim3 g((unsigned)((m + 63) / 64), (unsigned)ns), gs((unsigned)((m + 31) / 32));
     if (dt == QOB_C64) {
         hipLaunchKernelGGL(k_zgemv<double>, g, dim3(GV_NT), 0, s, (const double2 *)F, m, n, (const double2 *)x, len,
                            (double2 *)part, (double2 *)y, alpha, beta, bz);
         if (ns > 1)
-            hipLaunchKernelGGL(k_zgemv_sum<double>, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s,
-                               (const double2 *)part, (int)ns, m, (double2 *)y, alpha, beta, bz);
+            hipLaunchKernelGGL(k_zgemv_sum<double>, gs, dim3(256), 0, s, (const double2 *)part, (int)ns, m,
+                               (double2 *)y, alpha, beta, bz);
     } else {
         hipLaunchKernelGGL(k_zgemv<float>, g, dim3(GV_NT), 0, s, (const float2 *)F, m, n, (const float2 *)x, len,
                            (double2 *)part, (float2 *)y, alpha, beta, bz);
         if (ns > 1)
-            hipLaunchKernelGGL(k_zgemv_sum<float>, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s,
-                               (const double2 *)part, (int)ns, m, (float2 *)y, alpha, beta, bz);
+            hipLaunchKernelGGL(k_zgemv_sum<float>, gs, dim3(256), 0, s, (const double2 *)part, (int)ns, m,
+                               (float2 *)y, alpha, beta, bz);
     }
     return hipGetLastError();
 }
@@ -678,12 +788,22 @@ hipError_t launch_zgemv_t(qob_dtype dt, const void *A, int64_t k, int64_t m, con
     if (m <= 0) return hipSuccess;
     const int bz = (beta.x == 0.0 && beta.y == 0.0);
     const unsigned g = (unsigned)((m + 3) / 4);
-    if (dt == QOB_C64)
-        hipLaunchKernelGGL(k_zgemv_t<double>, dim3(g), dim3(256), 0, s, (const double2 *)A, k, m, (const double2 *)x,
-                           (double2 *)y, alpha, beta, bz);
-    else
-        hipLaunchKernelGGL(k_zgemv_t<float>, dim3(g), dim3(256), 0, s, (const float2 *)A, k, m, (const float2 *)x,
-                           (float2 *)y, alpha, beta, bz);
+    // Four loads in flight per lane, one for a matrix beyond the 256 MiB that
+    // the MALL holds, which then streams from HBM (n x n, one / four: ComplexF32
+    // 2013 13.0 / 7.2 us, 4500 36.0 / 29.9, 6143 55.4 / 56.1; ComplexF64 3009
+    // 26.5 / 22.8, 4500 48.5 / 55.4, 6143 91.6 / 102.4).
+    const bool one = (double)k * m * (dt == QOB_C64 ? 16 : 8) > (double)(256 << 20);
+#define QOB_GT(RR, U)                                                                                        \
+    hipLaunchKernelGGL((k_zgemv_t<RR, U>), dim3(g), dim3(256), 0, s, (const cplx<RR> *)A, k, m,              \
+                       (const cplx<RR> *)x, (cplx<RR> *)y, alpha, beta, bz)
+    if (dt == QOB_C64) {
+        if (one) QOB_GT(double, 1);
+        else QOB_GT(double, 4);
+    } else {
+        if (one) QOB_GT(float, 1);
+        else QOB_GT(float, 4);
+    }
+#undef QOB_GT
     return hipGetLastError();
 }
 

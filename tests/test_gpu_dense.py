@@ -409,3 +409,32 @@ def test_lazytensor_site_groups_nan_stays_in_its_fibres(dtype):
         want = np.zeros((105, 40), bool)
         want[[a + 5 * 3 + 35 * c for a in range(5) for c in range(3)], 7] = True
         assert np.array_equal(hit, want)
+
+
+# rows and columns around the tiles of 16, 32 and 64 rows and the runs of 4,
+# 64 and 256 columns, the last size of one launch and the first of two, many
+# splits, and a matrix beyond 256 MiB
+GEMV_SHAPES = [(1, 1), (1, 300), (300, 1), (15, 17), (16, 64), (17, 65), (64, 511), (65, 513), (33, 4097), (1536, 70),
+               (1537, 70), (1537, 129), (1600, 1500), (2013, 2013), (4200, 4100)]
+
+
+@pytest.mark.parametrize("shape", GEMV_SHAPES)
+@pytest.mark.parametrize("dtype", DTS)
+def test_dense_operator_on_vectors(shape, dtype):
+    """DenseOperator on a Ket and a Bra against numpy in ComplexF64: sums of up
+    to 4200 products, rounding within TOLS of the result's norm."""
+    m, n = shape
+    g = np.random.default_rng(m * 5000 + n)
+    A = (g.standard_normal((m, n)) + 1j * g.standard_normal((m, n))).astype(dtype)
+    x, y = cg(g, n, 1)[:, 0].astype(dtype), cg(g, m, 1)[:, 0].astype(dtype)
+    op = Q.DenseOperator(gb(m), gb(n), A, dtype)
+    A = A.astype(np.complex128)
+    k = Q.Ket(gb(m), np.full(m, np.nan + 0j), dtype)
+    assert rel(Q.mul_(k, op, Q.Ket(gb(n), x, dtype)).to_numpy(), A @ x) < TOLS[dtype]
+    w = 0.5j * (A @ x) - 0.25 * y
+    k = Q.Ket(gb(m), y, dtype)
+    assert rel(Q.mul_(k, op, Q.Ket(gb(n), x, dtype), 0.5j, -0.25).to_numpy(), w) < TOLS[dtype]
+    b = Q.Bra(gb(n), np.full(n, np.nan + 0j), dtype)
+    assert rel(Q.mul_(b, Q.Bra(gb(m), y, dtype), op).to_numpy(), y @ A) < TOLS[dtype]
+    b = Q.Bra(gb(n), x, dtype)
+    assert rel(Q.mul_(b, Q.Bra(gb(m), y, dtype), op, 0.5j, -0.25).to_numpy(), 0.5j * (y @ A) - 0.25 * x) < TOLS[dtype]
