@@ -1097,3 +1097,37 @@ def test_lazysum_fibre_tables(case, dtype, eps):
     r = Q.Operator(B, small, Q.DeviceArray.from_numpy(np.full(3 * n, np.nan, dtype)))
     Q.mul_(r, H, Q.Operator(B, small, Q.DeviceArray.from_numpy(x.ravel(order="F"))))
     check(r.data.to_numpy().reshape((n, 3), order="F"), M @ x, A @ abs(x))
+
+
+@pytest.mark.parametrize("m,n,w", [(1, 1, 1), (63, 70, 2), (64, 64, 4), (65, 64, 5), (257, 300, 8), (300, 257, 9), (193, 193, 12),
+                                   (500, 400, 13), (400, 400, 16), (400, 400, 17)])
+@pytest.mark.parametrize("dtype,tol", [(np.complex128, 1e-13), (np.complex64, 1e-6)])
+def test_sparse_operator_on_a_ket_of_any_row_width(m, n, w, dtype, tol):
+    """Rows of up to w entries (random columns, so one connected pattern), none
+    in every third slice of 64 rows, against scipy: sums of at most 17 products."""
+    g = np.random.default_rng(m * 17 + w)
+    cnt = g.integers(1, w + 1, m)
+    cnt[g.integers(0, m)] = w
+    cnt[(np.arange(m) // 64) % 3 == 1] = 0
+    cnt = np.minimum(cnt, n)
+    rows = np.repeat(np.arange(m), cnt)
+    cols = np.concatenate([g.choice(n, c, replace=False) for c in cnt]) if cnt.sum() else np.zeros(0, int)
+    M = sp.csc_matrix((g.standard_normal(len(rows)) + 1j * g.standard_normal(len(rows)), (rows, cols)), shape=(m, n))
+    Bl, Br = Q.GenericBasis(m), Q.GenericBasis(n)
+    op = Q.SparseOperator(Bl, Br, M)
+    x = (g.standard_normal(n) + 1j * g.standard_normal(n)).astype(dtype)
+    y = (g.standard_normal(m) + 1j * g.standard_normal(m)).astype(dtype)
+    x[g.integers(0, n)] = 1e3
+    A = abs(M)
+    k = Q.Ket(Bl, np.full(m, np.nan + 0j), dtype)
+    got = Q.mul_(k, op, Q.Ket(Br, x, dtype)).to_numpy()
+    assert np.all(abs(got - M @ x) <= tol * (A @ abs(x) + 1e-30) * 20)
+    k = Q.Ket(Bl, y, dtype)
+    got = Q.mul_(k, op, Q.Ket(Br, x, dtype), 0.5j, -0.25).to_numpy()
+    assert np.all(abs(got - (0.5j * (M @ x) - 0.25 * y)) <= tol * (A @ abs(x) + abs(y)) * 20)
+    bad = x.copy()
+    bad[0] = np.nan  # reaches the rows that have column 0 and no others
+    got = Q.mul_(Q.Ket(Bl, np.zeros(m), dtype), op, Q.Ket(Br, bad, dtype)).to_numpy()
+    hit = np.zeros(m, bool)
+    hit[rows[cols == 0]] = True
+    assert np.array_equal(np.isnan(got), hit)
