@@ -779,10 +779,12 @@ __global__ void __launch_bounds__(NTH) k_qubit_hi(const QubitStateDev *__restric
 // flips read partner tiles from v in global memory.  u and v's own tile are
 // in registers anyway, so sum conj(u) v, which a variance needs of the same
 // vectors, goes to partials[gridDim.x ...] for four more FMAs per element.
+// square (u = v): the sums are |H v|^2 and conj(v) H v instead, all of a
+// Hermitian H's variance in one pass over the state.
 template <typename T, int NTH, int TBITS>
 __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__restrict__ u, int ntiles,
                                                    const int32_t *__restrict__ prog, const T *__restrict__ vals,
-                                                   double2 *__restrict__ partials) {
+                                                   int square, double2 *__restrict__ partials) {
     constexpr int EPT = (1 << TBITS) / NTH;
     extern __shared__ unsigned char lds_raw[];
     T *tile = (T *)lds_raw;
@@ -813,11 +815,12 @@ __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__r
         for (int k = 0; k < EPT; ++k) {
             const int e = tid + k * NTH;
             if (e < tsize) {
-                const T a = u[base + e];
-                rx += (double)a.x * acc[k].x + (double)a.y * acc[k].y;
-                ry += (double)a.x * acc[k].y - (double)a.y * acc[k].x;
-                px += (double)a.x * xv[k].x + (double)a.y * xv[k].y;
-                py += (double)a.x * xv[k].y - (double)a.y * xv[k].x;
+                const T a = square ? xv[k] : u[base + e];
+                const T b = square ? acc[k] : a, c = square ? acc[k] : xv[k];
+                rx += (double)b.x * acc[k].x + (double)b.y * acc[k].y;
+                ry += (double)b.x * acc[k].y - (double)b.y * acc[k].x;
+                px += (double)a.x * c.x + (double)a.y * c.y;
+                py += (double)a.x * c.y - (double)a.y * c.x;
             }
         }
     }
@@ -1103,7 +1106,7 @@ int qubit_dot_blocks(int64_t ntiles) {
 }
 
 hipError_t launch_qubit_dot(qob_dtype dt, QubitStateDev single, const void *u, int tbits, const int32_t *prog,
-                            const void *vals, double2 *partials, hipStream_t s) {
+                            const void *vals, bool square, double2 *partials, hipStream_t s) {
     if (tbits < 10 || tbits > 13) return hipErrorInvalidValue;
     const int tb = std::min(tbits, (int)single.nbits);
     const int64_t ntiles = (int64_t)1 << (single.nbits - tb);
@@ -1122,7 +1125,7 @@ hipError_t launch_qubit_dot(qob_dtype dt, QubitStateDev single, const void *u, i
             lds_set.store(1);                                                                                   \
         }                                                                                                       \
         hipLaunchKernelGGL(kfn, dim3(g), dim3(NTD), lds, s, single, (const TT *)u, (int)ntiles, prog,           \
-                           (const TT *)vals, partials);                                                         \
+                           (const TT *)vals, square ? 1 : 0, partials);                                         \
         return hipGetLastError();                                                                               \
     } while (0)
     if (dt == QOB_C64) {

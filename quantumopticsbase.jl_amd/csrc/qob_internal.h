@@ -388,11 +388,13 @@ hipError_t launch_lt_any(qob_dtype dt, AnyPass S, const void *in, void *out, dou
 int gather_dot_blocks(int64_t n);
 hipError_t launch_gather_dot(qob_dtype dt, const GatherPlanDev &P, int mode, const void *u, const void *v, int64_t n,
                              double2 *partials, hipStream_t s);
-// sum_J conj(u[J]) (H v)[J] for one qubit state (single.in = v), FP64
-// partials, one per workgroup of the returned grid size
+// sums of conj(u[J]) (H v)[J] and conj(u[J]) v[J] for one qubit state
+// (single.in = v); square: of |(H v)[J]|^2 and conj(v[J]) (H v)[J].  FP64
+// partials, one of each per workgroup (qubit_dot_blocks), the second sum's
+// after the first's.
 int qubit_dot_blocks(int64_t ntiles);
 hipError_t launch_qubit_dot(qob_dtype dt, QubitStateDev single, const void *u, int tbits, const int32_t *prog,
-                            const void *vals, double2 *partials, hipStream_t s);
+                            const void *vals, bool square, double2 *partials, hipStream_t s);
 // sum over the nonzeros of a CSC matrix X (n columns) of val * V[c + row * n]:
 // tr(X V) for an n x n V (expect(::SparseOpPureType, ::Operator))
 int csc_trace_blocks(int64_t n);

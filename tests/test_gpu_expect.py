@@ -245,3 +245,57 @@ def test_scalars_on_many_streams_and_behind_a_long_queue():
     nrm = C.c_double()
     _lib.call("qob_norm", ctx.h, Q.QOB_C64, n, dev[0].ptr, C.byref(nrm), None)
     assert abs(nrm.value - np.linalg.norm(xs[0])) <= 1e-12 * nrm.value
+
+
+@pytest.mark.parametrize("L", [1, 5, 9, 10, 11, 12])
+@pytest.mark.parametrize("kind", ["hermitian", "pairs", "one_way", "phase"])
+@pytest.mark.parametrize("dtype,tol", [(np.complex128, 1e-12), (np.complex64, 1e-5)])
+def test_variance_of_hermitian_and_other_sums(L, kind, dtype, tol):
+    """Real combinations of Pauli strings and of sigma_+ sigma_- with its
+    adjoint (one pass over the state), and sums that only look like them: a
+    sigma_+ without its adjoint, a complex coefficient, and coefficients that
+    become complex on the device.  Against sparse algebra in ComplexF64."""
+    from test_gpu_qubit import PAULI
+
+    g = np.random.default_rng(1000 + L)
+    terms = []
+    for i in range(L):
+        terms.append((float(g.standard_normal()), (i + 1,), [PAULI[g.choice(list("xyzn"))]]))
+        if i + 1 < L:
+            terms.append((float(g.standard_normal()), (i + 1, i + 2), [PAULI[g.choice(list("xyz"))] for _ in range(2)]))
+            if kind != "hermitian":
+                c = float(g.standard_normal())
+                terms.append((c, (i + 1, i + 2), [PAULI["p"], PAULI["m"]]))
+                terms.append((c, (i + 1, i + 2), [PAULI["m"], PAULI["p"]]))
+    if kind == "one_way":
+        terms.append((0.7, (1,), [PAULI["p"]]))
+    if kind == "phase":
+        terms.append((0.3 + 0.4j, (L,), [PAULI["x"]]))
+    H, Ho, B = build_pair(L, terms)
+    psi = g.standard_normal(2 ** L) + 1j * g.standard_normal(2 ** L)
+    psi = (psi / np.linalg.norm(psi)).astype(dtype)
+    k = Q.Ket(B, psi, dtype)
+    psi = psi.astype(complex)
+    M = sp.csr_matrix(O.dense_of(Ho)) if L <= 10 else None
+    if M is None:
+        M = sp.csr_matrix((2 ** L, 2 ** L), dtype=complex)
+        for c, sites, mats in terms:
+            K = sp.identity(1, format="csr")
+            for s in range(1, L + 1):
+                K = sp.kron(mats[sites.index(s)] if s in sites else sp.identity(2), K, format="csr")
+            M = M + c * K
+    want = _var(M, psi)
+    scale = max(1.0, np.linalg.norm(M @ psi) ** 2)
+    assert abs(Q.variance(H, k) - want) <= tol * scale
+    # the same operator with one coefficient made complex on the device
+    fac = np.array([c for c, _, _ in terms], dtype=complex)
+    fac[0] *= 1j
+    c, sites, mats = terms[0]
+    K = sp.identity(1, format="csr")
+    for s in range(1, L + 1):
+        K = sp.kron(mats[sites.index(s)] if s in sites else sp.identity(2), K, format="csr")
+    M2 = M + (fac[0] - c) * K
+    d = Q.DeviceArray.from_numpy(fac)
+    H.set_factors_device(d)
+    got = Q.variance(H, k)
+    assert abs(got - _var(M2, psi)) <= tol * max(1.0, np.linalg.norm(M2 @ psi) * np.linalg.norm(M2.conj().T @ psi))
