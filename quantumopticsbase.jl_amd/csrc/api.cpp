@@ -1407,8 +1407,10 @@ static qob_status compile_plan(const std::vector<int64_t> &out_shape, const std:
     std::sort(cuts.begin(), cuts.end(), [&](int64_t a, int64_t b) { return a + Dout / a < b + Dout / b; });
     for (int64_t fib : cuts) {
         const int64_t nf = Dout / fib;
-        // tables of at most 2^18 values, counted once per term of the sum
-        // (each term's share of them is built for the coefficient refresh)
+        // tables of at most 2^16 values, counted once per term of the sum
+        // (each term's share of them is built for the coefficient refresh):
+        // building them stays below what the plan took without them (a sum on
+        // (20, 401, 2), whose one cut leaves 8020 below, 0.5 ms and 1.3 with)
         int parts = 0;
         bool fits = true;
         auto side = [&](const std::vector<int> &sites) {  // 1 below, 2 above, 3 both
@@ -1430,7 +1432,7 @@ static qob_status compile_plan(const std::vector<int64_t> &out_shape, const std:
         }
         parts += (int)std::min<size_t>(prods.size(), GP_PARTS + 1);
         if (!fits || parts > GP_PARTS) continue;
-        if ((fib + nf) * (parts + 1) * (int64_t)(terms.size() + 1) > (1 << 18)) continue;
+        if ((fib + nf) * (parts + 1) * (int64_t)(terms.size() + 1) > (1 << 16)) continue;
         GatherPlanDev &D = H.fibre;
         const int64_t len = fib + nf;
         D.fv = (int32_t)H.vals.size();
