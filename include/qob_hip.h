@@ -338,7 +338,8 @@ qob_status qob_expect_op(qob_ctx ctx, qob_dtype dt, qob_op a, const void *rho,
 /* variance(op, ket) = <psi|op op|psi> - <psi|op|psi>^2 with x = op psi
  * computed once (src/operators.jl:139-143); FP64 result for both element
  * types.  In the fused mode <psi|op x> is a single pass when op is a qubit
- * sum or an all-sparse lazy operator. */
+ * sum or an all-sparse lazy operator, and <x|x> without a stored x when op is
+ * a Hermitian qubit sum. */
 qob_status qob_variance_ket(qob_ctx ctx, qob_dtype dt, qob_op a, const void *psi,
                             int64_t n, qob_c64 *out, qob_stream s);
 /* variance(op, rho) = tr(op op rho) - tr(op rho)^2 with op * rho formed once

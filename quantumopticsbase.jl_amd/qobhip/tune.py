@@ -10,7 +10,9 @@ of libqob_hip.so (qob_tune_set / qob_tune_get):
                     kernel for leading dimensions below 16 as well,
                     a test and timing switch, not tuned)
   qubit sums        qubit_tbits (tile = 2^tbits states; 0 = 2^12 for
-                    ComplexF64, 2^11 for ComplexF32), qubit_nth (0 = 4
+                    ComplexF64 and 2^11 for ComplexF32 in a batch, 2^10 for
+                    single states, 2^11 above 20 sites in ComplexF32),
+                    qubit_nth (0 = 4
                     elements per lane in ComplexF64, 8 in ComplexF32),
                     qubit_grid (persistent workgroups; 0 = 1024 / nth per CU),
                     qubit_remap (0 plain, 1 XCD-contiguous rounds, 2 per-XCD
@@ -20,6 +22,8 @@ of libqob_hip.so (qob_tune_set / qob_tune_get):
                     code, 2 Gray code above 64 tiles), qubit_dbuf (two LDS tile
                     buffers in persistent walks), qubit_pair (ComplexF32
                     lanes on pairs of adjacent elements), qubit_split
+                    (0 = a second, strided pass for the high flips of long
+                    single states, 1 = for every flip above the tile)
   sparse products   sell_variant, sell_cj, sell_jchunk, sell_unr, csc_rows,
                     csc_rb, csc_cc, csc_remap, csc_order (column sweep order),
                     csc_sweep (row stripes / column-major / by reuse
