@@ -1006,14 +1006,16 @@ struct Workspace {
     DevBuf slot[WS_NSLOT];
 };
 
-// One scalar result on its way to the host, in pinned memory: the last kernel
-// of the reduction stores the values and then a sequence number, for which
-// the host waits.  A slot belongs to one call from its start to its end.
+// One scalar result on its way to the host, in pinned memory: workgroups (or
+// the last kernel's only one) store values and then a sequence number each,
+// for which the host waits.  A slot belongs to one call from its start to its
+// end.
+constexpr int HOST_PARTS = 8;
 struct alignas(64) HostSlot {
-    double2 v[2];
-    uint32_t flag;
+    double2 v[2 * HOST_PARTS];
+    uint32_t flag[HOST_PARTS];
 };
-constexpr int HOST_SLOTS = 64;
+constexpr int HOST_SLOTS = 63;
 
 // Device memory that queued work, or a live captured graph, may still read
 // when the library replaces it: kept until it is safe to free.
@@ -2777,7 +2779,7 @@ qob_status qob_ctx_create(int device, qob_ctx *out) {
     if (hipHostMalloc(&hs, sizeof(HostSlot) * HOST_SLOTS, hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess) {
         memset(hs, 0, sizeof(HostSlot) * HOST_SLOTS);
         c->hslot = (HostSlot *)hs;
-        c->hfree.store(~0ull);
+        c->hfree.store((1ull << HOST_SLOTS) - 1);
     } else {
         (void)hipGetLastError();
     }
@@ -3539,53 +3541,109 @@ static qob_status scal_ws(qob_ctx ctx, hipStream_t st, void *&p) { return ws_get
 
 }  // extern "C"
 
-// Sum one or two sets of partials queued on st and wait for the result h[2].
+// A scalar result on its way to the host.
 //
 // The copy of a scalar to pageable memory and hipStreamSynchronize cost about
-// 20 us, more than the kernels of a state below 18 sites.  The last kernel
-// stores to pinned memory instead and the host watches the slot's number:
-// expect of 8 sites 13.7 us instead of 26.4, of 18 sites 16.6 instead of
-// 29.4, a norm 12.8 instead of 25.5.  Everything queued on st before has
-// finished by then.  A result that takes longer than 200 us (where the wait
-// is a small part), and any error of the queue, is left to the synchronise.
-static qob_status sums_to_host(qob_ctx ctx, hipStream_t st, RedMode mode, RedSet a, RedSet b, double2 *h) {
+// 20 us, more than the kernels of a state below 18 sites.  The kernels store
+// to pinned memory instead and the host watches the slot's numbers.  Up to
+// HOST_PARTS workgroups' sums come as they are (out, sum); more are added by
+// another launch, about 3 us (final).  Stores of several workgroups to host
+// memory follow one another at about 80 ns: 16 sums cost what the launch does,
+// 64 sums 5 us more.  Expect of 8 / 18 sites takes 11.8 / 16.7 us instead of
+// 26.4 / 29.4, a norm of 8 sites 8.3 instead of 25.5.
+// Everything queued on the stream before has finished by then, and this
+// kernel has read all that it reads.  A result that takes longer than 200 us
+// (where the wait is a small part), and any error of the queue, is left to the
+// synchronise.
+//
+// While a stream is captured, and with 63 calls under way, there is no slot:
+// out is empty, and final adds, copies and synchronises (which a capture
+// refuses).
+struct HostSum {
+    qob_ctx ctx;
+    hipStream_t st;
     int i = -1;
-    if (ctx->hslot && !capturing(st)) {
+    bool queued = false;  // a kernel may store to the slot
+
+    HostSum(qob_ctx c, hipStream_t s) : ctx(c), st(s) {
+        if (!ctx->hslot || capturing(st)) return;
         uint64_t m = ctx->hfree.load(std::memory_order_relaxed);
         while (m && !ctx->hfree.compare_exchange_weak(m, m & (m - 1), std::memory_order_acquire)) {
         }
         if (m) i = __builtin_ctzll(m);
     }
-    if (i < 0) {  // capturing (refused by the synchronise), or 64 calls under way
-        void *d;
-        QOB_TRY(scal_ws(ctx, st, d));
-        QOB_HIP(launch_final(mode, a, b, d, nullptr, 0, st));
-        QOB_HIP(hipMemcpyAsync(h, d, (b.n ? 2 : 1) * sizeof(double2), hipMemcpyDeviceToHost, st));
-        QOB_HIP(hipStreamSynchronize(st));
+    HostSum(const HostSum &) = delete;
+    HostSum &operator=(const HostSum &) = delete;
+    ~HostSum() {
+        // after an error the slot stays taken if a kernel may still store there
+        if (i >= 0 && !queued) ctx->hfree.fetch_or(1ull << i, std::memory_order_release);
+    }
+    HostOut out(int parts) {
+        HostOut o;
+        if (i < 0 || parts > HOST_PARTS) return o;
+        queued = true;
+        o.v = ctx->hslot[i].v;
+        o.flag = ctx->hslot[i].flag;
+        o.seq = ++ctx->hseq[i];
+        return o;
+    }
+    qob_status wait(int parts) {
+        HostSlot &S = ctx->hslot[i];
+        const uint32_t seq = ctx->hseq[i];
+        int k = 0;  // numbers 0 .. k - 1 are there
+        auto there = [&] {
+            while (k < parts && __atomic_load_n(&S.flag[k], __ATOMIC_ACQUIRE) == seq) ++k;
+            return k == parts;
+        };
+        const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        bool ok = there();
+        while (!ok && std::chrono::steady_clock::now() < end) {
+            for (int q = 0; q < 16 && !(ok = there()); ++q) __builtin_ia32_pause();
+        }
+        if (!ok) {
+            QOB_HIP(hipStreamSynchronize(st));
+            if (!there()) return fail(QOB_EHIP, "a reduction finished without its result");
+        }
+        queued = false;
         return QOB_OK;
     }
-    HostSlot &S = ctx->hslot[i];
-    const uint32_t seq = ++ctx->hseq[i];
-    hipError_t e = launch_final(mode, a, b, S.v, &S.flag, seq, st);
-    if (e != hipSuccess) {
-        ctx->hfree.fetch_or(1ull << i, std::memory_order_release);
-        return fail(QOB_EHIP, "reduction launch: %s", hipGetErrorString(e));
+    // the sums of the workgroups that out(parts) was given to
+    qob_status sum(RedMode mode, int parts, int sets, double2 *h) {
+        QOB_TRY(wait(parts));
+        const HostSlot &S = ctx->hslot[i];
+        for (int t = 0; t < sets; ++t) {
+            double2 r = make_double2(0, 0);
+            for (int k = 0; k < parts; ++k) {
+                r.x += S.v[t * parts + k].x;
+                r.y += S.v[t * parts + k].y;
+            }
+            h[t] = r;
+        }
+        if (mode == RED_NORM) h[0].x = std::sqrt(h[0].x);
+        return QOB_OK;
     }
-    auto there = [&] { return __atomic_load_n(&S.flag, __ATOMIC_ACQUIRE) == seq; };
-    const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-    bool ok = there();
-    while (!ok && std::chrono::steady_clock::now() < end) {
-        for (int k = 0; k < 16 && !(ok = there()); ++k) __builtin_ia32_pause();
+    // the sums of one or two sets of partials queued in device memory
+    qob_status final(RedMode mode, RedSet a, RedSet b, double2 *h) {
+        if (i < 0) {
+            void *d;
+            QOB_TRY(scal_ws(ctx, st, d));
+            QOB_HIP(launch_final(mode, a, b, d, nullptr, 0, st));
+            QOB_HIP(hipMemcpyAsync(h, d, (b.n ? 2 : 1) * sizeof(double2), hipMemcpyDeviceToHost, st));
+            QOB_HIP(hipStreamSynchronize(st));
+            return QOB_OK;
+        }
+        const HostOut o = out(1);
+        QOB_HIP(launch_final(mode, a, b, o.v, o.flag, o.seq, st));
+        QOB_TRY(wait(1));
+        h[0] = o.v[0];
+        h[1] = o.v[1];
+        return QOB_OK;
     }
-    if (!ok) {
-        // on an error the slot stays taken: its kernel may still store there
-        QOB_HIP(hipStreamSynchronize(st));
-        if (!there()) return fail(QOB_EHIP, "a reduction finished without its result");
-    }
-    h[0] = S.v[0];
-    h[1] = S.v[1];
-    ctx->hfree.fetch_or(1ull << i, std::memory_order_release);
-    return QOB_OK;
+};
+
+static qob_status sums_to_host(qob_ctx ctx, hipStream_t st, RedMode mode, RedSet a, RedSet b, double2 *h) {
+    HostSum hs(ctx, st);
+    return hs.final(mode, a, b, h);
 }
 
 static qob_status reduce_to_host(qob_ctx ctx, qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y,
@@ -3593,9 +3651,14 @@ static qob_status reduce_to_host(qob_ctx ctx, qob_dtype dt, RedMode mode, int64_
     hipStream_t st = strm(ctx, s);
     double2 *part, h[2];
     QOB_TRY(red_ws(ctx, st, n, part));
-    hipError_t e = launch_partials(dt, mode, n, x, y, part, st);
+    HostSum hs(ctx, st);
+    // up to 2^13 elements as few sums as the host adds (four elements per thread)
+    const int nb = hs.i >= 0 && n <= 1024 * (int64_t)HOST_PARTS ? std::min(reduce_blocks(n), HOST_PARTS) : reduce_blocks(n);
+    const HostOut o = hs.out(nb);
+    hipError_t e = launch_partials(dt, mode, n, x, y, part, nb, o, st);
     if (e != hipSuccess) return fail(QOB_EHIP, "reduction launch: %s", hipGetErrorString(e));
-    QOB_TRY(sums_to_host(ctx, st, mode, RedSet{part, reduce_blocks(n)}, RedSet{}, h));
+    if (o.v) QOB_TRY(hs.sum(mode, nb, 1, h));
+    else QOB_TRY(hs.final(mode, RedSet{part, nb}, RedSet{}, h));
     r = h[0];
     return QOB_OK;
 }
@@ -3656,9 +3719,10 @@ qob_status qob_normalize_op(qob_ctx ctx, qob_dtype dt, int64_t n, void *A, qob_s
 
 // One pass of launch_qubit_dot over v, if op has a program for it: its two sets
 // of partials, or set.n = 0 and nothing launched.  square: only for an op that
-// is known to be Hermitian (not by device-held coefficients).
+// is known to be Hermitian (not by device-held coefficients).  Few partials go
+// to hs, which is the caller's to sum (set.p is null then).
 static qob_status qubit_dot_sums(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNode &op, const void *u, const void *v,
-                                 bool square, RedSet (&set)[2]) {
+                                 bool square, HostSum &hs, RedSet (&set)[2]) {
     set[0] = set[1] = RedSet{};
     if (!g_qubit_enable || (op.kind != K_LS && op.kind != K_LT) || (op.kind == K_LS && op.terms.empty()))
         return QOB_OK;
@@ -3675,26 +3739,28 @@ static qob_status qubit_dot_sums(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNo
     S.prog_hi_off = -1;
     S.in = v;
     S.out = nullptr;
+    const HostOut o = hs.out(nb);
     hipError_t e = launch_qubit_dot(dt, S, u, P->tbits, (const int32_t *)P->prog.p, P->vals.p, square, (double2 *)p,
-                                    st);
+                                    o, st);
     if (e != hipSuccess) return fail(QOB_EHIP, "fused expect: %s", hipGetErrorString(e));
-    set[0] = RedSet{(const double2 *)p, nb};
-    set[1] = RedSet{(const double2 *)p + nb, nb};
+    set[0] = RedSet{o.v ? nullptr : (const double2 *)p, nb};
+    set[1] = RedSet{o.v ? nullptr : (const double2 *)p + nb, nb};
     return QOB_OK;
 }
 
 // sum_J conj(u[J]) (op v)[J] without writing op v, when op has a fused
 // single-pass form: a qubit program or a square all-sparse gather plan.  The
 // partials are queued: hv of that sum, uv (on request) of sum conj(u[J]) v[J]
-// from the same pass.  hv.n = 0: no fused form, nothing launched.
+// from the same pass; on hs where p is null.  hv.n = 0: no fused form, nothing
+// launched.
 static qob_status fused_bilinear(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNode &op, const void *u,
-                                 const void *v, int64_t n, RedSet &hv, RedSet *uv = nullptr) {
+                                 const void *v, int64_t n, HostSum &hs, RedSet &hv, RedSet *uv = nullptr) {
     hv = RedSet{};
     if (op.kind != K_LS && op.kind != K_LT) return QOB_OK;
     if (op.kind == K_LS && op.terms.empty()) return QOB_OK;
     void *p;
     RedSet set[2];
-    QOB_TRY(qubit_dot_sums(ctx, st, dt, op, u, v, false, set));
+    QOB_TRY(qubit_dot_sums(ctx, st, dt, op, u, v, false, hs, set));
     if (set[0].n) {
         hv = set[0];
         if (uv) *uv = set[1];
@@ -3767,12 +3833,16 @@ qob_status qob_expect_ket(qob_ctx ctx, qob_dtype dt, qob_op a, const void *psi, 
     OpNode &op = *a->node;
     if (op.m != n || op.n != n) return fail(QOB_EDIM, "expect: operator %lldx%lld on state %lld", (long long)op.m, (long long)op.n, (long long)n);
     hipStream_t st = strm(ctx, s);
-    RedSet hv;
-    if (ctx->mode == QOB_MODE_FUSED) QOB_TRY(fused_bilinear(ctx, st, dt, op, psi, psi, n, hv));
-    if (hv.n) {
-        double2 h[2];
-        const qob_status q = sums_to_host(ctx, st, RED_DOT, hv, RedSet{}, h);
-        return give(q, h[0], out);
+    if (ctx->mode == QOB_MODE_FUSED) {
+        HostSum hs(ctx, st);
+        RedSet hv;
+        QOB_TRY(fused_bilinear(ctx, st, dt, op, psi, psi, n, hs, hv));
+        if (hv.n) {
+            double2 h[2];
+            if (hv.p) QOB_TRY(hs.final(RED_DOT, hv, RedSet{}, h));
+            else QOB_TRY(hs.sum(RED_DOT, hv.n, 1, h));
+            return give(QOB_OK, h[0], out);
+        }
     }
     // tmp = op * psi; <psi|tmp>  (src/operators.jl:119)
     void *tmp;
@@ -3814,16 +3884,17 @@ qob_status qob_variance_ket(qob_ctx ctx, qob_dtype dt, qob_op a, const void *psi
     RedSet e1, e2;
     void *x;
     Apply ap{ctx, st, dt, 1, 1, false};
+    HostSum hs(ctx, st);
     if (ctx->mode == QOB_MODE_FUSED) {
         RedSet set[2];
-        QOB_TRY(qubit_dot_sums(ctx, st, dt, op, psi, psi, true, set));
+        QOB_TRY(qubit_dot_sums(ctx, st, dt, op, psi, psi, true, hs, set));
         e2 = set[0];
         e1 = set[1];
     }
     if (!e2.n) {
         QOB_TRY(ws_get(ctx, st, WS_EXP, (size_t)n * esize(dt), x));
         QOB_TRY(apply_op(ap, op, psi, x, cd(1, 0), cd(0, 0)));
-        if (ctx->mode == QOB_MODE_FUSED) QOB_TRY(fused_bilinear(ctx, st, dt, op, psi, x, n, e2, &e1));
+        if (ctx->mode == QOB_MODE_FUSED) QOB_TRY(fused_bilinear(ctx, st, dt, op, psi, x, n, hs, e2, &e1));
     }
     if (!e2.n) {
         void *y, *part1;
@@ -3831,17 +3902,22 @@ qob_status qob_variance_ket(qob_ctx ctx, qob_dtype dt, qob_op a, const void *psi
         QOB_TRY(ws_get(ctx, st, WS_TMP1, (size_t)n * esize(dt), y));
         QOB_TRY(ws_get(ctx, st, WS_RED2, (size_t)reduce_blocks(n) * sizeof(double2), part1));
         QOB_TRY(red_ws(ctx, st, n, part2));
-        hipError_t e = launch_partials(dt, RED_DOT, n, psi, x, (double2 *)part1, st);
+        hipError_t e = launch_partials(dt, RED_DOT, n, psi, x, (double2 *)part1, reduce_blocks(n), HostOut{}, st);
         if (e == hipSuccess) {
             QOB_TRY(apply_op(ap, op, x, y, cd(1, 0), cd(0, 0)));
-            e = launch_partials(dt, RED_DOT, n, psi, y, part2, st);
+            e = launch_partials(dt, RED_DOT, n, psi, y, part2, reduce_blocks(n), HostOut{}, st);
         }
         if (e != hipSuccess) return fail(QOB_EHIP, "variance: %s", hipGetErrorString(e));
         e1 = RedSet{(const double2 *)part1, reduce_blocks(n)};
         e2 = RedSet{part2, reduce_blocks(n)};
     }
     double2 h[2];
-    QOB_TRY(sums_to_host(ctx, st, RED_DOT, e1, e2, h));
+    if (e2.p) {
+        QOB_TRY(hs.final(RED_DOT, e1, e2, h));
+    } else {  // the kernel's first sum is e2
+        QOB_TRY(hs.sum(RED_DOT, e2.n, 2, h));
+        std::swap(h[0], h[1]);
+    }
     const cd ex(h[0].x, h[0].y), ex2(h[1].x, h[1].y);
     const cd v = ex2 - ex * ex;
     out->re = v.real();

@@ -129,7 +129,7 @@ __device__ __forceinline__ double2 block_sum(double2 v, double2 *sh) {
 // mode 0: dot (conj(x) y), 1: |x|^2 in .x, 2: trace (x = A, stride ld+1)
 template <typename T, int MODE>
 __global__ void __launch_bounds__(BS) k_reduce1(int64_t n, const T *__restrict__ x, const T *__restrict__ y,
-                                               int64_t step, double2 *__restrict__ partials) {
+                                               int64_t step, double2 *__restrict__ partials, HostOut host) {
     __shared__ double2 sh[BS / 64];
     double2 acc = make_double2(0, 0);
     for (int64_t i = blockIdx.x * (int64_t)BS + threadIdx.x; i < n; i += (int64_t)gridDim.x * BS) {
@@ -149,7 +149,11 @@ __global__ void __launch_bounds__(BS) k_reduce1(int64_t n, const T *__restrict__
         }
     }
     double2 r = block_sum(acc, sh);
-    if (threadIdx.x == 0) partials[blockIdx.x] = r;
+    if (host.v) {
+        if (threadIdx.x < 64) put_host(host, 1, r);
+    } else if (threadIdx.x == 0) {
+        partials[blockIdx.x] = r;
+    }
 }
 
 // final stage: one block sums the partials of one or two sets; mode 1 writes
@@ -326,20 +330,19 @@ hipError_t launch_convert(qob_dtype from, const void *src, qob_dtype to, void *d
 
 template <int MODE>
 static hipError_t reduce1(qob_dtype dt, int64_t n, const void *x, const void *y, int64_t step, double2 *partials,
-                          hipStream_t s) {
-    const int g = reduce_blocks(n);
+                          int g, const HostOut &host, hipStream_t s) {
     if (dt == QOB_C64)
-        hipLaunchKernelGGL((k_reduce1<double2, MODE>), g, BS, 0, s, n, (const double2 *)x, (const double2 *)y, step, partials);
+        hipLaunchKernelGGL((k_reduce1<double2, MODE>), g, BS, 0, s, n, (const double2 *)x, (const double2 *)y, step, partials, host);
     else
-        hipLaunchKernelGGL((k_reduce1<float2, MODE>), g, BS, 0, s, n, (const float2 *)x, (const float2 *)y, step, partials);
+        hipLaunchKernelGGL((k_reduce1<float2, MODE>), g, BS, 0, s, n, (const float2 *)x, (const float2 *)y, step, partials, host);
     return hipGetLastError();
 }
 
 hipError_t launch_partials(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
-                           hipStream_t s) {
-    if (mode == RED_DOT) return reduce1<0>(dt, n, x, y, 1, partials, s);
-    if (mode == RED_NORM) return reduce1<1>(dt, n, x, x, 1, partials, s);
-    return reduce1<2>(dt, n, x, x, n + 1, partials, s);
+                           int blocks, const HostOut &host, hipStream_t s) {
+    if (mode == RED_DOT) return reduce1<0>(dt, n, x, y, 1, partials, blocks, host, s);
+    if (mode == RED_NORM) return reduce1<1>(dt, n, x, x, 1, partials, blocks, host, s);
+    return reduce1<2>(dt, n, x, x, n + 1, partials, blocks, host, s);
 }
 
 hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq, hipStream_t s) {
@@ -350,7 +353,7 @@ hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, uint32_t *f
 
 hipError_t launch_reduce(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
                          void *out, hipStream_t s) {
-    const hipError_t e = launch_partials(dt, mode, n, x, y, partials, s);
+    const hipError_t e = launch_partials(dt, mode, n, x, y, partials, reduce_blocks(n), HostOut{}, s);
     if (e != hipSuccess) return e;
     return launch_final(mode, RedSet{partials, reduce_blocks(n)}, RedSet{}, out, nullptr, 0, s);
 }

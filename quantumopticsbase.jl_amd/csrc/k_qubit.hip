@@ -784,7 +784,7 @@ __global__ void __launch_bounds__(NTH) k_qubit_hi(const QubitStateDev *__restric
 template <typename T, int NTH, int TBITS>
 __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__restrict__ u, int ntiles,
                                                    const int32_t *__restrict__ prog, const T *__restrict__ vals,
-                                                   int square, double2 *__restrict__ partials) {
+                                                   int square, double2 *__restrict__ partials, HostOut host) {
     constexpr int EPT = (1 << TBITS) / NTH;
     extern __shared__ unsigned char lds_raw[];
     T *tile = (T *)lds_raw;
@@ -836,13 +836,14 @@ __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__r
         red[1][tid >> 6] = make_double2(px, py);
     }
     __syncthreads();
-    if (tid < 2) {
+    if (tid < 64) {
         double2 t = make_double2(0, 0);
         for (int w = 0; w < NTH / 64; ++w) {
-            t.x += red[tid][w].x;
-            t.y += red[tid][w].y;
+            t.x += red[tid & 1][w].x;
+            t.y += red[tid & 1][w].y;
         }
-        partials[tid * gridDim.x + blockIdx.x] = t;
+        if (host.v) put_host(host, 2, t);
+        else if (tid < 2) partials[tid * gridDim.x + blockIdx.x] = t;
     }
 }
 
@@ -1106,7 +1107,8 @@ int qubit_dot_blocks(int64_t ntiles) {
 }
 
 hipError_t launch_qubit_dot(qob_dtype dt, QubitStateDev single, const void *u, int tbits, const int32_t *prog,
-                            const void *vals, bool square, double2 *partials, hipStream_t s) {
+                            const void *vals, bool square, double2 *partials, const HostOut &host,
+                            hipStream_t s) {
     if (tbits < 10 || tbits > 13) return hipErrorInvalidValue;
     const int tb = std::min(tbits, (int)single.nbits);
     const int64_t ntiles = (int64_t)1 << (single.nbits - tb);
@@ -1125,7 +1127,7 @@ hipError_t launch_qubit_dot(qob_dtype dt, QubitStateDev single, const void *u, i
             lds_set.store(1);                                                                                   \
         }                                                                                                       \
         hipLaunchKernelGGL(kfn, dim3(g), dim3(NTD), lds, s, single, (const TT *)u, (int)ntiles, prog,           \
-                           (const TT *)vals, square ? 1 : 0, partials);                                         \
+                           (const TT *)vals, square ? 1 : 0, partials, host);                                   \
         return hipGetLastError();                                                                               \
     } while (0)
     if (dt == QOB_C64) {

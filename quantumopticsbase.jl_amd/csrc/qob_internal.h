@@ -104,6 +104,29 @@ template <typename T> __device__ __forceinline__ void stg_stream(T *p, T v) {
     __builtin_nontemporal_store(w, (QOB_GLOBAL V *)p);
 }
 
+// ---------------------------------------------------- partials on the host
+// Where a kernel leaves few partial sums, the host adds them: workgroup b
+// stores its sum to v[b] (a second one to v[gridDim.x + b]) in pinned memory
+// and then seq to flag[b].  v == nullptr: the partials go to device memory.
+struct HostOut {
+    double2 *v = nullptr;
+    uint32_t *flag = nullptr;
+    uint32_t seq = 0;
+};
+// all threads of the wave that holds the workgroup's sums; lane k < n has
+// sum k.  System-scope stores are written through, so their acknowledgement
+// orders them before the flag; a release would write the L2 back first.
+__device__ __forceinline__ void put_host(const HostOut &H, int n, double2 r) {
+    const int k = threadIdx.x & 63;
+    if (k < n) {
+        double2 *p = H.v + k * (int)gridDim.x + blockIdx.x;
+        __hip_atomic_store(&p->x, r.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&p->y, r.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (k == 0) __hip_atomic_store(H.flag + blockIdx.x, H.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------ fast integer divide
 // q = n / d for 0 <= n < 2^31 with a host-computed multiplier:
 //   l = ceil(log2 d), m = floor(2^32 (2^l - d) / d) + 1,
@@ -209,7 +232,7 @@ struct RedSet {
 };
 int reduce_blocks(int64_t n);
 hipError_t launch_partials(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
-                           hipStream_t s);
+                           int blocks, const HostOut &host, hipStream_t s);
 hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq, hipStream_t s);
 hipError_t launch_reduce(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
                          void *out, hipStream_t s);
@@ -394,7 +417,7 @@ hipError_t launch_gather_dot(qob_dtype dt, const GatherPlanDev &P, int mode, con
 // after the first's.
 int qubit_dot_blocks(int64_t ntiles);
 hipError_t launch_qubit_dot(qob_dtype dt, QubitStateDev single, const void *u, int tbits, const int32_t *prog,
-                            const void *vals, bool square, double2 *partials, hipStream_t s);
+                            const void *vals, bool square, double2 *partials, const HostOut &host, hipStream_t s);
 // sum over the nonzeros of a CSC matrix X (n columns) of val * V[c + row * n]:
 // tr(X V) for an n x n V (expect(::SparseOpPureType, ::Operator))
 int csc_trace_blocks(int64_t n);

@@ -299,3 +299,24 @@ def test_variance_of_hermitian_and_other_sums(L, kind, dtype, tol):
     H.set_factors_device(d)
     got = Q.variance(H, k)
     assert abs(got - _var(M2, psi)) <= tol * max(1.0, np.linalg.norm(M2 @ psi) * np.linalg.norm(M2.conj().T @ psi))
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 2049, 8192, 8193, 70001])
+@pytest.mark.parametrize("dtype,eps", [(np.complex128, 1e-13), (np.complex64, 1e-13)])
+def test_scalars_of_few_and_many_workgroups(n, dtype, eps):
+    """norm, dot and trace whose sums the host adds (up to eight workgroups) and
+    those a second kernel adds: FP64 sums of products that are exact in FP64
+    for ComplexF32 inputs."""
+    g = np.random.default_rng(n)
+    x = (g.standard_normal(n) + 1j * g.standard_normal(n)).astype(dtype)
+    y = (g.standard_normal(n) + 1j * g.standard_normal(n)).astype(dtype)
+    B = Q.GenericBasis(n)
+    kx, ky = Q.Ket(B, x, dtype), Q.Ket(B, y, dtype)
+    x, y = x.astype(complex), y.astype(complex)
+    nx = np.linalg.norm(x)
+    assert abs(Q.norm(kx) - nx) <= eps * nx
+    assert abs(Q.dot(kx, ky) - np.vdot(x, y)) <= eps * nx * np.linalg.norm(y)
+    if n <= 2049:
+        M = np.zeros((n, n), dtype)
+        M[np.arange(n), np.arange(n)] = y
+        assert abs(Q.tr(Q.Operator(B, B, M, dtype)) - y.sum()) <= eps * abs(y).sum()
