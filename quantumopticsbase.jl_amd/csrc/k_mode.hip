@@ -28,6 +28,8 @@
 //                 with arbitrary element strides and a batch index, used for
 //                 factors wider than 64 and for DenseOperator on a density
 //                 matrix (and qob_gemm).
+//   k_zgemm_small the same with one 16 x 16 tile per workgroup, for products
+//                 of at most two tiles per CU.
 //   k_zgemv       a single vector (DenseOperator on a Ket or Bra): columns
 //                 of F split over workgroups, deterministic two-stage sum;
 //                 up to 1536 rows in one launch (k_zgemv_one).
@@ -316,7 +318,7 @@ __global__ void __launch_bounds__(CHUNK_NT) k_mode_chunk(const cplx<R> *__restri
 // Measured (ComplexF64 / ComplexF32, square, against one 64 x 64 tile shape
 // with none of these): 4096: 7.64 / 4.22 ms (71.9 / 130 TFLOP/s) from 9.76 /
 // 4.69; 3001: 3.21 / 1.76 from 4.05 / 1.97; 1000: 130 / 76 us from 186 / 110;
-// 200: 11 / 7.8 us from 40 / 25.  Not kept: loads two chunks ahead (no
+// 200: 11 / 7.8 us from 40 / 25 (k_zgemm_small since).  Not kept: loads two chunks ahead (no
 // change), k split over wave groups of one workgroup (no gain from 64^3 to
 // 4096^3), 8 k per chunk, a 64 x 64 tile (1-3% faster above 3000^3 in
 // ComplexF32, slower below 2000^3).
@@ -482,6 +484,74 @@ __global__ void __launch_bounds__(GNT, WPE) k_zgemm(int64_t M, int64_t N, int64_
                     *c = v;
                 }
             }
+}
+
+// ---------------------------------------------------------- k_zgemm_small
+// The same product where its tiles would leave most CUs idle: a workgroup has
+// one 16 x 16 tile of C, its four waves every fourth k-step of it, with the
+// fragments straight from memory (the operands fit the caches).  Bound by load
+// latency: k_zgemm waits for about one round trip per 16 k, here a wave has
+// SM_U k-steps of both operands in flight and the waves share the k range.
+// Their partial sums are added through LDS in wave order.  Against k_zgemm,
+// ComplexF64 / ComplexF32: (3000, 16, 3000) 149 / 99 -> 51 / 28 us, (128, 128,
+// 2000) 80 / 48 -> 30 / 20, 200^3 11.1 / 8.0 -> 6.6 / 5.0.
+constexpr int SM_U = 4;
+template <typename R>
+__global__ void __launch_bounds__(256) k_zgemm_small(int64_t M, int64_t N, int64_t K, const cplx<R> *__restrict__ A,
+                                                     int64_t sam, int64_t sak, int64_t sa, const cplx<R> *__restrict__ B,
+                                                     int64_t sbk, int64_t sbn, int64_t sb, cplx<R> *__restrict__ C,
+                                                     int64_t scm, int64_t scn, int64_t sc, int64_t tiles_m,
+                                                     int64_t tiles_n, double2 alpha_, double2 beta_, int beta_zero) {
+    using T = cplx<R>;
+    using V = typename mf<R>::v4;
+    __shared__ T red[4][16 * 17];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    int64_t bid = blockIdx.x;
+    const int64_t tm = bid % tiles_m;
+    bid /= tiles_m;
+    const int64_t tn = bid % tiles_n, z = bid / tiles_n;
+    const int64_t m0 = tm * 16, n0 = tn * 16;
+    // rows past M and columns past N read the last one (they only reach
+    // outputs that are not stored); k past K reads the last one as a zero
+    const T *a = A + z * sa + (m0 + lr < M ? m0 + lr : M - 1) * sam;
+    const T *b = B + z * sb + (n0 + lr < N ? n0 + lr : N - 1) * sbn;
+    V cr = V{0, 0, 0, 0}, ci = V{0, 0, 0, 0};
+    auto load = [&](int64_t k0, T (&x)[SM_U], T (&y)[SM_U]) {
+#pragma unroll
+        for (int u = 0; u < SM_U; ++u) {
+            const int64_t k = k0 + 16 * u + lk, kc = k < K ? k : K - 1;
+            x[u] = ldg(a + kc * sak);
+            y[u] = ldg(b + kc * sbk);
+        }
+#pragma unroll
+        for (int u = 0; u < SM_U; ++u)
+            if (k0 + 16 * u + lk >= K) x[u] = y[u] = czero<T>();
+    };
+    T x[SM_U], y[SM_U], xn[SM_U], yn[SM_U];
+    int64_t k0 = 4 * wave;
+    load(k0, x, y);
+    for (; k0 < K; k0 += 16 * SM_U) {
+        load(k0 + 16 * SM_U, xn, yn);
+#pragma unroll
+        for (int u = 0; u < SM_U; ++u) cmma4<R>(x[u], y[u], cr, ci);
+#pragma unroll
+        for (int u = 0; u < SM_U; ++u) {
+            x[u] = xn[u];
+            y[u] = yn[u];
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][mf<R>::row(lane, r) + 17 * lr] = mk((R)cr[r], (R)ci[r]);
+    __syncthreads();
+    const int i = tid & 15, j = tid >> 4;
+    if (m0 + i < M && n0 + j < N) {
+        T s = red[0][i + 17 * j];
+        for (int w = 1; w < 4; ++w) s = cadd(s, red[w][i + 17 * j]);
+        const T alpha = mk((R)alpha_.x, (R)alpha_.y), beta = mk((R)beta_.x, (R)beta_.y);
+        T *o = C + z * sc + (m0 + i) * scm + (n0 + j) * scn;
+        *o = axpby(alpha, s, beta, o, beta_zero != 0);
+    }
 }
 
 // --------------------------------------------------------------- k_zgemv
@@ -748,11 +818,27 @@ hipError_t launch_zgemm(qob_dtype dt, int64_t M, int64_t N, int64_t K, const voi
                            (const cplx<RR> *)B, sbk, sbn, sb, (cplx<RR> *)C, scm, scn, sc, tmn, tnn, alpha, beta, bz); \
         return hipGetLastError();                                                                               \
     } while (0)
+    const int64_t ncu = device_cu_count();
+    // Few 16 x 16 tiles and a k range worth splitting: one tile per workgroup
+    // (square, k_zgemm / k_zgemm_small: ComplexF64 200 11.1 / 6.6 us, 350 18.1 /
+    // 13.4, 400 (625 tiles) 19.8 / 20.1; ComplexF32 200 8.0 / 5.0, 350 13.9 / 9.7,
+    // 400 14.8 / 16.4; (350, 350, 64) in ComplexF32 4.7 / 6.3, so short ranges
+    // only where half of the CUs would have no tile).
+    const int64_t t16m = (M + 15) / 16, t16n = (N + 15) / 16, t16 = t16m * t16n * batch;
+    if (t16 <= 2 * ncu && (K >= 128 || 2 * t16 <= ncu)) {
+#define QOB_ZS(RR)                                                                                                  \
+    hipLaunchKernelGGL(k_zgemm_small<RR>, dim3((unsigned)t16), dim3(256), 0, s, M, N, K, (const cplx<RR> *)A, sam,  \
+                       sak, sa, (const cplx<RR> *)B, sbk, sbn, sb, (cplx<RR> *)C, scm, scn, sc, t16m, t16n, alpha,  \
+                       beta, bz)
+        if (dt == QOB_C64) QOB_ZS(double);
+        else QOB_ZS(float);
+#undef QOB_ZS
+        return hipGetLastError();
+    }
     // Tile: a launch takes about (rounds of tiles over the CUs) x (tile area),
     // the 32 x 32 tile at 0.92 of the 64 x 32 tile's rate (68 against 72
     // TFLOP/s at 4096^3 in ComplexF64).  With few tiles per CU the smaller
     // one also keeps more waves in flight (700^3: 52 against 58 us).
-    const int64_t ncu = device_cu_count();
     const int64_t nl = ((M + 63) / 64) * ((N + 31) / 32) * batch, ns = ((M + 31) / 32) * ((N + 31) / 32) * batch;
     const int64_t rl = (nl + ncu - 1) / ncu, rs = (ns + ncu - 1) / ncu;
     const bool large = rl > 2 && 200 * rl < 109 * rs;

@@ -438,3 +438,29 @@ def test_dense_operator_on_vectors(shape, dtype):
     assert rel(Q.mul_(b, Q.Bra(gb(m), y, dtype), op).to_numpy(), y @ A) < TOLS[dtype]
     b = Q.Bra(gb(n), x, dtype)
     assert rel(Q.mul_(b, Q.Bra(gb(m), y, dtype), op, 0.5j, -0.25).to_numpy(), 0.5j * (y @ A) - 0.25 * x) < TOLS[dtype]
+
+
+# 16 x 16 tiles and k ranges around a wave's four k-steps of 4 (k_zgemm_small),
+# one shape on each side of its tile count and of its shortest k range, and the
+# 32 x 32 tile at its edges
+GEMM_SMALL = [(1, 2, 1), (15, 17, 3), (16, 16, 4), (17, 33, 5), (5, 7, 63), (16, 32, 64), (31, 16, 65), (100, 2, 257),
+              (3, 3000, 200), (350, 352, 127), (350, 352, 128), (361, 353, 130), (385, 400, 33), (400, 385, 16)]
+
+
+@pytest.mark.parametrize("mnk", GEMM_SMALL)
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("dtype", DTS)
+def test_qob_gemm_few_tiles(mnk, transa, dtype):
+    """Against numpy in ComplexF64 (sums of at most 257 products), and a NaN row of
+    op(A) reaches its row of the result and no other."""
+    test_qob_gemm_tile_edges(mnk, transa, dtype)
+    g = np.random.default_rng(12)
+    m, n, k = mnk
+    opA, B = cg(g, m, k).astype(dtype), cg(g, k, n).astype(dtype)
+    opA[m // 2, k - 1] = np.nan
+    dA = Q.DeviceArray.from_numpy(opA.T if transa else opA, dtype)
+    dB, dC = Q.DeviceArray.from_numpy(B, dtype), Q.DeviceArray.from_numpy(np.zeros((m, n), complex), dtype)
+    _lib.call("qob_gemm", Q.context().h, dA.qdt, transa, m, n, k, _lib.c64(1.0), dA.ptr, dB.ptr, _lib.c64(0.0), dC.ptr,
+              None)
+    bad = np.isnan(dC.to_numpy())
+    assert bad[m // 2].all() and bad.sum() == n
