@@ -29,7 +29,7 @@
 //                 factors wider than 64 and for DenseOperator on a density
 //                 matrix (and qob_gemm).
 //   k_zgemm_small the same with one 16 x 16 tile per workgroup, for products
-//                 of at most two tiles per CU.
+//                 of few tiles per CU.
 //   k_zgemv       a single vector (DenseOperator on a Ket or Bra): columns
 //                 of F split over workgroups, deterministic two-stage sum;
 //                 up to 1536 rows in one launch (k_zgemv_one).
@@ -493,8 +493,8 @@ __global__ void __launch_bounds__(GNT, WPE) k_zgemm(int64_t M, int64_t N, int64_
 // latency: k_zgemm waits for about one round trip per 16 k, here a wave has
 // SM_U k-steps of both operands in flight and the waves share the k range.
 // Their partial sums are added through LDS in wave order.  Against k_zgemm,
-// ComplexF64 / ComplexF32: (3000, 16, 3000) 149 / 99 -> 51 / 28 us, (128, 128,
-// 2000) 80 / 48 -> 30 / 20, 200^3 11.1 / 8.0 -> 6.6 / 5.0.
+// ComplexF64 / ComplexF32: (3000, 16, 3000) 149 / 99 -> 53 / 28 us, (128, 128,
+// 2000) 80 / 48 -> 34 / 20, 200^3 11.1 / 8.0 -> 6.6 / 5.0.
 constexpr int SM_U = 4;
 template <typename R>
 __global__ void __launch_bounds__(256) k_zgemm_small(int64_t M, int64_t N, int64_t K, const cplx<R> *__restrict__ A,
@@ -513,32 +513,50 @@ __global__ void __launch_bounds__(256) k_zgemm_small(int64_t M, int64_t N, int64
     const int64_t tn = bid % tiles_n, z = bid / tiles_n;
     const int64_t m0 = tm * 16, n0 = tn * 16;
     // rows past M and columns past N read the last one (they only reach
-    // outputs that are not stored); k past K reads the last one as a zero
+    // outputs that are not stored)
     const T *a = A + z * sa + (m0 + lr < M ? m0 + lr : M - 1) * sam;
     const T *b = B + z * sb + (n0 + lr < N ? n0 + lr : N - 1) * sbn;
     V cr = V{0, 0, 0, 0}, ci = V{0, 0, 0, 0};
-    auto load = [&](int64_t k0, T (&x)[SM_U], T (&y)[SM_U]) {
+    // a wave's groups of 4 SM_U k at k0, k0 + 16 SM_U, ...: full of them lie
+    // inside K and need one address addition per load
+    constexpr int G = 4 * SM_U;
+    const int64_t k0 = G * wave;
+    const int64_t full = K >= k0 + G ? (K - k0 - G) / (4 * G) + 1 : 0;
+    const T *pa = a + (k0 + lk) * sak, *pb = b + (k0 + lk) * sbk;
+    T x[SM_U], y[SM_U], xn[SM_U], yn[SM_U];
+    auto load = [&](T (&x)[SM_U], T (&y)[SM_U]) {
 #pragma unroll
         for (int u = 0; u < SM_U; ++u) {
-            const int64_t k = k0 + 16 * u + lk, kc = k < K ? k : K - 1;
-            x[u] = ldg(a + kc * sak);
-            y[u] = ldg(b + kc * sbk);
+            x[u] = ldg(pa + 4 * u * sak);
+            y[u] = ldg(pb + 4 * u * sbk);
         }
-#pragma unroll
-        for (int u = 0; u < SM_U; ++u)
-            if (k0 + 16 * u + lk >= K) x[u] = y[u] = czero<T>();
     };
-    T x[SM_U], y[SM_U], xn[SM_U], yn[SM_U];
-    int64_t k0 = 4 * wave;
-    load(k0, x, y);
-    for (; k0 < K; k0 += 16 * SM_U) {
-        load(k0 + 16 * SM_U, xn, yn);
+    if (full > 0) load(x, y);
+    for (int64_t g = 0; g < full; ++g) {
+        // the last group is loaded once more in place of one that is not there
+        pa += g + 1 < full ? 4 * G * sak : 0;
+        pb += g + 1 < full ? 4 * G * sbk : 0;
+        load(xn, yn);
 #pragma unroll
         for (int u = 0; u < SM_U; ++u) cmma4<R>(x[u], y[u], cr, ci);
 #pragma unroll
         for (int u = 0; u < SM_U; ++u) {
             x[u] = xn[u];
             y[u] = yn[u];
+        }
+    }
+    const int64_t kt = k0 + 4 * G * full;
+    if (kt < K) {  // k past K reads the last one as a zero
+#pragma unroll
+        for (int u = 0; u < SM_U; ++u) {
+            const int64_t k = kt + 4 * u + lk, kc = k < K ? k : K - 1;
+            x[u] = ldg(a + kc * sak);
+            y[u] = ldg(b + kc * sbk);
+        }
+#pragma unroll
+        for (int u = 0; u < SM_U; ++u) {
+            if (kt + 4 * u + lk >= K) x[u] = y[u] = czero<T>();
+            cmma4<R>(x[u], y[u], cr, ci);
         }
     }
 #pragma unroll
@@ -819,13 +837,16 @@ hipError_t launch_zgemm(qob_dtype dt, int64_t M, int64_t N, int64_t K, const voi
         return hipGetLastError();                                                                               \
     } while (0)
     const int64_t ncu = device_cu_count();
-    // Few 16 x 16 tiles and a k range worth splitting: one tile per workgroup
-    // (square, k_zgemm / k_zgemm_small: ComplexF64 200 11.1 / 6.6 us, 350 18.1 /
-    // 13.4, 400 (625 tiles) 19.8 / 20.1; ComplexF32 200 8.0 / 5.0, 350 13.9 / 9.7,
-    // 400 14.8 / 16.4; (350, 350, 64) in ComplexF32 4.7 / 6.3, so short ranges
-    // only where half of the CUs would have no tile).
+    // Few 16 x 16 tiles and a k range worth splitting: one tile per workgroup,
+    // up to two tiles per CU, in ComplexF64 up to four where A's rows are
+    // contiguous (square, k_zgemm / k_zgemm_small: ComplexF64 200 11.1 / 6.6 us,
+    // 350 18.1 / 11.0, 400 (625 tiles) 19.8 / 15.9, 500 24.5 / 22.4, but A
+    // transposed 512 23.7 / 34.3; ComplexF32 200 8.0 / 5.0, 350 13.9 / 8.7, 400
+    // 14.8 / 15.0, 512 17.2 / 22.4; (350, 350, 64) in ComplexF32 4.7 / 6.3, so
+    // short ranges only where half of the CUs would have no tile).
     const int64_t t16m = (M + 15) / 16, t16n = (N + 15) / 16, t16 = t16m * t16n * batch;
-    if (t16 <= 2 * ncu && (K >= 128 || 2 * t16 <= ncu)) {
+    const int64_t most = (dt == QOB_C64 && sam <= sak ? 4 : 2) * ncu;
+    if (t16 <= most && (K >= 128 || 2 * t16 <= ncu)) {
 #define QOB_ZS(RR)                                                                                                  \
     hipLaunchKernelGGL(k_zgemm_small<RR>, dim3((unsigned)t16), dim3(256), 0, s, M, N, K, (const cplx<RR> *)A, sam,  \
                        sak, sa, (const cplx<RR> *)B, sbk, sbn, sb, (cplx<RR> *)C, scm, scn, sc, t16m, t16n, alpha,  \

@@ -444,7 +444,7 @@ def test_dense_operator_on_vectors(shape, dtype):
 # one shape on each side of its tile count and of its shortest k range, and the
 # 32 x 32 tile at its edges
 GEMM_SMALL = [(1, 2, 1), (15, 17, 3), (16, 16, 4), (17, 33, 5), (5, 7, 63), (16, 32, 64), (31, 16, 65), (100, 2, 257),
-              (3, 3000, 200), (350, 352, 127), (350, 352, 128), (361, 353, 130), (385, 400, 33), (400, 385, 16)]
+              (3, 3000, 200), (350, 352, 127), (350, 352, 128), (361, 353, 130), (400, 500, 131), (513, 512, 129), (385, 400, 33), (400, 385, 16)]
 
 
 @pytest.mark.parametrize("mnk", GEMM_SMALL)
