@@ -994,8 +994,8 @@ namespace qob {
 // ------------------------------------------------------------- workspace
 // slots: chain temporaries, reductions, scalars, expect temporary, the
 // split partial sums of a dense matrix-vector product, the widened state and
-// result of a call whose state and result element types differ, op * rho of
-// a variance, and two LazyProduct temporaries per nesting depth (up to 4)
+// result of a call whose state and result element types differ, op * rho (op *
+// op * psi) of a variance, and two LazyProduct temporaries per nesting depth (up to 4)
 enum {
     WS_TMP1 = 0, WS_TMP2 = 1, WS_RED = 2, WS_SCAL = 3, WS_EXP = 4, WS_GEMV = 5, WS_MIXB = 6, WS_MIXR = 7,
     WS_VAR = 8, WS_LP0 = 9, WS_RED2 = 17, WS_NSLOT = 18
@@ -3899,7 +3899,8 @@ qob_status qob_variance_ket(qob_ctx ctx, qob_dtype dt, qob_op a, const void *psi
     if (!e2.n) {
         void *y, *part1;
         double2 *part2;
-        QOB_TRY(ws_get(ctx, st, WS_TMP1, (size_t)n * esize(dt), y));
+        // not one of the slots that an application takes for itself
+        QOB_TRY(ws_get(ctx, st, WS_VAR, (size_t)n * esize(dt), y));
         QOB_TRY(ws_get(ctx, st, WS_RED2, (size_t)reduce_blocks(n) * sizeof(double2), part1));
         QOB_TRY(red_ws(ctx, st, n, part2));
         hipError_t e = launch_partials(dt, RED_DOT, n, psi, x, (double2 *)part1, reduce_blocks(n), HostOut{}, st);

@@ -320,3 +320,60 @@ def test_scalars_of_few_and_many_workgroups(n, dtype, eps):
         M = np.zeros((n, n), dtype)
         M[np.arange(n), np.arange(n)] = y
         assert abs(Q.tr(Q.Operator(B, B, M, dtype)) - y.sum()) <= eps * abs(y).sum()
+
+
+@pytest.mark.parametrize("mode", ["fused", "plain"])
+@pytest.mark.parametrize("kind", ["sparse_dense", "wide", "three", "sum"])
+@pytest.mark.parametrize("dtype,eps", [(np.complex128, 2.0 ** -52), (np.complex64, 2.0 ** -23)])
+def test_variance_ket_of_several_passes(kind, mode, dtype, eps):
+    """variance on a Ket of operators whose application goes through a
+    temporary of its own: mode chains (a sparse factor beside a dense one,
+    factors wider than a site group takes) of two and three steps, and a sum
+    whose second term is applied over the first term's result.  An application
+    of factors of widths d rounds by less than 3/2 (sum d + 4) eps |M| |psi| per
+    element (complex products and sums, 3 for the modulus of both parts)."""
+    shape = {"sparse_dense": (6, 5), "wide": (70, 70), "three": (12, 45, 7), "sum": (41, 44)}[kind]
+    g = np.random.default_rng(41)
+    bases = [Q.GenericBasis(d) for d in shape]
+    B = Q.tensor(*bases)
+
+    def factors(sparse):
+        ms, fs = [], []
+        for i, (d, b) in enumerate(zip(shape, bases)):
+            m = (g.standard_normal((d, d)) + 1j * g.standard_normal((d, d))) / d
+            if i in sparse:
+                m = m * (g.random((d, d)) < 0.4)
+            m = m + np.diag(1 + g.random(d))
+            ms.append(m)
+            fs.append(Q.SparseOperator(b, b, sp.csc_matrix(m)) if i in sparse else Q.DenseOperator(b, b, m))
+        return ms, tuple(fs)
+
+    def dense(ms):
+        K = np.ones((1, 1))
+        for m in ms:  # the first site is the fastest
+            K = np.kron(m, K)
+        return K
+
+    sites = tuple(range(1, len(shape) + 1))
+    if kind == "sum":
+        (ma, fa), (mb, fb) = factors(()), factors((0,))
+        op = Q.LazySum(B, B, [0.7, -1.3j], (Q.LazyTensor(B, B, sites, fa), Q.LazyTensor(B, B, sites, fb)))
+        M = 0.7 * dense(ma) - 1.3j * dense(mb)
+        absM = 0.7 * abs(dense(ma)) + 1.3 * abs(dense(mb))
+    else:
+        ms, fs = factors({"sparse_dense": (0,), "three": (2,)}.get(kind, ()))
+        op, M = Q.LazyTensor(B, B, sites, fs), dense(ms)
+        absM = abs(M)
+    psi = g.standard_normal(len(B)) + 1j * g.standard_normal(len(B))
+    psi = (psi / np.linalg.norm(psi)).astype(dtype)
+    k = Q.Ket(B, psi, dtype)
+    want = _var(M, psi.astype(complex))
+    a = abs(psi.astype(complex))
+    bound = 3 * (sum(shape) + 4) * eps * (a @ (absM @ (absM @ a)) + (a @ (absM @ a)) ** 2)
+    ctx = Q.context()
+    ctx.set_mode(Q.QOB_MODE_PLAIN if mode == "plain" else Q.QOB_MODE_FUSED)
+    try:
+        got = Q.variance(op, k)
+    finally:
+        ctx.set_mode(Q.QOB_MODE_FUSED)
+    assert abs(got - want) <= bound
