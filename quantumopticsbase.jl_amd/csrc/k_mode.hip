@@ -32,8 +32,9 @@
 //                 of few tiles per CU.
 //   k_zgemv       a single vector (DenseOperator on a Ket or Bra): columns
 //                 of F split over workgroups, deterministic two-stage sum;
-//                 up to 1536 rows in one launch (k_zgemv_one).
+//                 up to 1536 rows and columns in one launch (k_zgemv_one).
 #include "qob_mfma.h"
+#include "qob_rules.h"
 
 #include <map>
 #include <mutex>
@@ -663,8 +664,9 @@ __global__ void __launch_bounds__(256) k_zgemv_sum(const cplx<double> *__restric
 }
 
 // The same in one launch: a workgroup covers 16 rows, lane l of wave w row
-// l % 16 and the columns 4 w + l / 16 + 64 t (runs of 16 rows).  The 64
-// partial sums of a row are added in FP64, in column order within a wave.
+// l % 16 and the columns 4 w + l / 16 + 64 t (runs of 16 rows).  A lane adds
+// GV_U products in the element type, everything above in FP64: a run that
+// does not grow with the number of columns.
 template <typename R>
 __global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ F, int64_t m, int64_t n,
                                                     const cplx<R> *__restrict__ x, cplx<R> *__restrict__ y,
@@ -675,7 +677,7 @@ __global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ 
     const int r = lane & 15;
     const int64_t i = (int64_t)blockIdx.x * 16 + r;
     const T *Fi = F + (i < m ? i : m - 1);
-    T acc = czero<T>();
+    double2 s = make_double2(0, 0);
     for (int64_t j = wave * 4 + (lane >> 4); j < n; j += 64 * GV_U) {
         T f[GV_U], v[GV_U];
 #pragma unroll
@@ -684,11 +686,13 @@ __global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ 
             f[u] = Fi[jj * m];
             v[u] = x[jj];
         }
+        T acc = czero<T>();
 #pragma unroll
         for (int u = 0; u < GV_U; ++u)
             if (j + 64 * u < n) acc = cfma(f[u], v[u], acc);
+        s.x += acc.x;
+        s.y += acc.y;
     }
-    double2 s = make_double2(acc.x, acc.y);
     for (int o = 16; o <= 32; o <<= 1) {
         s.x += __shfl_xor(s.x, o, 64);
         s.y += __shfl_xor(s.y, o, 64);
@@ -801,14 +805,8 @@ template <typename K> hipError_t raise_lds(K kfn, size_t bytes) {
 // and timing; the LDS chunks measured 2% faster on a (16, 32, 16) chain)
 int g_mode_kernel = 0;
 
-// Rows up to which one launch does it (k_zgemv_one): for the split kernel and
-// its sum the second launch costs more than their better use of the CUs gains
-// (n x n, ComplexF32: 803 6.2 against 4.6 + 2.8 us and a launch, 1414 8.5
-// against 5.8 + 2.8, but 2013 11.4 against 8.1 + 2.6).
-constexpr int64_t GV_ONE = 1536;
-
 int64_t zgemv_splits(int64_t m, int64_t n) {
-    if (m <= GV_ONE) return 1;
+    if (zgemv_in_one(m, n)) return 1;
     const int64_t rt = (m + 63) / 64;
     int64_t s = 1;
     while (rt * s < 1024 && n / (s * 2) >= 64) s *= 2;
@@ -876,7 +874,7 @@ hipError_t launch_zgemv(qob_dtype dt, const void *F, int64_t m, int64_t n, const
                         double2 alpha, double2 beta, hipStream_t s) {
     if (m <= 0) return hipSuccess;
     const int bz = (beta.x == 0.0 && beta.y == 0.0);
-    if (m <= GV_ONE) {
+    if (zgemv_in_one(m, n)) {
         const unsigned g = (unsigned)((m + 15) / 16);
         if (dt == QOB_C64)
             hipLaunchKernelGGL(k_zgemv_one<double>, dim3(g), dim3(1024), 0, s, (const double2 *)F, m, n,

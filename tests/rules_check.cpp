@@ -1,0 +1,24 @@
+// Prints the choices of csrc/qob_rules.h, one a line, for the questions on
+// stdin ("name arguments"); test_rules_host.py compares them.
+#include "../quantumopticsbase.jl_amd/csrc/qob_rules.h"
+
+#include <iostream>
+#include <sstream>
+#include <string>
+
+int main() {
+    std::string line, name;
+    while (std::getline(std::cin, line)) {
+        std::istringstream s(line);
+        s >> name;
+        if (name == "zgemv_in_one") {
+            long long m, n;
+            s >> m >> n;
+            std::cout << qob::zgemv_in_one(m, n) << "\n";
+        } else {
+            return 1;
+        }
+        if (!s) return 2;
+    }
+    return 0;
+}

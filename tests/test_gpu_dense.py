@@ -464,3 +464,18 @@ def test_qob_gemm_few_tiles(mnk, transa, dtype):
               None)
     bad = np.isnan(dC.to_numpy())
     assert bad[m // 2].all() and bad.sum() == n
+
+
+@pytest.mark.parametrize("m,n", [(1, 65536), (64, 65536), (40, 1536), (40, 1537), (1000, 5000)])
+def test_wide_matrix_on_a_ket_keeps_small_terms(m, n):
+    """A ComplexF32 row whose first products are 1 and all others 2^-25, which
+    a sum in FP32 that starts with a 1 drops.  At most 32 products and the four
+    waves' sums of them are added in FP32 (33 + 3 roundings of 2^-24 of the sum of
+    the magnitudes), all else in FP64, with one rounding of the result."""
+    A = np.full((m, n), 2.0 ** -25, np.complex64)
+    A[:, :64] = 1
+    want = 64 + (n - 64) * 2.0 ** -25
+    op = Q.Operator(gb(m), gb(n), A, np.complex64)
+    x = Q.Ket(gb(n), np.ones(n, np.complex64), np.complex64)
+    got = Q.mul_(Q.Ket(gb(m), np.full(m, np.nan + 0j), np.complex64), op, x, 1.0, 0.0).to_numpy().astype(complex)
+    assert np.abs(got - want).max() <= 37 * 2.0 ** -24 * want
