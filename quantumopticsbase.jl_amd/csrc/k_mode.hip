@@ -664,9 +664,10 @@ __global__ void __launch_bounds__(256) k_zgemv_sum(const cplx<double> *__restric
 }
 
 // The same in one launch: a workgroup covers 16 rows, lane l of wave w row
-// l % 16 and the columns 4 w + l / 16 + 64 t (runs of 16 rows).  A lane adds
-// GV_U products in the element type, everything above in FP64: a run that
-// does not grow with the number of columns.
+// l % 16 and the columns 4 w + l / 16 + 64 t (runs of 16 rows).  The 64
+// partial sums of a row are added in FP64, in column order within a wave: a
+// lane's run in the element type is at most 24 products (zgemv_in_one), as
+// long as the split kernel's.
 template <typename R>
 __global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ F, int64_t m, int64_t n,
                                                     const cplx<R> *__restrict__ x, cplx<R> *__restrict__ y,
@@ -677,7 +678,7 @@ __global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ 
     const int r = lane & 15;
     const int64_t i = (int64_t)blockIdx.x * 16 + r;
     const T *Fi = F + (i < m ? i : m - 1);
-    double2 s = make_double2(0, 0);
+    T acc = czero<T>();
     for (int64_t j = wave * 4 + (lane >> 4); j < n; j += 64 * GV_U) {
         T f[GV_U], v[GV_U];
 #pragma unroll
@@ -686,13 +687,11 @@ __global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ 
             f[u] = Fi[jj * m];
             v[u] = x[jj];
         }
-        T acc = czero<T>();
 #pragma unroll
         for (int u = 0; u < GV_U; ++u)
             if (j + 64 * u < n) acc = cfma(f[u], v[u], acc);
-        s.x += acc.x;
-        s.y += acc.y;
     }
+    double2 s = make_double2(acc.x, acc.y);
     for (int o = 16; o <= 32; o <<= 1) {
         s.x += __shfl_xor(s.x, o, 64);
         s.y += __shfl_xor(s.y, o, 64);
