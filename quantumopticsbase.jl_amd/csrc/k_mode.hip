@@ -708,55 +708,61 @@ __global__ void __launch_bounds__(1024) k_zgemv_one(const cplx<R> *__restrict__ 
 // y[i] = alpha * sum_l A[l + i k] x[l] + beta * y[i] (y = A^T x for a
 // column-major k x m A): one wave per output, lanes along the column (1 KiB
 // runs), U loads of each in flight, then a butterfly sum over the wave in a
-// fixed order.  A load is 16 bytes, one complex double or two complex floats
-// (8-byte aligned in a matrix of odd height; ComplexF32 6143 65.8 -> 51.1 us,
-// 7389 95.7 -> 75.9, 2013 unchanged.  The same for k_zgemv: 6143 58.4 -> 55.2,
-// but 8192 92 -> 99, not kept).
-template <typename R> constexpr int GV_VL = sizeof(R) == 8 ? 1 : 2;
+// fixed order.  A load is VL elements: 16 bytes, one complex double or two complex
+// floats (8-byte aligned in a matrix of odd height; ComplexF32 6143 65.8 ->
+// 51.1 us, 7389 95.7 -> 75.9, 2013 unchanged.  The same for k_zgemv: 6143 58.4 ->
+// 55.2, but 8192 92 -> 99, not kept), or one complex float of a short column.
 typedef float gv_f4 __attribute__((ext_vector_type(4), aligned(8)));
 __device__ __forceinline__ void gv_load(const double2 *p, double2 (&v)[1]) { v[0] = *p; }
+__device__ __forceinline__ void gv_load(const float2 *p, float2 (&v)[1]) { v[0] = *p; }
 __device__ __forceinline__ void gv_load(const float2 *p, float2 (&v)[2]) {
     const gv_f4 w = *(const gv_f4 *)p;
     v[0] = make_float2(w.x, w.y);
     v[1] = make_float2(w.z, w.w);
 }
-template <typename R, int U>
+template <typename R, int U, int VL>
 __global__ void __launch_bounds__(256) k_zgemv_t(const cplx<R> *__restrict__ A, int64_t k, int64_t m,
                                                  const cplx<R> *__restrict__ x, cplx<R> *__restrict__ y,
                                                  double2 alpha_, double2 beta_, int beta_zero) {
     using T = cplx<R>;
-    constexpr int VL = GV_VL<R>;
     constexpr int64_t ST = 64 * VL;
     const int lane = threadIdx.x & 63;
     const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= m) return;
     const T *Ai = A + i * k;
     T acc = czero<T>();
-    int64_t l = lane * VL;
-    for (; l + ST * (U - 1) + VL <= k; l += ST * U) {
+    int64_t b = 0;
+    for (; b + ST * U <= k; b += ST * U) {
         T a[U][VL], v[U][VL];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            gv_load(Ai + l + ST * u, a[u]);
-            gv_load(x + l + ST * u, v[u]);
+            gv_load(Ai + b + lane * VL + ST * u, a[u]);
+            gv_load(x + b + lane * VL + ST * u, v[u]);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int e = 0; e < VL; ++e) acc = cfma(a[u][e], v[u][e], acc);
     }
-    // what is left of the column, element by element
-    {
-        T a[U * VL], v[U * VL];
+    // what is left of the column, element by element, no loads for runs that
+    // start behind its end (uniform)
+    if (b < k) {
+        T a[U][VL], v[U][VL];
 #pragma unroll
-        for (int q = 0; q < U * VL; ++q) {
-            const int64_t p = l + ST * (q / VL) + q % VL, c = p < k ? p : k - 1;
-            a[q] = Ai[c];
-            v[q] = x[c];
-        }
+        for (int u = 0; u < U; ++u)
+            if (u == 0 || b + ST * u < k) {
 #pragma unroll
-        for (int q = 0; q < U * VL; ++q)
-            if (l + ST * (q / VL) + q % VL < k) acc = cfma(a[q], v[q], acc);
+                for (int e = 0; e < VL; ++e) {
+                    const int64_t p = b + ST * u + lane * VL + e, c = p < k ? p : k - 1;
+                    a[u][e] = Ai[c];
+                    v[u][e] = x[c];
+                }
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < VL; ++e)
+                if (b + ST * u + lane * VL + e < k) acc = cfma(a[u][e], v[u][e], acc);
     }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
@@ -908,21 +914,17 @@ hipError_t launch_zgemv_t(qob_dtype dt, const void *A, int64_t k, int64_t m, con
     if (m <= 0) return hipSuccess;
     const int bz = (beta.x == 0.0 && beta.y == 0.0);
     const unsigned g = (unsigned)((m + 3) / 4);
-    // Four loads in flight per lane, one for a matrix that streams from HBM
-    // anyway (n x n, one / four: ComplexF64 2013 13.6 / 11.6 us, 3009 26.5 /
-    // 22.8, 4500 48.5 / 55.4, 6143 91.6 / 102.4; ComplexF32, half as many loads
-    // per column, 2013 8.0 / 7.5, 3009 12.3 / 13.0, 4500 30.3 / 33.2, 6143 51.2 /
-    // 54.2).
-    const bool one = (double)k * m * (dt == QOB_C64 ? 16 : 8) > (double)((dt == QOB_C64 ? 256 : 64) << 20);
-#define QOB_GT(RR, U)                                                                                        \
-    hipLaunchKernelGGL((k_zgemv_t<RR, U>), dim3(g), dim3(256), 0, s, (const cplx<RR> *)A, k, m,              \
+#define QOB_GT(RR, U, VL)                                                                                    \
+    hipLaunchKernelGGL((k_zgemv_t<RR, U, VL>), dim3(g), dim3(256), 0, s, (const cplx<RR> *)A, k, m,          \
                        (const cplx<RR> *)x, (cplx<RR> *)y, alpha, beta, bz)
+    const GemvT f = zgemv_t_form(dt == QOB_C64, k, m);
     if (dt == QOB_C64) {
-        if (one) QOB_GT(double, 1);
-        else QOB_GT(double, 4);
+        if (f.loads == 1) QOB_GT(double, 1, 1);
+        else QOB_GT(double, 4, 1);
     } else {
-        if (one) QOB_GT(float, 1);
-        else QOB_GT(float, 4);
+        if (f.elems == 1) QOB_GT(float, 1, 1);
+        else if (f.loads == 1) QOB_GT(float, 1, 2);
+        else QOB_GT(float, 4, 2);
     }
 #undef QOB_GT
     return hipGetLastError();

@@ -15,4 +15,28 @@ namespace qob {
 // more rows: (2013, 2013) in ComplexF32 11.4 / 10.7.
 inline bool zgemv_in_one(int64_t m, int64_t n) { return m <= 1536 && n <= 1536; }
 
+// y = A^T x for a column-major k x m A, a wave per column (k_zgemv_t): loads in
+// flight per lane and elements per load.  Four loads hide the latency of
+// columns that come from the caches; a matrix that streams from HBM has enough
+// in flight with one where it also has the waves (n x n, one / four, us:
+// ComplexF64 2048 13.5 / 10.9, 3009 21.9 / 21.5, 3300 25.6 / 26.9, 4096 38.8 /
+// 40.7, 6143 91.6 / 102.4; ComplexF32, half as many loads per column, 2048 6.9 /
+// 5.1, 2896 11.3 / 11.4, 3300 13.7 / 14.9, 6143 51.2 / 54.2; fewer waves in
+// ComplexF64: (16384, 512) 80 / 29, (16384, 2048) 146 / 95, (16384, 3072) 164 /
+// 141, (2^20, 16) 5980 / 1930).  Columns that end within the first of four
+// loads leave the others idle, and in ComplexF32 half of the lanes too: (16,
+// 65536) four loads of two elements 13.0 us (31.5 with every load issued at the
+// column's end), one of two 10.6, one of one 9.8; (128, 262144) 56.1, 48.8, 54.9.
+struct GemvT {
+    int loads, elems;
+};
+inline GemvT zgemv_t_form(bool c64, int64_t k, int64_t m) {
+    const double mib = (double)k * m * (c64 ? 16 : 8) / (1 << 20);
+    GemvT f{4, c64 ? 1 : 2};
+    if (mib > (c64 ? 160 : 64) && m > 3072) f.loads = 1;
+    if (!c64 && k < 256) f.loads = 1;
+    if (!c64 && k < 128) f.elems = 1;
+    return f;
+}
+
 }  // namespace qob

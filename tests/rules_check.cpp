@@ -15,6 +15,11 @@ int main() {
             long long m, n;
             s >> m >> n;
             std::cout << qob::zgemv_in_one(m, n) << "\n";
+        } else if (name == "zgemv_t_form") {
+            long long c64, k, m;
+            s >> c64 >> k >> m;
+            const qob::GemvT f = qob::zgemv_t_form(c64 != 0, k, m);
+            std::cout << 10 * f.loads + f.elems << "\n";
         } else {
             return 1;
         }

@@ -479,3 +479,18 @@ def test_wide_matrix_on_a_ket_keeps_small_terms(m, n):
     x = Q.Ket(gb(n), np.ones(n, np.complex64), np.complex64)
     got = Q.mul_(Q.Ket(gb(m), np.full(m, np.nan + 0j), np.complex64), op, x, 1.0, 0.0).to_numpy().astype(complex)
     assert np.abs(got - want).max() <= 37 * 2.0 ** -24 * want
+
+
+@pytest.mark.parametrize("k", [1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 640, 1025])
+@pytest.mark.parametrize("dtype", DTS)
+def test_bra_over_column_lengths(k, dtype):
+    """The ends of a column around the runs of 64 and 128 elements and the loads in
+    flight, with a matrix of the width of a part of a workgroup, and a NaN in the
+    Bra's last element in every result."""
+    g = np.random.default_rng(k)
+    A, x = cg(g, k, 7).astype(dtype), cg(g, k, 1)[:, 0].astype(dtype)
+    op = Q.Operator(gb(k), gb(7), A, dtype)
+    b = Q.Bra(gb(7), np.full(7, np.nan + 0j), dtype)
+    assert rel(Q.mul_(b, Q.Bra(gb(k), x, dtype), op).to_numpy(), x.astype(complex) @ A) < TOLS[dtype]
+    x[k - 1] = np.nan
+    assert np.isnan(Q.mul_(b, Q.Bra(gb(k), x, dtype), op).to_numpy()).all()

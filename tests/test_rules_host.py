@@ -26,3 +26,11 @@ def ask(tmp_path_factory):
 def test_matrix_vector_in_one_launch_only_while_both_sides_are_short(ask):
     sizes = [(1, 1), (16, 1536), (1536, 1536), (1537, 16), (1536, 1537), (1, 1 << 20), (64, 65536), (1 << 20, 1)]
     assert ask(*(("zgemv_in_one", m, n) for m, n in sizes)) == [1, 1, 1, 0, 0, 0, 0, 0]
+
+
+def test_transposed_matrix_vector_loads(ask):
+    """10 * loads in flight + elements per load."""
+    c64 = [(16, 65536), (2048, 2048), (3200, 3200), (3300, 3300), (65536, 4), (1 << 20, 16)]
+    assert ask(*(("zgemv_t_form", 1, k, m) for k, m in c64)) == [41, 41, 41, 11, 41, 41]
+    c32 = [(3, 1 << 20), (16, 65536), (127, 10), (128, 10), (255, 10), (256, 10), (2048, 2048), (3300, 3300)]
+    assert ask(*(("zgemv_t_form", 0, k, m) for k, m in c32)) == [11, 11, 11, 12, 12, 42, 42, 12]
