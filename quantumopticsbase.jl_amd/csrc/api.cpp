@@ -10,6 +10,7 @@
 // Planning that the reference does per call (identity filtering, isometries,
 // strides, temporaries) is done once per operator and cached on its handle.
 #include "qob_internal.h"
+#include "qob_rules.h"
 
 #include <algorithm>
 #include <array>
@@ -1655,10 +1656,9 @@ struct QubitSplitSpec {
     int c(int nbits) const { return tb - (nbits - s); }
 };
 
-// tb: tile bits of the first pass.  With a second pass, the groups whose flips
-// stay inside its tiles go to a separate program.
-static bool compile_qubit(int nbits, const std::vector<TermSpec> &terms, QubitProgHost &Q, int tb,
-                          const QubitSplitSpec &sp) {
+// With a second pass, the groups whose flips stay inside its tiles go to a
+// separate program.  The first pass's program serves every tile size.
+static bool compile_qubit(int nbits, const std::vector<TermSpec> &terms, QubitProgHost &Q, const QubitSplitSpec &sp) {
     struct QT {
         cd coef;
         uint32_t F;
@@ -1759,13 +1759,18 @@ static bool compile_qubit(int nbits, const std::vector<TermSpec> &terms, QubitPr
         std::stable_partition(gs.begin(), gs.end(), [](const GroupOut &g) { return g.win.empty(); });
         int nconst = 0;
         for (auto &g : gs) nconst += g.win.empty() ? 1 : 0;
-        // header word 2: the first constant group whose flip leaves a tile of
-        // 2^min(tb, nbits) states (constant groups are in ascending F, so the
-        // ones before it read the tile and the rest read partner tiles)
-        int first_out = 0;
-        const int tbe = std::min(tb, nbits);
-        while (first_out < nconst && (gs[first_out].F >> tbe) == 0) ++first_out;
-        P.insert(P.end(), {nconst, (int32_t)gs.size() - nconst, pass == 0 ? first_out : 0, 0});
+        // header words 2 and 3: 16 bits for each tile size from 2^10 to 2^13,
+        // the first constant group whose flip leaves such a tile (constant
+        // groups are in ascending F, so the ones before it read the tile and
+        // the rest read partner tiles; one beyond 65535 reads its own tile as
+        // a partner's, which is slower but right)
+        uint32_t inside[2] = {0, 0};
+        for (int t = 0; t < 4 && pass == 0; ++t) {
+            int k = 0;
+            while (k < std::min(nconst, 0xffff) && (gs[k].F >> (10 + t)) == 0) ++k;
+            inside[t >> 1] |= (uint32_t)k << (16 * (t & 1));
+        }
+        P.insert(P.end(), {nconst, (int32_t)gs.size() - nconst, (int32_t)inside[0], (int32_t)inside[1]});
         for (auto &g : gs) {
             P.insert(P.end(), {(int32_t)g.F, (int32_t)g.win.size(), 0, 0});
             put_cd(P, g.c);
@@ -1783,7 +1788,6 @@ static bool compile_qubit(int nbits, const std::vector<TermSpec> &terms, QubitPr
 struct QubitPlan {
     bool ok = false;
     int nbits = 0;
-    int tbits = 12;
     int32_t hi_off = -1;  // offset of the second pass's program in prog, or -1
     QubitSplitSpec hi;
     DevBuf prog, vals;
@@ -1897,19 +1901,13 @@ int g_qubit_enable = 1;
 extern int g_qubit_tbits;
 int qubit_tbits(qob_dtype dt);
 
-// log2 of the tile of a single state (or of each column of a matrix).
-static int qubit_single_tbits(int nbits, qob_dtype dt) {
-    // Small tiles put a single state on more CUs: 18 sites 9.5 (2^12) -> 6.8 us
-    // (2^10) in ComplexF64, 9.7 (2^11) -> 7.7 us in ComplexF32; above 2^20
-    // states ComplexF32 does better with half the partner tiles (21 sites: 22
-    // against 24 us), ComplexF64 with more workgroups per CU (21 sites: 35
-    // against 40 us).
-    if (g_qubit_tbits) return g_qubit_tbits;
-    return dt == QOB_C64 || nbits <= 20 ? 10 : 11;
+// log2 of the tile of ncols states (qubit_state_tbits)
+static int qubit_tile_of(int nbits, qob_dtype dt, int64_t ncols, bool two_pass) {
+    return g_qubit_tbits ? g_qubit_tbits : qubit_state_tbits(nbits, dt == QOB_C64, ncols, two_pass);
 }
 
-// The second pass of one state of nbits bits whose first pass has 2^tb-state
-// tiles.
+// The second pass of one state of nbits bits (tb: of every bit above 2^tb-state
+// tiles, on request).
 static QubitSplitSpec qubit_split_of(int nbits, int tb, qob_dtype dt, bool single) {
     QubitSplitSpec sp;
     if (g_qubit_split) {
@@ -1946,9 +1944,9 @@ static qob_status qubit_plan(OpNode &op, bool trans, qob_dtype dt, hipStream_t s
         int nbits = 0;
         QubitProgHost H;
         const bool terms = qubit_terms(op, trans, specs, store, nbits, &base);
-        const int tb = qubit_single_tbits(nbits, dt);
-        const QubitSplitSpec sp = nosplit ? QubitSplitSpec() : qubit_split_of(nbits, tb, dt, true);
-        if (terms && compile_qubit(nbits, specs, H, tb, sp)) {
+        const QubitSplitSpec sp = nosplit || !terms ? QubitSplitSpec()
+                                                    : qubit_split_of(nbits, qubit_tile_of(nbits, dt, 1, false), dt, true);
+        if (terms && compile_qubit(nbits, specs, H, sp)) {
             std::vector<int32_t> all = H.prog;
             if (!H.prog_hi.empty()) {
                 P->hi_off = (int32_t)all.size();
@@ -1958,7 +1956,6 @@ static qob_status qubit_plan(OpNode &op, bool trans, qob_dtype dt, hipStream_t s
             QOB_TRY(P->prog.upload(all.data(), all.size() * 4));
             QOB_TRY(upload_vals(P->vals, H.vals, dt));
             P->nbits = nbits;
-            P->tbits = tb;
             P->dt = dt;
             P->ok = true;
             P->hermitian = qubit_hermitian(H.prog, H.vals) && qubit_hermitian(H.prog_hi, H.vals);
@@ -1974,7 +1971,7 @@ static qob_status qubit_plan(OpNode &op, bool trans, qob_dtype dt, hipStream_t s
                     std::vector<TermSpec> unit = specs;
                     for (size_t q = 0; q < unit.size(); ++q) unit[q].coef = (q == t) ? base[q] : cd(0, 0);
                     QubitProgHost U;
-                    same = compile_qubit(nbits, unit, U, tb, sp) && U.prog.size() == H.prog.size() &&
+                    same = compile_qubit(nbits, unit, U, sp) && U.prog.size() == H.prog.size() &&
                            U.prog_hi.size() == H.prog_hi.size() && U.vals.size() == H.vals.size();
                     if (!same) break;
                     std::vector<int32_t> ua = U.prog;
@@ -2410,8 +2407,9 @@ static qob_status apply_qubit(const Apply &ap, OpNode &op, const void *in, void 
     S.hi_shift = P->hi.s;
     S.in = in;
     S.out = out;
-    hipError_t e = launch_qubit_cols(ap.dt, S, ap.trail, P->tbits, (const int32_t *)P->prog.p, P->vals.p, d2(alpha),
-                                     d2(beta), make_double2(0, 0), ap.s);
+    hipError_t e = launch_qubit_cols(ap.dt, S, ap.trail, qubit_tile_of(P->nbits, ap.dt, ap.trail, P->hi_off >= 0),
+                                     (const int32_t *)P->prog.p, P->vals.p, d2(alpha), d2(beta), make_double2(0, 0),
+                                     ap.s);
     if (e == hipSuccess && P->hi_off >= 0)  // high-bit flips: out += alpha * high
         e = launch_qubit_hi_cols(ap.dt, S, ap.trail, P->hi.tb, (const int32_t *)P->prog.p, P->vals.p, d2(alpha),
                                  ap.s);
@@ -3729,7 +3727,7 @@ static qob_status qubit_dot_sums(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNo
     std::shared_ptr<QubitPlan> P;
     QOB_TRY(qubit_plan(op, false, dt, st, P, true));
     if (!P->ok || P->hi_off >= 0 || (square && (!P->hermitian || op.dcoef_on))) return QOB_OK;
-    const int tb = std::min(P->tbits, P->nbits);
+    const int tile = qubit_tile_of(P->nbits, dt, 1, false), tb = std::min(tile, P->nbits);
     const int nb = qubit_dot_blocks((int64_t)1 << (P->nbits - tb));
     void *p;
     QOB_TRY(ws_get(ctx, st, WS_RED, (size_t)nb * 2 * sizeof(double2), p));
@@ -3740,7 +3738,7 @@ static qob_status qubit_dot_sums(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNo
     S.in = v;
     S.out = nullptr;
     const HostOut o = hs.out(nb);
-    hipError_t e = launch_qubit_dot(dt, S, u, P->tbits, (const int32_t *)P->prog.p, P->vals.p, square, (double2 *)p,
+    hipError_t e = launch_qubit_dot(dt, S, u, tile, (const int32_t *)P->prog.p, P->vals.p, square, (double2 *)p,
                                     o, st);
     if (e != hipSuccess) return fail(QOB_EHIP, "fused expect: %s", hipGetErrorString(e));
     set[0] = RedSet{o.v ? nullptr : (const double2 *)p, nb};
@@ -4006,7 +4004,7 @@ qob_status qob_batch_create(qob_ctx ctx, int n, const qob_op *ops, qob_dtype dt,
         std::vector<std::vector<RowLists>> store;
         int nb = 0;
         QubitProgHost H;
-        if (!qubit_terms(*ops[j]->node, false, specs, store, nb) || !compile_qubit(nb, specs, H, B->tbits, qubit_split_of(nb, B->tbits, dt, false)))
+        if (!qubit_terms(*ops[j]->node, false, specs, store, nb) || !compile_qubit(nb, specs, H, qubit_split_of(nb, B->tbits, dt, false)))
             return fail(QOB_EUNSUPPORTED, "operator %d is not a qubit sum of monomial factors", j);
         // rebase the value offsets of this state's programs into the shared pool
         const int32_t vb = (int32_t)vals.size();

@@ -20,7 +20,7 @@
 //
 // Program of a state (int32, read with wave-uniform scalar loads; records
 // are multiples of 4 ints, so every record starts 16-byte aligned):
-//   header            [nconst, nwgroups, 0, 0]
+//   header            [nconst, nwgroups, groups inside a tile (see qb_inside)]
 //   nconst records    [F, 0, 0, 0, w.re, w.im]   (w as two doubles = 4 ints)
 //                     flip F with a constant, nonzero weight w
 //   nwgroups records  [F, nwin, 0, 0, c.re, c.im] each followed by nwin
@@ -186,6 +186,14 @@ struct HiMap {
     __device__ __forceinline__ uint32_t fq(uint32_t F) const { return ((F >> s) << c) | (F & lowmask); }
 };
 
+// Constant groups whose flips stay inside the 2^10..2^13-state tile of NTH EPT
+// elements: 16 bits each of header words 2 and 3, computed on the host.
+template <int NTH, int EPT> __device__ __forceinline__ int qb_inside(const int32_t *__restrict__ pg, int nconst) {
+    constexpr int t = NTH * EPT == 1024 ? 0 : NTH * EPT == 2048 ? 1 : NTH * EPT == 4096 ? 2 : 3;
+    static_assert(NTH * EPT == 1024 << t, "a tile of 2^10 to 2^13 states");
+    return min((int)(((uint32_t)pg[2 + t / 2] >> (16 * (t & 1))) & 0xffffu), nconst);
+}
+
 // acc[k] += w_F(J) * in[J ^ F] over the groups of one program, for the
 // EPT elements e = tid + k NTH of the lane's tile.  Elements past a partial
 // tile compute on unused LDS words and are never stored; partners of a
@@ -220,12 +228,12 @@ __device__ __forceinline__ void qb_run(const int32_t *__restrict__ pg, const T *
         };
         auto accum = [&](T wt, const T (&x)[EPT]) { qb_acc<T, EPT>(wt, x, acc); };
         // Constant groups are in ascending F: groups [0, nin) flip bits inside
-        // the tile (header word 2), the rest read partner tiles.  Partner
+        // the tile (qb_inside), the rest read partner tiles.  Partner
         // loads run one group ahead through two buffers, the first group's
         // during the in-tile groups; accumulation stays in program order.
-        // (nin is computed on the host for this tile size; the tile mask keeps
-        // every LDS read inside the tile whatever the program holds)
-        const int nin = min(max(pg[2], 0), nconst);
+        // (the tile mask keeps every LDS read inside the tile whatever the
+        // program holds)
+        const int nin = qb_inside<NTH, EPT>(pg, nconst);
         T A[EPT], B[EPT];
         // the first out-of-tile group's loads fly during the in-tile groups
         if (nin < nconst) issue((uint32_t)__builtin_amdgcn_readfirstlane(r[8 * nin]), A);
@@ -535,7 +543,7 @@ __device__ __forceinline__ void qb_run_pair(const int32_t *__restrict__ pg, cons
         qp_load_all<NTH, EPT, true>(gp, tpb_of(Fp), dst);
     };
     auto accum = [&](T wt, const T (&x)[EPT], uint32_t F) { qp_acc<EPT>(wt, x, (F & 1u) != 0, acc); };
-    const int nin = min(max(pg[2], 0), nconst);
+    const int nin = qb_inside<NTH, EPT>(pg, nconst);
     T A[EPT], B[EPT];
     if (nin < nconst) issue((uint32_t)__builtin_amdgcn_readfirstlane(r[8 * nin]), A);
     if (nin > 0) {
@@ -970,7 +978,7 @@ static hipError_t launch_qubit_any(qob_dtype dt, const QubitStateDev *states, co
     QubitSplit ws;
     const int flags = (beta.x == 0.0 && beta.y == 0.0 ? 1 : 0) | (gamma.x == 0.0 && gamma.y == 0.0 ? 2 : 0) |
                       qubit_walk_flags(nitems, g, xs, ws) | (g_qubit_ntfar ? 16 | ((g_qubit_ntfar - 1) << 5) : 0) |
-                      (dbuf ? 256 : 0) | (!states && single.prog_hi_off >= 0 ? 512 : 0);
+                      (dbuf ? 256 : 0) | (!states && single.prog_hi_off >= 0 && single.nbits >= tbits ? 512 : 0);
 #define QOB_QB(TT, NT, TB)                                                                                    \
     do {                                                                                                      \
         auto kfn = k_qubit<TT, NT, TB>;                                                                       \

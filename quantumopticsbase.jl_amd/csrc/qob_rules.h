@@ -39,4 +39,29 @@ inline GemvT zgemv_t_form(bool c64, int64_t k, int64_t m) {
     return f;
 }
 
+// log2 of the tile of ncols states of nbits bits (k_qubit; a reduction has one
+// column).  A larger tile reads fewer partner tiles from memory, a smaller one
+// gives more workgroups and waits less in each: 2^10 states while the tiles
+// are few or the partners are read from the caches.  2^10 / 2^11 / 2^12 tiles of
+// chains, us.  ComplexF32, 2^11 above 2^20 elements: 18 sites 6.6 / 7.7 / 9.6,
+// 12 sites of 256 columns (2^20) 7.9 / 8.2 / 8.1 and of 1024 25.7 / 19.0 / 20.2,
+// 16 sites of 256 111 / 79 / 83.  ComplexF64, 2^12 from about 2^23 elements on, where
+// input and output leave the Infinity Cache, later for shorter states, which
+// have fewer partners: 18 sites of 16 columns 38.8 / 40.6 / 42.0, of 32 (2^23) 78.6 /
+// 79.0 / 71.5, of 256 955 / 757 / 627; 16 sites of 128 62.5 / 60.3 / 64.4, of 256
+// (2^24) 124 / 112 / 116; 14 sites of 1024 106 / 100 / 110, of 4096 587 / 544 / 513;
+// 13 sites of 4096 (2^25) 251 / 247 / 240; expect of 25 sites 952 / 910 / 910.
+// The first of two passes has fewer partners: 23 sites 120 / 127 / 129, 24 of 2
+// columns (2^25) 666 / 658 / 624.
+inline int qubit_state_tbits(int nbits, bool c64, int64_t ncols, bool two_pass) {
+    int lg = nbits;  // log2 of all elements, rounded down
+    while (ncols > 1) {
+        ncols >>= 1;
+        ++lg;
+    }
+    if (!c64) return nbits > 10 && lg > 20 ? 11 : 10;
+    const int from = two_pass || nbits < 16 ? 25 : nbits < 18 ? 24 : 23;
+    return nbits >= 12 && lg >= from ? 12 : 10;
+}
+
 }  // namespace qob

@@ -20,6 +20,10 @@ int main() {
             s >> c64 >> k >> m;
             const qob::GemvT f = qob::zgemv_t_form(c64 != 0, k, m);
             std::cout << 10 * f.loads + f.elems << "\n";
+        } else if (name == "qubit_state_tbits") {
+            long long nbits, c64, ncols, two;
+            s >> nbits >> c64 >> ncols >> two;
+            std::cout << qob::qubit_state_tbits((int)nbits, c64 != 0, ncols, two != 0) << "\n";
         } else {
             return 1;
         }

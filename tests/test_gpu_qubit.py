@@ -489,3 +489,37 @@ def test_single_state_tiles_match_one_batch(L, dtype, tol):
     bt.apply(0, 0.3 - 0.8j, 0.0, 0.0)
     got = Q.mul_(Q.Ket(B, np.full(n, np.nan + 0j), dtype), H, psi, 0.3 - 0.8j, 0.0).to_numpy()
     assert O.rel_frobenius(got, out.to_numpy()) < tol
+
+
+# both sides of the lines of the tile rule, one and two passes
+@pytest.mark.parametrize("L,cols,dtype,tol", [
+    (11, 1023, np.complex64, 1e-6), (11, 1024, np.complex64, 1e-6), (18, 4, np.complex64, 1e-6), (18, 8, np.complex64, 1e-6),
+    (12, 8192, np.complex128, 1e-13), (16, 256, np.complex128, 1e-13), (18, 31, np.complex128, 1e-13),
+    (18, 32, np.complex128, 1e-13), (22, 3, np.complex128, 1e-13), (22, 8, np.complex128, 1e-13)])
+def test_columns_over_the_tile_rule(L, cols, dtype, tol):
+    """One operator on a Ket, then on the columns of a matrix (whose tile may be
+    another), then on the Ket again: each column against the same sum as a batch
+    of one (whose tile does not depend on the columns)."""
+    g = np.random.default_rng(L + cols)
+    H, _, B = build_pair(L, _long_terms(g, L) if L >= 20 else random_pauli_sum(g, L, 14))
+    n = 2 ** L
+    X = np.resize(cg(g, min(n * cols, 1 << 21)), n * cols + cols)[:n * cols].reshape((n, cols), order="F")
+    C = Q.GenericBasis(cols)
+    bt = Q.Batch([H], dtype)
+    out = Q.DeviceArray(n, dtype)
+
+    def check(got, j, al):
+        k = Q.Ket(B, np.ascontiguousarray(X[:, j]), dtype)
+        bt.bind(0, [k.data], [out])
+        bt.apply(0, al, 0.0, 0.0)
+        assert np.all(np.isfinite(got)) and O.rel_frobenius(got, out.to_numpy()) < tol
+
+    def ket(j, al):
+        k = Q.Ket(B, np.ascontiguousarray(X[:, j]), dtype)
+        check(Q.mul_(Q.Ket(B, np.full(n, np.nan + 0j), dtype), H, k, al, 0.0).to_numpy(), j, al)
+    ket(0, 1.0)
+    R = Q.Operator(B, C, Q.DeviceArray.from_numpy(np.full((n, cols), np.nan + 0j), dtype))
+    got = Q.mul_(R, H, Q.Operator(B, C, Q.DeviceArray.from_numpy(X, dtype)), 0.3 - 0.8j, 0.0).to_numpy()
+    for j in {0, 1, cols // 2, cols - 1}:
+        check(got[:, j], j, 0.3 - 0.8j)
+    ket(cols - 1, 0.5j)

@@ -34,3 +34,11 @@ def test_transposed_matrix_vector_loads(ask):
     assert ask(*(("zgemv_t_form", 1, k, m) for k, m in c64)) == [41, 41, 41, 11, 41, 41]
     c32 = [(3, 1 << 20), (16, 65536), (127, 10), (128, 10), (255, 10), (256, 10), (2048, 2048), (3300, 3300)]
     assert ask(*(("zgemv_t_form", 0, k, m) for k, m in c32)) == [11, 11, 11, 12, 12, 42, 42, 12]
+
+
+def test_tile_of_states_by_their_number(ask):
+    c64 = [(10, 1), (18, 1), (21, 1), (12, 256), (12, 8192), (11, 1 << 20), (16, 255), (16, 256), (18, 31), (18, 32), (22, 1), (25, 1)]
+    assert ask(*(("qubit_state_tbits", n, 1, c, 0) for n, c in c64)) == [10, 10, 10, 10, 12, 10, 10, 12, 10, 12, 10, 12]
+    assert ask(*(("qubit_state_tbits", n, 1, c, 1) for n, c in [(22, 4), (22, 8), (24, 1), (24, 2)])) == [10, 12, 10, 12]
+    c32 = [(3, 1), (10, 4096), (11, 1023), (11, 1024), (18, 4), (18, 8), (20, 1), (21, 1)]
+    assert ask(*(("qubit_state_tbits", n, 0, c, 0) for n, c in c32)) == [10, 10, 10, 11, 10, 11, 10, 11]
