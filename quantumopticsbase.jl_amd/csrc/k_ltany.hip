@@ -31,6 +31,7 @@
 // factors, three times as long on 40 wide ones), two groups of fibres per
 // wave at a time, 3 signed planes of the factor in LDS.
 #include "qob_mfma.h"
+#include "qob_rules.h"
 
 #include <atomic>
 #include <type_traits>
@@ -324,15 +325,7 @@ size_t any_plan(qob_dtype dt, AnyPass &S) {
             pad = E / S.m[0].d;
         }
     } else {
-        const int wmin = es == 16 ? 8 : 16;
-        int W = wmin;
-        // Too few tiles for the CUs: shorter runs, down to two rows, as long as
-        // the tiles stay one round (from the right on a rho that the MALL holds
-        // anyway; ComplexF64 / ComplexF32 (14, 9, 8): 8 / 16 rows 22.1 / 26.7 us,
-        // 4 rows and 252 tiles 17.7 / 18.5, 2 rows and 504 tiles 26.4 / 24.8).
-        while (W > 2 && 2 * ((S.n1 + W - 1) / W) * S.n3 <= device_cu_count()) W /= 2;
-        if (W == wmin)
-            while (W < 256 && (int64_t)(2 * W) * S.P * (int64_t)es <= 32 * 1024 && W < S.n1) W *= 2;
+        const int W = any_rows(es == 16, S.n1, S.P, S.n3, device_cu_count());
         S.W = W;
         while ((1 << S.lw) < W) ++S.lw;
         S.units = W;

@@ -64,4 +64,26 @@ inline int qubit_state_tbits(int nbits, bool c64, int64_t ncols, bool two_pass) 
     return nbits >= 12 && lg >= from ? 12 : 10;
 }
 
+// Rows of a tile of a site-group pass over n1 >= 16 rows of P elements in n3
+// blocks (k_ltany): runs of 128 bytes.
+// Too few tiles for the CUs: shorter runs, down to two rows, as long as the tiles
+// stay one round (from the right on a rho that the MALL holds anyway; ComplexF64 /
+// ComplexF32 (14, 9, 8): 8 / 16 rows 22.1 / 26.7 us, 4 rows and 252 tiles 17.7 /
+// 18.5, 2 rows and 504 tiles 26.4 / 24.8).
+// Small blocks: longer runs, up to 32 KiB of tile, while every CU still has a
+// tile (from the right, us: ComplexF32 without the first site of (16, 4, 4), 1000
+// rows, 256-row tiles 15.0, 64-row ones 9.7; (20, 3), 2469 rows, 64 / 32 / 16 rows
+// 15.4 / 7.8 / 7.8; ComplexF64 the outer two of (3, 6, 7), 2298 rows, 16 / 8 rows
+// 10.8 / 9.1).
+inline int any_rows(bool c64, int64_t n1, int64_t P, int64_t n3, int64_t ncu) {
+    const int64_t wmin = c64 ? 8 : 16, es = c64 ? 16 : 8;
+    auto tiles = [&](int64_t w) { return (n1 + w - 1) / w; };
+    int64_t W = wmin;
+    while (W > 2 && 2 * tiles(W) * n3 <= ncu) W /= 2;
+    if (W == wmin)
+        while (W < 256 && W < n1 && 2 * W * P * es <= 32 * 1024 && tiles(2 * W) * n3 >= ncu)
+            W *= 2;
+    return (int)W;
+}
+
 }  // namespace qob

@@ -24,6 +24,10 @@ int main() {
             long long nbits, c64, ncols, two;
             s >> nbits >> c64 >> ncols >> two;
             std::cout << qob::qubit_state_tbits((int)nbits, c64 != 0, ncols, two != 0) << "\n";
+        } else if (name == "any_rows") {
+            long long c64, n1, P, n3, ncu;
+            s >> c64 >> n1 >> P >> n3 >> ncu;
+            std::cout << qob::any_rows(c64 != 0, n1, P, n3, ncu) << "\n";
         } else {
             return 1;
         }

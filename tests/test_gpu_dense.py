@@ -494,3 +494,37 @@ def test_bra_over_column_lengths(k, dtype):
     assert rel(Q.mul_(b, Q.Bra(gb(k), x, dtype), op).to_numpy(), x.astype(complex) @ A) < TOLS[dtype]
     x[k - 1] = np.nan
     assert np.isnan(Q.mul_(b, Q.Bra(gb(k), x, dtype), op).to_numpy()).all()
+
+
+# (dims, sites, other dimension of the matrix, side) on both sides of the lines
+# that the choice of a pass and of its tile has: rows of a tile
+GROUP_RULES = [((16, 4, 4), (2, 3), 1000, "right"), ((20, 3), (1, 2), 2469, "right"), ((3, 6, 7), (1, 3), 2298, "right"),
+               ((4, 22, 9), (2,), 150, "right"), ((40, 24, 2), (2,), 254, "left"), ((4, 21, 3), (2, 3), 1003, "right")]
+
+
+@pytest.mark.parametrize("case", range(len(GROUP_RULES)))
+@pytest.mark.parametrize("dtype", DTS)
+def test_site_group_rules(case, dtype):
+    """Against the mode-by-mode chain (fused_lt = 0), beta = 0 over NaN and a
+    general alpha and beta."""
+    dims, sites, nc, side = GROUP_RULES[case]
+    g = np.random.default_rng(900 + case)
+    op = to_q(rand_lt(g, dims, dims, sites, ("dense",) * len(sites)))
+    D, c = int(np.prod(dims)), gb(nc)
+    shape = (D, nc) if side == "left" else (nc, D)
+    X, Y = cg(g, *shape), cg(g, *shape)
+    b = (op.basis_l, c) if side == "left" else (c, op.basis_r)
+    for al, be in ((1.0, 0.0), (0.3 - 0.8j, 0.5 + 0.1j)):
+        outs = []
+        for fused in (1, 0):
+            old = _tune("fused_lt", fused)
+            try:
+                R = Q.Operator(*b, Y if be else np.full(shape, np.nan + 0j), dtype)
+                if side == "left":
+                    Q.mul_(R, op, Q.Operator(op.basis_r, c, X, dtype), al, be)
+                else:
+                    Q.mul_(R, Q.Operator(c, op.basis_l, X, dtype), op, al, be)
+                outs.append(R.to_numpy())
+            finally:
+                _tune("fused_lt", old)
+        assert np.all(np.isfinite(outs[0])) and rel(outs[0], outs[1]) < TOLS[dtype]

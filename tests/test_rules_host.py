@@ -42,3 +42,12 @@ def test_tile_of_states_by_their_number(ask):
     assert ask(*(("qubit_state_tbits", n, 1, c, 1) for n, c in [(22, 4), (22, 8), (24, 1), (24, 2)])) == [10, 12, 10, 12]
     c32 = [(3, 1), (10, 4096), (11, 1023), (11, 1024), (18, 4), (18, 8), (20, 1), (21, 1)]
     assert ask(*(("qubit_state_tbits", n, 0, c, 0) for n, c in c32)) == [10, 10, 10, 11, 10, 11, 10, 11]
+
+
+def test_rows_of_a_site_group_tile(ask):
+    """Long runs only while every one of 256 CUs has a tile, short ones only while
+    the tiles stay one round."""
+    c64 = [(16, 50, 1), (64, 90, 1), (2048, 4, 1), (4096, 4, 1), (16000, 16, 1), (1 << 20, 16, 1), (1 << 20, 2000, 1)]
+    assert ask(*(("any_rows", 1, n1, P, n3, 256) for n1, P, n3 in c64)) == [2, 2, 8, 16, 32, 128, 8]
+    c32 = [(16, 50, 1), (1000, 121, 4), (4096, 16, 1), (16000, 16, 1), (1 << 20, 16, 1), (40, 24, 508)]
+    assert ask(*(("any_rows", 0, n1, P, n3, 256) for n1, P, n3 in c32)) == [2, 16, 16, 32, 256, 64]
