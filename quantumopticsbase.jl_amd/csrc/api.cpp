@@ -2135,19 +2135,6 @@ static qob_status chain_step(const Apply &ap, OpNode &owner, const std::string &
     return QOB_OK;
 }
 
-// A pass of one factor, over `total` elements: the mode kernels (k_mode_fib
-// without an LDS round trip, k_mode_chunk for n1 < 16) pad the factor to
-// multiples of 16 both ways, the group kernel to multiples of 8 and 2.  Up to
-// width 16 the mode kernels run at copy speed; wider ones, measured on a
-// 2160^2 / 5940^2 / 1600^2 ComplexF64 rho with n1 >= 16 (mode / group kernel):
-// width 20: 46 / 27 us, 33: 376 / 345 us, 40: 27 / 38 us; with n1 = 1 width 33:
-// 928 / 369 us, 40: 61 / 33 us.  On a few thousand elements (a Ket) the group
-// kernel has too few tiles for its factor's load.
-static bool mode_better(int64_t total, int64_t n1, int d) {
-    const int f = (d + 15) / 16 * 16, g8 = (d + 7) / 8 * 8, g2 = (d + 1) / 2 * 2;
-    return d <= 16 || total < (1 << 16) || (n1 >= 16 && 10 * f * f < 17 * g8 * g2);
-}
-
 // Square dense factors of any width up to ANY_MAXD (in site order) through
 // passes that each apply the factors of a group of consecutive sites
 // (k_ltany.hip).  A group takes the next factor while two workgroups of its
@@ -2217,10 +2204,13 @@ static qob_status apply_lt_any(const Apply &ap, const std::vector<ChainOp> &ops,
         void *dst = last ? out : t[i & 1];
         const AnyPass &S = passes[i];
         const AnyMode &M = S.m[0];
-        if (S.nmodes == 1 && M.d == S.P && mode_better(ap.lead * ap.trail * D, S.n1, M.d)) {
-            QOB_TRY(run_mode(ap, M.A, M.d, M.d, src, dst, S.n1, S.n3, last ? alpha : cd(1, 0), last ? beta : cd(0, 0)));
-            src = dst;
-            continue;
+        if (S.nmodes == 1) {  // M.m1: the dimensions before its site that the group took in
+            const int64_t n1 = S.n1 * M.m1;
+            if (one_factor_by_mode(ap.dt == QOB_C64, ap.lead * ap.trail * D, n1, M.d)) {
+                QOB_TRY(run_mode(ap, M.A, M.d, M.d, src, dst, n1, S.n3, last ? alpha : cd(1, 0), last ? beta : cd(0, 0)));
+                src = dst;
+                continue;
+            }
         }
         hipError_t e = launch_lt_any(ap.dt, passes[i], src, dst, d2(last ? alpha : cd(1, 0)),
                                      d2(last ? beta : cd(0, 0)), ap.s);

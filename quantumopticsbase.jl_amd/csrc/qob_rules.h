@@ -86,4 +86,34 @@ inline int any_rows(bool c64, int64_t n1, int64_t P, int64_t n3, int64_t ncu) {
     return (int)W;
 }
 
+// Whether one d x d factor on n1 x d x n3 (total elements) takes a mode kernel
+// (k_mode_fib for n1 >= 16, else k_mode_chunk) and not a site-group pass of its
+// own.  The mode kernels pad the factor to multiples of 16 both ways, the group
+// kernel to multiples of 8 and 2, but each of its workgroups loads the factor and
+// it needs tiles enough to hide that.  Up to width 16 the mode kernels run at
+// copy speed.  Mode / group kernel, us, total 10^5, 10^6, 10^7:
+//   ComplexF64 n1 = 1      17: 6.1 / 5.7, 15 / 12, 129 / 63;  25: 6.3 / 8.3, 14 /
+//                          15, 108 / 104;  33: 9.6 / 10.6, 30 / 17, 264 / 107
+//   ComplexF32 n1 = 1      20: 5.6 / 5.6, 9.3 / 8.9, 51 / 40;  21: 5.6 / 5.9, 8.2 /
+//                          9.9, 49 / 49;  28: 5.8 / 7.1, 8.4 / 12.5, 40 / 67;
+//                          33: 8.0 / 8.7, 13 / 12, 83 / 60
+//   ComplexF32 n1 = 5      21: 7.3 / 5.9, 10 / 10.5, 57 / 49
+//   n1 = 16                21: ComplexF64 7.1 / 6.7, 13 / 15, 80 / 111; ComplexF32
+//                          5.7 / 5.8, 8.4 / 13, 45 / 93;  17: 7.1 / 5.8, 12 / 14,
+//                          94 / 96; 5.7 / 5.3, 8.1 / 12, 52 / 83
+//   n1 = 600               22: ComplexF64 7.2 / 6.7, 13 / 10, 81 / 67; ComplexF32
+//                          5.7 / 5.7, 8.3 / 10, 45 / 40
+inline bool one_factor_by_mode(bool c64, int64_t total, int64_t n1, int d) {
+    if (d <= 16 || (total < (1 << 16) && (n1 == 1 || n1 >= 16))) return true;
+    if (n1 >= 16) {
+        if (d <= 20) return n1 < (c64 ? 20 : 32) && total >= (1 << 17);
+        if (d <= 24) return n1 < 64 || total < (c64 ? 1 << 19 : 1 << 21);
+        return true;
+    }
+    if (d <= 20) return false;
+    if (c64) return total < (d <= 24 ? 1 << 19 : d <= 32 ? 1 << 20 : 1 << 18);
+    if (d <= 24) return total < (1 << 21) && (n1 <= 2 || total >= (1 << 18));
+    return d <= 32 || total < (1 << 19);
+}
+
 }  // namespace qob

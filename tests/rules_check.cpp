@@ -28,6 +28,10 @@ int main() {
             long long c64, n1, P, n3, ncu;
             s >> c64 >> n1 >> P >> n3 >> ncu;
             std::cout << qob::any_rows(c64 != 0, n1, P, n3, ncu) << "\n";
+        } else if (name == "one_factor_by_mode") {
+            long long c64, total, n1, d;
+            s >> c64 >> total >> n1 >> d;
+            std::cout << qob::one_factor_by_mode(c64 != 0, total, n1, (int)d) << "\n";
         } else {
             return 1;
         }

@@ -51,3 +51,11 @@ def test_rows_of_a_site_group_tile(ask):
     assert ask(*(("any_rows", 1, n1, P, n3, 256) for n1, P, n3 in c64)) == [2, 2, 8, 16, 32, 128, 8]
     c32 = [(16, 50, 1), (1000, 121, 4), (4096, 16, 1), (16000, 16, 1), (1 << 20, 16, 1), (40, 24, 508)]
     assert ask(*(("any_rows", 0, n1, P, n3, 256) for n1, P, n3 in c32)) == [2, 16, 16, 32, 256, 64]
+
+
+def test_one_factor_by_a_mode_kernel(ask):
+    q = [(1, 1 << 24, 1, 16), (1, 1 << 15, 1, 17), (1, 1 << 15, 5, 17), (1, 1 << 20, 1, 25), (1, (1 << 20) - 1, 1, 25), (1, 1 << 19, 2, 24), (1, 1 << 18, 5, 33),
+         (1, (1 << 18) - 1, 5, 33), (0, 1 << 24, 1, 28), (0, 1 << 20, 1, 22), (0, 1 << 21, 1, 22), (0, 1 << 17, 5, 22),
+         (0, 1 << 18, 5, 22), (0, 1 << 19, 2, 33), (1, 1 << 17, 16, 17), (1, 1 << 17, 26, 17), (0, 1 << 17, 26, 17),
+         (1, 1 << 20, 40, 24), (1, 1 << 20, 64, 24), (0, 1 << 20, 64, 24), (0, 1 << 21, 64, 24), (1, 1 << 24, 600, 25)]
+    assert ask(*(("one_factor_by_mode",) + x for x in q)) == [1, 1, 0, 0, 1, 0, 0, 1, 1, 1, 0, 0, 1, 0, 1, 0, 1, 1, 0, 1, 0, 1]
