@@ -86,6 +86,15 @@ inline int any_rows(bool c64, int64_t n1, int64_t P, int64_t n3, int64_t ncu) {
     return (int)W;
 }
 
+// Whether blocks of P elements are too long for one site-group pass over few
+// rows: ComplexF32 tiles of two rows are runs of 16 bytes and one tile's modes are
+// the pass's time (from the right, chain of modes / one group of all factors, us,
+// factors at their sites of the shape: (8, 4, 5, 3, 5) at 1, 3, 5 on 54 rows 11.4 /
+// 19.9, (7, 3, 4, 23) at 1, 2, 4 on 64 14.6 / 20.9, (36, 5, 7) on 64 17.0 / 18.9,
+// (34, 5, 5), blocks of 850, on 55 16.4 / 14.9; in ComplexF64 (36, 5, 7) 21.6 /
+// 17.7, (12, 2, 7, 9) on 448 40.9 / 21.8).  The factors then form several groups.
+inline bool group_too_thin(bool c64, int64_t n1, int W, int64_t P) { return !c64 && n1 > 1 && W <= 2 && P > 1024; }
+
 // Whether one d x d factor on n1 x d x n3 (total elements) takes a mode kernel
 // (k_mode_fib for n1 >= 16, else k_mode_chunk) and not a site-group pass of its
 // own.  The mode kernels pad the factor to multiples of 16 both ways, the group

@@ -498,11 +498,13 @@ def test_bra_over_column_lengths(k, dtype):
 
 # (dims, sites, other dimension of the matrix, side) on both sides of the lines
 # that the choice of a pass and of its tile has: rows of a tile; a pass of one
-# factor, behind a short prefix, a long one, and none
+# factor, behind a short prefix, a long one, and none; long blocks on few rows
 GROUP_RULES = [((16, 4, 4), (2, 3), 1000, "right"), ((20, 3), (1, 2), 2469, "right"), ((3, 6, 7), (1, 3), 2298, "right"),
                ((4, 22, 9), (2,), 150, "right"), ((40, 24, 2), (2,), 254, "left"), ((4, 21, 3), (2, 3), 1003, "right"),
                ((3, 27), (2,), 40, "left"), ((10, 24), (2,), 1001, "left"), ((5, 22, 3), (2,), 900, "left"),
-               ((1, 36), (2,), 7300, "left"), ((2, 30), (2,), 20000, "left"), ((17, 2), (1,), 3001, "right"), ((24, 3), (1,), 65, "right")]
+               ((1, 36), (2,), 7300, "left"), ((2, 30), (2,), 20000, "left"), ((17, 2), (1,), 3001, "right"), ((24, 3), (1,), 65, "right"),
+               ((8, 4, 5, 3, 5), (1, 3, 5), 54, "right"), ((22, 7, 22), (1, 3), 35, "right"), ((7, 3, 4, 23), (1, 2, 4), 65, "right"),
+               ((5, 6, 12, 10), (2, 3, 4), 17, "right")]
 
 
 @pytest.mark.parametrize("case", range(len(GROUP_RULES)))

@@ -59,3 +59,8 @@ def test_one_factor_by_a_mode_kernel(ask):
          (0, 1 << 18, 5, 22), (0, 1 << 19, 2, 33), (1, 1 << 17, 16, 17), (1, 1 << 17, 26, 17), (0, 1 << 17, 26, 17),
          (1, 1 << 20, 40, 24), (1, 1 << 20, 64, 24), (0, 1 << 20, 64, 24), (0, 1 << 21, 64, 24), (1, 1 << 24, 600, 25)]
     assert ask(*(("one_factor_by_mode",) + x for x in q)) == [1, 1, 0, 0, 1, 0, 0, 1, 1, 1, 0, 0, 1, 0, 1, 0, 1, 1, 0, 1, 0, 1]
+
+
+def test_groups_over_few_rows(ask):
+    q = [(0, 54, 2, 2400), (0, 54, 2, 1024), (0, 54, 4, 2400), (0, 1, 1, 2400), (1, 54, 2, 2400)]
+    assert ask(*(("group_too_thin",) + x for x in q)) == [1, 0, 0, 0, 0]
