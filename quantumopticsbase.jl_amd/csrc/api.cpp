@@ -3769,8 +3769,8 @@ static qob_status fused_bilinear(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNo
         QOB_TRY(lazy_plan(op, "ls" + std::to_string(op.version), lts, op.coef, false, dt, G, true, st));
     }
     const int nb = gather_dot_blocks(n);
-    QOB_TRY(ws_get(ctx, st, WS_RED, (size_t)nb * 2 * sizeof(double2), p));
-    hipError_t e = launch_gather_dot(dt, G, 0, u, v, n, (double2 *)p, st);
+    QOB_TRY(ws_get(ctx, st, WS_RED, (size_t)nb * (uv ? 2 : 1) * sizeof(double2), p));
+    hipError_t e = launch_gather_dot(dt, G, uv ? GD_BILINEAR_DOT : GD_BILINEAR, u, v, n, (double2 *)p, st);
     if (e != hipSuccess) return fail(QOB_EHIP, "fused expect: %s", hipGetErrorString(e));
     hv = RedSet{(const double2 *)p, nb};
     if (uv) *uv = RedSet{(const double2 *)p + nb, nb};
@@ -3811,7 +3811,7 @@ static qob_status fused_trace(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNode 
     }
     const int nb = gather_dot_blocks(n);
     QOB_TRY(ws_get(ctx, st, WS_RED, (size_t)nb * sizeof(double2), p));
-    hipError_t e = launch_gather_dot(dt, G, 1, nullptr, V, n, (double2 *)p, st);
+    hipError_t e = launch_gather_dot(dt, G, GD_TRACE, nullptr, V, n, (double2 *)p, st);
     if (e != hipSuccess) return fail(QOB_EHIP, "fused trace: %s", hipGetErrorString(e));
     tr = RedSet{(const double2 *)p, nb};
     return QOB_OK;

@@ -233,6 +233,7 @@ __device__ __forceinline__ double2 block_sum256(double2 v) {
     return sh[0];
 }
 
+// mode: GatherDot
 template <typename T, int MODE>
 __global__ void __launch_bounds__(256) k_gather_dot(GatherPlanDev P, const T *__restrict__ u, const T *__restrict__ v,
                                                     int64_t n, double2 *__restrict__ partials) {
@@ -240,14 +241,16 @@ __global__ void __launch_bounds__(256) k_gather_dot(GatherPlanDev P, const T *__
     for (int64_t J = blockIdx.x * (int64_t)256 + threadIdx.x; J < n; J += (int64_t)gridDim.x * 256) {
         Digits dg{0, 0};
         T acc;
-        if (MODE == 0) {
+        if (MODE != GD_TRACE) {
             acc = eval_terms<T, true>((uint32_t)J, P, dg, [&](int64_t K) { return v[K]; });
             const T a = u[J];
             r.x += (double)a.x * acc.x + (double)a.y * acc.y;
             r.y += (double)a.x * acc.y - (double)a.y * acc.x;
-            const T b = v[J];  // sum conj(u) v, which a variance needs as well
-            p.x += (double)a.x * b.x + (double)a.y * b.y;
-            p.y += (double)a.x * b.y - (double)a.y * b.x;
+            if (MODE == GD_BILINEAR_DOT) {
+                const T b = v[J];
+                p.x += (double)a.x * b.x + (double)a.y * b.y;
+                p.y += (double)a.x * b.y - (double)a.y * b.x;
+            }
         } else {
             const T *col = v + J * n;
             acc = eval_terms<T, true>((uint32_t)J, P, dg, [&](int64_t K) { return col[K]; });
@@ -257,7 +260,7 @@ __global__ void __launch_bounds__(256) k_gather_dot(GatherPlanDev P, const T *__
     }
     const double2 t = block_sum256(r);
     if (threadIdx.x == 0) partials[blockIdx.x] = t;
-    if (MODE == 0) {
+    if (MODE == GD_BILINEAR_DOT) {
         __syncthreads();
         const double2 q = block_sum256(p);
         if (threadIdx.x == 0) partials[gridDim.x + blockIdx.x] = q;
@@ -268,14 +271,21 @@ __global__ void __launch_bounds__(256) k_gather_dot(GatherPlanDev P, const T *__
 
 int gather_dot_blocks(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(1024, (n + 255) / 256)); }
 
-hipError_t launch_gather_dot(qob_dtype dt, const GatherPlanDev &P, int mode, const void *u, const void *v, int64_t n,
+hipError_t launch_gather_dot(qob_dtype dt, const GatherPlanDev &P, GatherDot mode, const void *u, const void *v, int64_t n,
                              double2 *partials, hipStream_t s) {
     if (!P.square) return hipErrorInvalidValue;
     const int g = gather_dot_blocks(n);
 #define QOB_GD(TT, MD) \
     hipLaunchKernelGGL((k_gather_dot<TT, MD>), dim3(g), dim3(256), 0, s, P, (const TT *)u, (const TT *)v, n, partials)
-    if (dt == QOB_C64) { if (mode == 0) QOB_GD(double2, 0); else QOB_GD(double2, 1); }
-    else { if (mode == 0) QOB_GD(float2, 0); else QOB_GD(float2, 1); }
+#define QOB_GDM(TT)                                                    \
+    do {                                                               \
+        if (mode == GD_BILINEAR) QOB_GD(TT, GD_BILINEAR);              \
+        else if (mode == GD_TRACE) QOB_GD(TT, GD_TRACE);               \
+        else QOB_GD(TT, GD_BILINEAR_DOT);                              \
+    } while (0)
+    if (dt == QOB_C64) QOB_GDM(double2);
+    else QOB_GDM(float2);
+#undef QOB_GDM
 #undef QOB_GD
     return hipGetLastError();
 }

@@ -406,11 +406,14 @@ hipError_t launch_lt_any(qob_dtype dt, AnyPass S, const void *in, void *out, dou
                          hipStream_t s);
 
 // Fused reductions over a square gather plan (FP64 partials, one per block):
-//   mode 0: sum_J conj(u[J]) (H v)[J]          (expect / bilinear on a Ket)
-//   mode 1: sum_J (H V[:, J])[J], V n x n       (tr(H V), expect on rho)
+//   GD_BILINEAR      sum_J conj(u[J]) (H v)[J]      (expect / bilinear on a Ket)
+//   GD_TRACE         sum_J (H V[:, J])[J], V n x n  (tr(H V), expect on rho)
+//   GD_BILINEAR_DOT  as the first, and sum_J conj(u[J]) v[J] in a second set of
+//                    partials after the first's (a variance needs both)
+enum GatherDot { GD_BILINEAR, GD_TRACE, GD_BILINEAR_DOT };
 int gather_dot_blocks(int64_t n);
-hipError_t launch_gather_dot(qob_dtype dt, const GatherPlanDev &P, int mode, const void *u, const void *v, int64_t n,
-                             double2 *partials, hipStream_t s);
+hipError_t launch_gather_dot(qob_dtype dt, const GatherPlanDev &P, GatherDot mode, const void *u, const void *v,
+                             int64_t n, double2 *partials, hipStream_t s);
 // sums of conj(u[J]) (H v)[J] and conj(u[J]) v[J] for one qubit state
 // (single.in = v); square: of |(H v)[J]|^2 and conj(v[J]) (H v)[J].  FP64
 // partials, one of each per workgroup (qubit_dot_blocks), the second sum's

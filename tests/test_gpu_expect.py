@@ -377,3 +377,35 @@ def test_variance_ket_of_several_passes(kind, mode, dtype, eps):
     finally:
         ctx.set_mode(Q.QOB_MODE_FUSED)
     assert abs(got - want) <= bound
+
+
+@pytest.mark.parametrize("shape", [(15, 17), (16, 16), (1, 257), (510, 514), (512, 512), (513, 512)])
+@pytest.mark.parametrize("dtype,eps", [(np.complex128, 2.0 ** -52), (np.complex64, 2.0 ** -23)])
+def test_expect_and_variance_of_sparse_sums_by_length(shape, dtype, eps):
+    """Around one workgroup of 256 elements and the largest grid (2^18 elements):
+    the sum alone (expect) and with conj(psi) op psi beside it (variance).  An
+    element of op psi is a sum of at most 5 complex products of up to 3 factors:
+    less than 12 eps |M| |psi|."""
+    g = np.random.default_rng(sum(shape))
+    ba, bb = (Q.GenericBasis(d) for d in shape)
+    B = Q.tensor(ba, bb)
+
+    def factor(d):
+        m = sp.diags([g.standard_normal(d - 1) + 0.5j, g.standard_normal(d) + 0j], [1, 0] if d > 1 else [0], shape=(d, d)) \
+            if d > 1 else sp.csc_matrix([[0.8 + 0.3j]])
+        return sp.csc_matrix(m).astype(complex)
+    a, b, c, d = factor(shape[0]), factor(shape[1]), factor(shape[0]), factor(shape[1])
+    S = lambda bas, m: Q.SparseOperator(bas, bas, m)
+    co = [0.7, -0.4 + 0.2j, 1.1j]
+    op = Q.LazySum(B, B, co, (Q.LazyTensor(B, B, (1,), (S(ba, a),)), Q.LazyTensor(B, B, (2,), (S(bb, b),)),
+                              Q.LazyTensor(B, B, (1, 2), (S(ba, c), S(bb, d)))))
+    parts = (sp.kron(sp.identity(shape[1]), a), sp.kron(b, sp.identity(shape[0])), sp.kron(d, c))
+    M = sum(z * m for z, m in zip(co, parts)).tocsr()
+    W = sum(abs(z) * abs(m) for z, m in zip(co, parts)).tocsr()
+    psi = g.standard_normal(len(B)) + 1j * g.standard_normal(len(B))
+    psi = (psi / np.linalg.norm(psi)).astype(dtype)
+    k, x = Q.Ket(B, psi, dtype), psi.astype(complex)
+    r = abs(x)
+    e, e2 = np.vdot(x, M @ x), np.vdot(x, M @ (M @ x))
+    assert abs(Q.expect(op, k) - e) <= 12 * eps * (r @ (W @ r))
+    assert abs(Q.variance(op, k) - (e2 - e * e)) <= 30 * eps * (r @ (W @ (W @ r)) + (r @ (W @ r)) ** 2)
