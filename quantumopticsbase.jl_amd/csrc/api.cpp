@@ -1008,13 +1008,11 @@ struct Workspace {
 };
 
 // One scalar result on its way to the host, in pinned memory: workgroups (or
-// the last kernel's only one) store values and then a sequence number each,
-// for which the host waits.  A slot belongs to one call from its start to its
-// end.
+// the last kernel's only one) store numbered words (HostOut), for which the
+// host waits.  A slot belongs to one call from its start to its end.
 constexpr int HOST_PARTS = 8;
 struct alignas(64) HostSlot {
-    double2 v[2 * HOST_PARTS];
-    uint32_t flag[HOST_PARTS];
+    uint64_t w[4 * 2 * HOST_PARTS];
 };
 constexpr int HOST_SLOTS = 63;
 
@@ -3571,18 +3569,23 @@ struct HostSum {
         HostOut o;
         if (i < 0 || parts > HOST_PARTS) return o;
         queued = true;
-        o.v = ctx->hslot[i].v;
-        o.flag = ctx->hslot[i].flag;
+        o.w = ctx->hslot[i].w;
         o.seq = ++ctx->hseq[i];
         return o;
     }
-    qob_status wait(int parts) {
-        HostSlot &S = ctx->hslot[i];
+    // waits for the first n sums of the slot
+    qob_status wait(int n, double2 *v) {
+        const uint64_t *w = ctx->hslot[i].w;
         const uint32_t seq = ctx->hseq[i];
-        int k = 0;  // numbers 0 .. k - 1 are there
+        uint32_t b[4 * 2 * HOST_PARTS];
+        int k = 0;  // words 0 .. k - 1 are there
         auto there = [&] {
-            while (k < parts && __atomic_load_n(&S.flag[k], __ATOMIC_ACQUIRE) == seq) ++k;
-            return k == parts;
+            for (; k < 4 * n; ++k) {
+                const uint64_t x = __atomic_load_n(&w[k], __ATOMIC_RELAXED);
+                if ((uint32_t)(x >> 32) != seq) return false;
+                b[k] = (uint32_t)x;
+            }
+            return true;
         };
         const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
         bool ok = there();
@@ -3593,18 +3596,20 @@ struct HostSum {
             QOB_HIP(hipStreamSynchronize(st));
             if (!there()) return fail(QOB_EHIP, "a reduction finished without its result");
         }
+        memcpy(v, b, n * sizeof(double2));
         queued = false;
         return QOB_OK;
     }
-    // the sums of the workgroups that out(parts) was given to
+    // the sums of the workgroups that out(parts) was given to, all that they
+    // store (a word of this call must not arrive in the next one's)
     qob_status sum(RedMode mode, int parts, int sets, double2 *h) {
-        QOB_TRY(wait(parts));
-        const HostSlot &S = ctx->hslot[i];
+        double2 v[2 * HOST_PARTS];
+        QOB_TRY(wait(parts * sets, v));
         for (int t = 0; t < sets; ++t) {
             double2 r = make_double2(0, 0);
             for (int k = 0; k < parts; ++k) {
-                r.x += S.v[t * parts + k].x;
-                r.y += S.v[t * parts + k].y;
+                r.x += v[t * parts + k].x;
+                r.y += v[t * parts + k].y;
             }
             h[t] = r;
         }
@@ -3616,17 +3621,13 @@ struct HostSum {
         if (i < 0) {
             void *d;
             QOB_TRY(scal_ws(ctx, st, d));
-            QOB_HIP(launch_final(mode, a, b, d, nullptr, 0, st));
+            QOB_HIP(launch_final(mode, a, b, d, HostOut{}, st));
             QOB_HIP(hipMemcpyAsync(h, d, (b.n ? 2 : 1) * sizeof(double2), hipMemcpyDeviceToHost, st));
             QOB_HIP(hipStreamSynchronize(st));
             return QOB_OK;
         }
-        const HostOut o = out(1);
-        QOB_HIP(launch_final(mode, a, b, o.v, o.flag, o.seq, st));
-        QOB_TRY(wait(1));
-        h[0] = o.v[0];
-        h[1] = o.v[1];
-        return QOB_OK;
+        QOB_HIP(launch_final(mode, a, b, nullptr, out(1), st));
+        return wait(b.n ? 2 : 1, h);
     }
 };
 
@@ -3646,7 +3647,7 @@ static qob_status reduce_to_host(qob_ctx ctx, qob_dtype dt, RedMode mode, int64_
     const HostOut o = hs.out(nb);
     hipError_t e = launch_partials(dt, mode, n, x, y, part, nb, o, st);
     if (e != hipSuccess) return fail(QOB_EHIP, "reduction launch: %s", hipGetErrorString(e));
-    if (o.v) QOB_TRY(hs.sum(mode, nb, 1, h));
+    if (o.w) QOB_TRY(hs.sum(mode, nb, 1, h));
     else QOB_TRY(hs.final(mode, RedSet{part, nb}, RedSet{}, h));
     r = h[0];
     return QOB_OK;
@@ -3732,8 +3733,8 @@ static qob_status qubit_dot_sums(qob_ctx ctx, hipStream_t st, qob_dtype dt, OpNo
     hipError_t e = launch_qubit_dot(dt, S, u, tile, (const int32_t *)P->prog.p, P->vals.p, square, (double2 *)p,
                                     o, st);
     if (e != hipSuccess) return fail(QOB_EHIP, "fused expect: %s", hipGetErrorString(e));
-    set[0] = RedSet{o.v ? nullptr : (const double2 *)p, nb};
-    set[1] = RedSet{o.v ? nullptr : (const double2 *)p + nb, nb};
+    set[0] = RedSet{o.w ? nullptr : (const double2 *)p, nb};
+    set[1] = RedSet{o.w ? nullptr : (const double2 *)p + nb, nb};
     return QOB_OK;
 }
 
@@ -3829,7 +3830,7 @@ qob_status qob_expect_ket(qob_ctx ctx, qob_dtype dt, qob_op a, const void *psi, 
         if (hv.n) {
             double2 h[2];
             if (hv.p) QOB_TRY(hs.final(RED_DOT, hv, RedSet{}, h));
-            else QOB_TRY(hs.sum(RED_DOT, hv.n, 1, h));
+            else QOB_TRY(hs.sum(RED_DOT, hv.n, 2, h));  // both that the kernel stores
             return give(QOB_OK, h[0], out);
         }
     }

@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(BS) k_reduce1(int64_t n, const T *__restrict__
         }
     }
     double2 r = block_sum(acc, sh);
-    if (host.v) {
+    if (host.w) {
         if (threadIdx.x < 64) put_host(host, 1, r);
     } else if (threadIdx.x == 0) {
         partials[blockIdx.x] = r;
@@ -157,10 +157,9 @@ __global__ void __launch_bounds__(BS) k_reduce1(int64_t n, const T *__restrict__
 }
 
 // final stage: one block sums the partials of one or two sets; mode 1 writes
-// sqrt into a double.  flag: out lies in pinned host memory, and the host
-// waits for seq there, which the release makes visible after the results.
+// sqrt into a double
 template <int MODE>
-__global__ void __launch_bounds__(BS) k_reduce2(RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq) {
+__global__ void __launch_bounds__(BS) k_reduce2(RedSet a, RedSet b, void *out, HostOut host) {
     __shared__ double2 sh[2][BS / 64];
     double2 acc = make_double2(0, 0), acc2 = make_double2(0, 0);
     for (int i = threadIdx.x; i < a.n; i += BS) {
@@ -171,13 +170,18 @@ __global__ void __launch_bounds__(BS) k_reduce2(RedSet a, RedSet b, void *out, u
         acc2.x += b.p[i].x;
         acc2.y += b.p[i].y;
     }
-    const double2 r = block_sum(acc, sh[0]);
+    double2 r = block_sum(acc, sh[0]);
     const double2 r2 = b.n ? block_sum(acc2, sh[1]) : make_double2(0, 0);
-    if (threadIdx.x == 0) {
-        if (MODE == 1) *(double *)out = sqrt(r.x);
+    if (MODE == 1) r.x = sqrt(r.x);
+    if (host.w) {
+        if (threadIdx.x < 64) {  // thread 0 has both: sum 1 to lane 1
+            const double x = __shfl(r2.x, 0, 64), y = __shfl(r2.y, 0, 64);
+            put_host(host, b.n ? 2 : 1, threadIdx.x == 0 ? r : make_double2(x, y));
+        }
+    } else if (threadIdx.x == 0) {
+        if (MODE == 1) *(double *)out = r.x;
         else *(double2 *)out = r;
         if (b.n) ((double2 *)out)[1] = r2;
-        if (flag) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -345,9 +349,9 @@ hipError_t launch_partials(qob_dtype dt, RedMode mode, int64_t n, const void *x,
     return reduce1<2>(dt, n, x, x, n + 1, partials, blocks, host, s);
 }
 
-hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq, hipStream_t s) {
-    if (mode == RED_NORM) hipLaunchKernelGGL(k_reduce2<1>, 1, BS, 0, s, a, b, out, flag, seq);
-    else hipLaunchKernelGGL(k_reduce2<0>, 1, BS, 0, s, a, b, out, flag, seq);
+hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, const HostOut &host, hipStream_t s) {
+    if (mode == RED_NORM) hipLaunchKernelGGL(k_reduce2<1>, 1, BS, 0, s, a, b, out, host);
+    else hipLaunchKernelGGL(k_reduce2<0>, 1, BS, 0, s, a, b, out, host);
     return hipGetLastError();
 }
 
@@ -355,7 +359,7 @@ hipError_t launch_reduce(qob_dtype dt, RedMode mode, int64_t n, const void *x, c
                          void *out, hipStream_t s) {
     const hipError_t e = launch_partials(dt, mode, n, x, y, partials, reduce_blocks(n), HostOut{}, s);
     if (e != hipSuccess) return e;
-    return launch_final(mode, RedSet{partials, reduce_blocks(n)}, RedSet{}, out, nullptr, 0, s);
+    return launch_final(mode, RedSet{partials, reduce_blocks(n)}, RedSet{}, out, HostOut{}, s);
 }
 
 hipError_t launch_scale_by_inv_norm(qob_dtype dt, int64_t n, const double *nrm, void *x, hipStream_t s) {

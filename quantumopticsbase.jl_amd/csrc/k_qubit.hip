@@ -850,7 +850,7 @@ __global__ void __launch_bounds__(NTH) k_qubit_dot(QubitStateDev S, const T *__r
             t.x += red[tid & 1][w].x;
             t.y += red[tid & 1][w].y;
         }
-        if (host.v) put_host(host, 2, t);
+        if (host.w) put_host(host, 2, t);
         else if (tid < 2) partials[tid * gridDim.x + blockIdx.x] = t;
     }
 }

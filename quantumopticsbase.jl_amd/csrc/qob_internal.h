@@ -105,26 +105,26 @@ template <typename T> __device__ __forceinline__ void stg_stream(T *p, T v) {
 }
 
 // ---------------------------------------------------- partials on the host
-// Where a kernel leaves few partial sums, the host adds them: workgroup b
-// stores its sum to v[b] (a second one to v[gridDim.x + b]) in pinned memory
-// and then seq to flag[b].  v == nullptr: the partials go to device memory.
+// Sums on their way to the host: a sum is four words in pinned memory, 32 bits of
+// it in each beside the number of the call, which tells the host that the word
+// is there.  A word is one atomic store, so nothing has to be ordered between
+// them (results and then a flag: a release, which writes the L2 back first, or a
+// wait that the memory model does not know).
+// w == nullptr: the sums go to device memory.
 struct HostOut {
-    double2 *v = nullptr;
-    uint32_t *flag = nullptr;
+    uint64_t *w = nullptr;
     uint32_t seq = 0;
 };
-// all threads of the wave that holds the workgroup's sums; lane k < n has
-// sum k.  System-scope stores are written through, so their acknowledgement
-// orders them before the flag; a release would write the L2 back first.
+// all threads of the wave that holds the workgroup's n <= 2 sums, sum k in lane
+// k; workgroup b's sum k goes to place k gridDim.x + b
 __device__ __forceinline__ void put_host(const HostOut &H, int n, double2 r) {
-    const int k = threadIdx.x & 63;
-    if (k < n) {
-        double2 *p = H.v + k * (int)gridDim.x + blockIdx.x;
-        __hip_atomic_store(&p->x, r.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(&p->y, r.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (k == 0) __hip_atomic_store(H.flag + blockIdx.x, H.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    const int l = threadIdx.x & 63, k = l >> 2;
+    const double x = __shfl(r.x, k, 64), y = __shfl(r.y, k, 64);
+    const double d = l & 2 ? y : x;
+    const uint32_t b = (uint32_t)(l & 1 ? __double2hiint(d) : __double2loint(d));
+    if (k < n)
+        __hip_atomic_store(H.w + 4 * (k * (int)gridDim.x + (int)blockIdx.x) + (l & 3), (uint64_t)H.seq << 32 | b,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ------------------------------------------------------ fast integer divide
@@ -223,8 +223,7 @@ hipError_t launch_convert(qob_dtype from, const void *src, qob_dtype to, void *d
 // Two-stage FP64 reductions: reduce_blocks(n) partials of a dot product, a
 // squared norm or the trace of an n x n matrix, then their sum (the root of
 // it for RED_NORM) into out, a double2 (a double for RED_NORM).  launch_final
-// sums one or two sets of partials; with flag, out and flag are pinned host
-// memory and flag becomes seq once the results are there.
+// sums one or two sets of partials, to host where it has a place.
 enum RedMode { RED_DOT = 0, RED_NORM = 1, RED_TRACE = 2 };
 struct RedSet {
     const double2 *p = nullptr;
@@ -233,7 +232,7 @@ struct RedSet {
 int reduce_blocks(int64_t n);
 hipError_t launch_partials(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
                            int blocks, const HostOut &host, hipStream_t s);
-hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, uint32_t *flag, uint32_t seq, hipStream_t s);
+hipError_t launch_final(RedMode mode, RedSet a, RedSet b, void *out, const HostOut &host, hipStream_t s);
 hipError_t launch_reduce(qob_dtype dt, RedMode mode, int64_t n, const void *x, const void *y, double2 *partials,
                          void *out, hipStream_t s);
 // x *= 1/|norm| or 1/trace taken from a device scalar

@@ -409,3 +409,54 @@ def test_expect_and_variance_of_sparse_sums_by_length(shape, dtype, eps):
     e, e2 = np.vdot(x, M @ x), np.vdot(x, M @ (M @ x))
     assert abs(Q.expect(op, k) - e) <= 12 * eps * (r @ (W @ r))
     assert abs(Q.variance(op, k) - (e2 - e * e)) <= 30 * eps * (r @ (W @ (W @ r)) + (r @ (W @ r)) ** 2)
+
+
+def test_scalars_of_many_threads_and_streams_word_by_word():
+    """Scalar results of four threads in turn over states whose sums are whole
+    numbers: every result is exactly its own (a word of another call, or of the
+    slot's last one, would change it), by one workgroup's sums, several, and two
+    launches, one sum and two."""
+    import ctypes as C
+    import threading
+
+    from qobhip.serve import new_stream
+    g = np.random.default_rng(8)
+    L = 6
+    Hq, _, B = build_pair(L, [(1.0, (i + 1,), [np.diag([1.0 + 0j, -1.0])]) for i in range(L)])
+    Hq._handle()
+    ctx, errors = Q.context(), []
+
+    def work(seed):
+        r = np.random.default_rng(seed)
+        st = new_stream()
+        try:
+            xs = []
+            for n in (3, 300, 2048, 5000):
+                x = (r.integers(-9, 10, n) + 1j * r.integers(-9, 10, n)).astype(complex)
+                y = (r.integers(-9, 10, n) + 1j * r.integers(-9, 10, n)).astype(complex)
+                xs.append((n, Q.DeviceArray.from_numpy(x), Q.DeviceArray.from_numpy(y), np.vdot(x, y)))
+            p = (r.integers(-9, 10, 2 ** L) + 1j * r.integers(-9, 10, 2 ** L)).astype(complex)
+            z = L - 2 * np.array([bin(i).count("1") for i in range(2 ** L)])
+            pd, e, e2 = Q.DeviceArray.from_numpy(p), (abs(p) ** 2 * z).sum(), (abs(p) ** 2 * z ** 2).sum()
+            e, e2 = round(e), round(e2)
+            Q.synchronize()
+            out = _lib.qob_c64()
+            for _ in range(300):
+                for n, x, y, want in xs:
+                    _lib.call("qob_dot", ctx.h, x.qdt, n, x.ptr, y.ptr, C.byref(out), st)
+                    if complex(out.re, out.im) != want:
+                        errors.append((seed, n, out.re, out.im, want))
+                _lib.call("qob_expect_ket", ctx.h, pd.qdt, Hq._handle(), pd.ptr, 2 ** L, C.byref(out), st)
+                if complex(out.re, out.im) != e:
+                    errors.append((seed, "expect", out.re, out.im, e))
+                _lib.call("qob_variance_ket", ctx.h, pd.qdt, Hq._handle(), pd.ptr, 2 ** L, C.byref(out), st)
+                if complex(out.re, out.im) != e2 - e * e:
+                    errors.append((seed, "variance", out.re, out.im, e2 - e * e))
+        finally:
+            _lib.call("qob_stream_destroy", ctx.h, st)
+    ts = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errors, errors[:5]
