@@ -864,6 +864,28 @@ hipError_t launch_zgemm(qob_dtype dt, int64_t M, int64_t N, int64_t K, const voi
     // TFLOP/s at 4096^3 in ComplexF64).  With few tiles per CU the smaller
     // one also keeps more waves in flight (700^3: 52 against 58 us).
     const int64_t nl = ((M + 63) / 64) * ((N + 31) / 32) * batch, ns = ((M + 31) / 32) * ((N + 31) / 32) * batch;
+    // A launch has less than 2^32 threads: more tiles go in two halves (of the
+    // batch, of C's columns or of its rows).
+    if (ns > 0xffffffffll / GNT && ns <= 0x7fffffff) {
+        const size_t es = dt == QOB_C64 ? sizeof(double2) : sizeof(float2);
+        auto at = [&](const void *p, int64_t e) { return (void *)((char *)p + e * (int64_t)es); };
+        auto part = [&](int64_t m, int64_t n, int64_t z, int64_t m0, int64_t n0, int64_t z0) {
+            return launch_zgemm(dt, m, n, K, at(A, z0 * sa + m0 * sam), sam, sak, sa, at(B, z0 * sb + n0 * sbn), sbk, sbn,
+                                sb, at(C, z0 * sc + m0 * scm + n0 * scn), scm, scn, sc, z, alpha, beta, s);
+        };
+        const int64_t hz = batch / 2, hn = (N / 2 + 31) / 32 * 32, hm = (M / 2 + 31) / 32 * 32;
+        hipError_t e;
+        if (batch > 1) {
+            e = part(M, N, hz, 0, 0, 0);
+            return e != hipSuccess ? e : part(M, N, batch - hz, 0, 0, hz);
+        }
+        if (N >= M) {
+            e = part(M, hn, 1, 0, 0, 0);
+            return e != hipSuccess ? e : part(M, N - hn, 1, 0, hn, 0);
+        }
+        e = part(hm, N, 1, 0, 0, 0);
+        return e != hipSuccess ? e : part(M - hm, N, 1, hm, 0, 0);
+    }
     const int64_t rl = (nl + ncu - 1) / ncu, rs = (ns + ncu - 1) / ncu;
     const bool large = rl > 2 && 200 * rl < 109 * rs;
     if (dt == QOB_C64) {

@@ -533,3 +533,19 @@ def test_site_group_rules(case, dtype):
             finally:
                 _tune("fused_lt", old)
         assert np.all(np.isfinite(outs[0])) and rel(outs[0], outs[1]) < TOLS[dtype]
+
+
+def test_gemm_of_more_tiles_than_one_launch_holds():
+    """2^24 tiles of 256 threads are more than a launch takes: a 1 x 1 matrix on a row of
+    2^29 + 33 elements (4 GiB in ComplexF32)."""
+    n = (1 << 29) + 33
+    B = np.zeros((1, n), np.complex64)
+    at = [0, 31, 32, 1 << 28, n - 66, n - 65, n - 34, n - 33, n - 2, n - 1]
+    B[0, at] = np.arange(1, 11) - 0.5j
+    dA, dB = Q.DeviceArray.from_numpy(np.array([[2 + 1j]]), np.complex64), Q.DeviceArray.from_numpy(B, np.complex64)
+    dC = Q.DeviceArray.from_numpy(np.full((1, n), np.nan, np.complex64), np.complex64)
+    _lib.call("qob_gemm", Q.context().h, dA.qdt, 0, 1, n, 1, _lib.c64(1.0), dA.ptr, dB.ptr, _lib.c64(0.0), dC.ptr, None)
+    C_ = dC.to_numpy()
+    assert np.array_equal(C_[0, at], (2 + 1j) * B[0, at])
+    C_[0, at] = 0
+    assert not C_.any()
