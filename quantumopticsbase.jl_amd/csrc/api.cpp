@@ -2139,7 +2139,9 @@ static qob_status chain_step(const Apply &ap, OpNode &owner, const std::string &
 // tiles share a CU's LDS, or while the whole product stays one pass (left
 // application of (33, 12, 15) in ComplexF64, one workgroup per CU: 609 us in
 // one pass, 730 us in two; chain of modes 1546 us); with few tiles, while
-// they stay small.  done is left false when some factor does not fit a pass.
+// they stay small (and see group_too_thin).  A pass of one factor may be a mode
+// kernel (one_factor_by_mode).  done is left false when some factor does not fit
+// a pass.
 static qob_status apply_lt_any(const Apply &ap, const std::vector<ChainOp> &ops, const std::vector<int64_t> &sh,
                                const void *in, void *out, cd alpha, cd beta, bool &done) {
     done = false;

@@ -18,10 +18,11 @@
 // of 16: 640 for a k padded to 4).  The rows of the embedding are ordered so
 // that a lane's accumulator registers hold both parts of its outputs.
 //
-// Bound by the MFMA rate plus what a wave issues between its MFMAs (on
-// ComplexF64 (12, 20, 9): MFMA pipes busy 50% of the time, other vector
-// instructions 20%) and by the barrier between modes; three or four small
-// workgroups per CU overlap one's loads and stores with another's modes.
+// Bound by the MFMA rate plus what a wave issues between its MFMAs (the left
+// pass of (12, 20, 9) on 2160^2 in ComplexF64, 67 us: MFMA pipes busy 51% of the
+// cycles in which a CU is, 42% of the kernel, other vector instructions 18%) and
+// by the barrier between modes; three or four small workgroups per CU overlap
+// one's loads and stores with another's modes.
 // Left application on a square rho, ComplexF64 / ComplexF32, mode-by-mode
 // chain -> this: (12, 20, 9) 114 / 76 -> 62 / 36 us (2.4 / 2.1 TB/s),
 // (8, 8, 8, 8) 423 / 283 -> 160 / 87 us (3.4 / 3.1 TB/s), (33, 12, 15) 1545 /

@@ -489,13 +489,15 @@ __global__ void __launch_bounds__(GNT, WPE) k_zgemm(int64_t M, int64_t N, int64_
 
 // ---------------------------------------------------------- k_zgemm_small
 // The same product where its tiles would leave most CUs idle: a workgroup has
-// one 16 x 16 tile of C, its four waves every fourth k-step of it, with the
-// fragments straight from memory (the operands fit the caches).  Bound by load
-// latency: k_zgemm waits for about one round trip per 16 k, here a wave has
-// SM_U k-steps of both operands in flight and the waves share the k range.
-// Their partial sums are added through LDS in wave order.  Against k_zgemm,
-// ComplexF64 / ComplexF32: (3000, 16, 3000) 149 / 99 -> 53 / 28 us, (128, 128,
-// 2000) 80 / 48 -> 34 / 20, 200^3 11.1 / 8.0 -> 6.6 / 5.0.
+// one 16 x 16 tile of C, its four waves runs of 16 k of it in turn, with the
+// fragments straight from memory.  Bound by load latency: k_zgemm waits for
+// about one round trip per 16 k, here a wave has SM_U k-steps of both operands
+// in flight and the waves share the k range.  Their partial sums are added
+// through LDS in wave order.  Against k_zgemm, ComplexF64 / ComplexF32: (3000, 16,
+// 3000) 149 / 99 -> 54 / 34 us, (128, 128, 2000) 80 / 48 -> 34 / 20, 200^3 11.1 /
+// 8.0 -> 7.0 / 5.1.  Long k ranges, whose operands leave the caches, gain as much
+// or nothing: (128, 128, 10^5) 4.9 / 3.2 -> 1.6 / 1.0 ms, (64, 64, 10^6) 50 / 44
+// -> 15 / 12, (400, 400, 10^5) in ComplexF64 4.9 -> 3.4, (500, 500, 10^5) 4.9 -> 4.6.
 constexpr int SM_U = 4;
 template <typename R>
 __global__ void __launch_bounds__(256) k_zgemm_small(int64_t M, int64_t N, int64_t K, const cplx<R> *__restrict__ A,

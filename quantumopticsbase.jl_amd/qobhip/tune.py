@@ -10,8 +10,9 @@ of libqob_hip.so (qob_tune_set / qob_tune_get):
                     kernel for leading dimensions below 16 as well,
                     a test and timing switch, not tuned)
   qubit sums        qubit_tbits (tile = 2^tbits states; 0 = 2^12 for
-                    ComplexF64 and 2^11 for ComplexF32 in a batch, 2^10 for
-                    single states, 2^11 above 20 sites in ComplexF32),
+                    ComplexF64 and 2^11 for ComplexF32 in a batch; for states
+                    and the columns of matrices 2^10 up to some 2^20 elements
+                    in all, then as in a batch),
                     qubit_nth (0 = 4
                     elements per lane in ComplexF64, 8 in ComplexF32),
                     qubit_grid (persistent workgroups; 0 = 1024 / nth per CU),
