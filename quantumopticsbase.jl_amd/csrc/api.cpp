@@ -2185,7 +2185,7 @@ static qob_status apply_lt_any(const Apply &ap, const std::vector<ChainOp> &ops,
             if (n1 > 1 && S.nmodes == 2 && ops.size() == 2 && nt < device_cu_count() &&
                 (ap.dt == QOB_C32 ? dsum > 44 : S.m[0].d > 20 && S.m[1].d > 20))
                 return QOB_OK;
-            if (k > i && group_too_thin(ap.dt == QOB_C64, n1, F.W, P)) continue;
+            if (k > i && group_too_thin(ap.dt == QOB_C64, n1, F.W, P, S.nmodes)) continue;
             if (k == i || (nt >= 64 ? lds <= 80 * 1024 || whole : P <= 2560 && dsum <= 64)) {
                 best = S;
                 j = k + 1;

@@ -86,14 +86,19 @@ inline int any_rows(bool c64, int64_t n1, int64_t P, int64_t n3, int64_t ncu) {
     return (int)W;
 }
 
-// Whether blocks of P elements are too long for one site-group pass over few
-// rows: ComplexF32 tiles of two rows are runs of 16 bytes and one tile's modes are
-// the pass's time (from the right, chain of modes / one group of all factors, us,
-// factors at their sites of the shape: (8, 4, 5, 3, 5) at 1, 3, 5 on 54 rows 11.4 /
-// 19.9, (7, 3, 4, 23) at 1, 2, 4 on 64 14.6 / 20.9, (36, 5, 7) on 64 17.0 / 18.9,
-// (34, 5, 5), blocks of 850, on 55 16.4 / 14.9; in ComplexF64 (36, 5, 7) 21.6 /
-// 17.7, (12, 2, 7, 9) on 448 40.9 / 21.8).  The factors then form several groups.
-inline bool group_too_thin(bool c64, int64_t n1, int W, int64_t P) { return !c64 && n1 > 1 && W <= 2 && P > 1024; }
+// Whether blocks of P elements are too long for one site-group pass of so many
+// modes over few rows: with tiles of two rows one tile's modes are the pass's
+// time, and runs are 32 bytes, 16 in ComplexF32.  From the right, chain of modes /
+// one group of all factors, us, factors at their sites of the shape: ComplexF32
+// (8, 4, 5, 3, 5) at 1, 3, 5 on 54 rows 11.4 / 19.9, (7, 3, 4, 23) at 1, 2, 4 on 64
+// 14.6 / 20.9, (36, 5, 7) on 64 17.0 / 18.9, (34, 5, 5), blocks of 850, on 55 16.4 /
+// 14.9; ComplexF64 two factors (3, 32, 14) at 1, 3 on 38 8.4 / 12.0, (33, 8, 13) at
+// 1, 3 on 138 20.1 / 26.8, (35, 5, 5), blocks of 875, at 1, 3 on 20 16.4 / 13.7, more
+// factors (13, 8, 19) on 184 20.1 / 16.6, (12, 2, 7, 9) on 448 40.9 / 21.8, (9, 4, 28)
+// on 52 15.6 / 18.2.  The factors then form several groups.
+inline bool group_too_thin(bool c64, int64_t n1, int W, int64_t P, int modes) {
+    return n1 > 1 && W <= 2 && P > 1024 && (!c64 || modes == 2);
+}
 
 // Whether one d x d factor on n1 x d x n3 (total elements) takes a mode kernel
 // (k_mode_fib for n1 >= 16, else k_mode_chunk) and not a site-group pass of its

@@ -33,9 +33,9 @@ int main() {
             s >> c64 >> total >> n1 >> d;
             std::cout << qob::one_factor_by_mode(c64 != 0, total, n1, (int)d) << "\n";
         } else if (name == "group_too_thin") {
-            long long c64, n1, W, P;
-            s >> c64 >> n1 >> W >> P;
-            std::cout << qob::group_too_thin(c64 != 0, n1, (int)W, P) << "\n";
+            long long c64, n1, W, P, modes;
+            s >> c64 >> n1 >> W >> P >> modes;
+            std::cout << qob::group_too_thin(c64 != 0, n1, (int)W, P, (int)modes) << "\n";
         } else {
             return 1;
         }

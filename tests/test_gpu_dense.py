@@ -504,7 +504,7 @@ GROUP_RULES = [((16, 4, 4), (2, 3), 1000, "right"), ((20, 3), (1, 2), 2469, "rig
                ((3, 27), (2,), 40, "left"), ((10, 24), (2,), 1001, "left"), ((5, 22, 3), (2,), 900, "left"),
                ((1, 36), (2,), 7300, "left"), ((2, 30), (2,), 20000, "left"), ((17, 2), (1,), 3001, "right"), ((24, 3), (1,), 65, "right"),
                ((8, 4, 5, 3, 5), (1, 3, 5), 54, "right"), ((22, 7, 22), (1, 3), 35, "right"), ((7, 3, 4, 23), (1, 2, 4), 65, "right"),
-               ((5, 6, 12, 10), (2, 3, 4), 17, "right")]
+               ((5, 6, 12, 10), (2, 3, 4), 17, "right"), ((3, 32, 14), (1, 3), 38, "right"), ((33, 8, 13), (1, 3), 21, "right")]
 
 
 @pytest.mark.parametrize("case", range(len(GROUP_RULES)))

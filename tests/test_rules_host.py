@@ -62,5 +62,6 @@ def test_one_factor_by_a_mode_kernel(ask):
 
 
 def test_groups_over_few_rows(ask):
-    q = [(0, 54, 2, 2400), (0, 54, 2, 1024), (0, 54, 4, 2400), (0, 1, 1, 2400), (1, 54, 2, 2400)]
-    assert ask(*(("group_too_thin",) + x for x in q)) == [1, 0, 0, 0, 0]
+    q = [(0, 54, 2, 2400, 3), (0, 54, 2, 1024, 3), (0, 54, 4, 2400, 3), (0, 1, 1, 2400, 3), (1, 54, 2, 2400, 3),
+         (1, 54, 2, 2400, 2), (1, 54, 2, 1024, 2), (1, 1, 1, 2400, 2)]
+    assert ask(*(("group_too_thin",) + x for x in q)) == [1, 0, 0, 0, 0, 1, 0, 0]
